@@ -3,32 +3,23 @@
 // f16 dot (kernels_avx2.c:118-148), softmax (kernels.c:855-885) and the
 // softmax's exp polynomial (kernels.c:820-850).
 //
-// Three launches on one stream:
-//   attn_scores_kernel   sc[h][j] = dot(K[hk][j], f16(q_h)) * kq_scale
-//   attn_softmax_kernel  p[h][j] = f16(softmax(sc[h])[j])
-//   attn_pv_kernel       out[h][c] = dot(V[hk][c][0..n), p[h])
-// or, for n <= kAttnFuseMax, two: attn_scores_kernel, then attn_pv_kernel
-// with NG > 0, each of whose waves computes the softmax of its query head
-// itself (wave_softmax) into LDS instead of loading probabilities.
+// Up to kAttnFuseMax positions one launch, attn_fused_kernel: a workgroup per
+// query head and 16 value rows scores every position itself. Beyond, three
+// launches on one stream:
+//   attn_scores_kernel   s[h][j] = dot(K[hk][j], f16(q_h)) * kq_scale, and the
+//                        maximum of each block of positions
+//   attn_exp_kernel      e[h][j] = exp(s[h][j] - max), and each block's total
+//   attn_pv_kernel       out[h][c] = dot(V[hk][c][0..n), f16(e[h] / total))
 //
 // The f16 dot is evaluated in the reference's order. Its 32 f32
 // accumulators (accumulator a takes elements i with i % 32 == a, by FMA in
-// increasing i) are spread over 8 lanes of one row, 4 each: lane L of the
-// row holds accumulators 4L..4L+3. The reference reduces them as
-// registers r0+r2, r1+r3, then their sum, then lanes l and l+4, then two
-// pairwise rounds; with that lane assignment these are additions of lanes
-// L + 4, L + 2, L + 1 followed by two in-lane additions. Elements past the last
-// multiple of 32 are added to the double total one by one, as in the
-// reference.
-//
-// Each accumulator is one chain of n / 32 dependent FMAs over the whole
-// context, so the value contraction cannot be split along the positions
-// without changing the result. attn_pv_kernel instead stages a whole
-// chunk of value rows and probabilities in LDS with every thread's loads in
-// flight at once, then runs the chains out of LDS. Workspace rows (scores
-// and probabilities) hold lw >= n entries, lw a multiple of kAttnBlock, so
-// whole-block loads stay inside the allocation; entries past n are loaded
-// but not used.
+// increasing i) are reduced as registers r0+r2, r1+r3 (8 accumulators
+// each), then their sum, then elements l and l+4, then two pairwise rounds;
+// elements past the last multiple of 32 are added to the double total one
+// by one. Each accumulator is one chain of n / 32 dependent FMAs over the
+// whole context, so the value contraction cannot be split along the
+// positions without changing the result: the parallelism is over rows,
+// heads and accumulators.
 //
 // The softmax sums its 8-element group totals in double in a tree rather
 // than in the reference's sequential order. The two double totals differ
@@ -44,11 +35,9 @@
 
 namespace sihip {
 
-constexpr int kAttnThreads = 256;
-constexpr int kAttnRowLanes = 8;                                // lanes per dot
-constexpr int kAttnRows = kAttnThreads / kAttnRowLanes;         // dots per workgroup
-constexpr int kAttnHeads = 4;                                   // query heads per pass
 constexpr int kAttnMaxHd = 512;
+constexpr int kAttnHeads = 4;  // query heads per workgroup of the scores launch
+constexpr int64_t kAttnWsBlock = 4096;  // positions that workspace rows are a multiple of
 
 struct AttnArgs {
     const float *q;        // [n_head * hd]
@@ -57,14 +46,30 @@ struct AttnArgs {
     float *out;            // [n_head * hd]
     float *sc;             // [n_head][ld] scaled scores (caller's, optional)
     uint16_t *p16;         // [n_head][ld] f16 probabilities (caller's, optional)
-    float *sw;             // [n_head][lw] scaled scores (workspace)
-    uint16_t *pw;          // [n_head][lw] f16 probabilities (workspace)
+    float *sw;             // [n_head][lw] scores, then exponentials (workspace)
+    float *pm;             // [n_head][nbs] maxima of the score blocks (workspace)
+    double *ps;            // [n_head][nbe] totals of the exponential blocks (workspace)
     int64_t n_ctx, ld, lw;
-    int n, hd, gqa, n_head;
+    int n, hd, gqa, n_kv;
+    int nbs, nbe;
     float kq_scale;
 };
 
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+
 __device__ inline float f16_at(const uint16_t *p, int64_t i) { return f16_bits_to_f32(p[i]); }
+
+// f32_to_f16_bits by the hardware's conversion (RNE, subnormals kept; the
+// bits of a NaN as f32_to_f16_bits makes them). The empty asm keeps a
+// product in f from being folded into the conversion (v_fma_mixlo_f16), which
+// would round once where the reference rounds to f32 first.
+__device__ inline uint32_t f32_to_f16_hw(float f) {
+    asm("" : "+v"(f));
+    const uint32_t u = __float_as_uint(f), m = (u >> 13) & 0x3ffu;
+    const uint32_t nan = ((u >> 16) & 0x8000u) | 0x7e00u | (m == 0u ? 1u : m);
+    const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)f);
+    return (u & 0x7fffffffu) > 0x7f800000u ? nan : h;
+}
 
 // Lane i receives lane i + K of its 16-lane row (a DPP row shift; lanes
 // whose source lies past the row receive 0, and are not used below).
@@ -73,21 +78,47 @@ __device__ inline float from_lane_up(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x100 + K, 0xf, 0xf, true));
 }
 
-// The reference's tree over the 32 accumulators of one row; lane L of the
-// row (lane & 7, rows of 8 lanes) holds acc[e] = accumulator 4L + e. Lane
-// L adds lane L + 4 (registers r0 + r2 at L = 0, 1; r1 + r3 at L = 2, 3),
-// then lane L + 2 (the sum of those), then lane L + 1 (lanes l and l + 4
-// of the reference's 8-wide registers); the result is valid in L == 0.
-// Every lane of the wave takes part.
-__device__ inline float dot_tree(const float acc[4]) {
-    float x[4];
+__device__ inline float max_sel(float a, float b) { return b > a ? b : a; }
+
+// Reductions over a wave without LDS round trips: DPP within the 16-lane
+// rows, then the gfx950 row and half swaps (each returns both lanes' values).
+__device__ inline uint2 swap16(uint32_t x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return make_uint2(r[0], r[1]);
+}
+__device__ inline uint2 swap32(uint32_t x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return make_uint2(r[0], r[1]);
+}
+
+__device__ inline float wave_max(float x) {
+    const int ctrls[4] = {kDppXor1, kDppXor2, kDppHalfMirror, kDppMirror};
 #pragma unroll
-    for (int e = 0; e < 4; e++) x[e] = acc[e] + from_lane_up<4>(acc[e]);
+    for (int i = 0; i < 4; i++) x = max_sel(x, __uint_as_float(dpp_u32(__float_as_uint(x), ctrls[i])));
+    uint2 t = swap16(__float_as_uint(x));
+    x = max_sel(__uint_as_float(t.x), __uint_as_float(t.y));
+    t = swap32(__float_as_uint(x));
+    return max_sel(__uint_as_float(t.x), __uint_as_float(t.y));
+}
+
+__device__ inline double wave_sum(double x) {
+    const int ctrls[4] = {kDppXor1, kDppXor2, kDppHalfMirror, kDppMirror};
 #pragma unroll
-    for (int e = 0; e < 4; e++) x[e] = x[e] + from_lane_up<2>(x[e]);
+    for (int i = 0; i < 4; i++) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, x);
+        const uint64_t o = (uint64_t)dpp_u32((uint32_t)u, ctrls[i]) |
+                           ((uint64_t)dpp_u32((uint32_t)(u >> 32), ctrls[i]) << 32);
+        x += __builtin_bit_cast(double, o);
+    }
 #pragma unroll
-    for (int e = 0; e < 4; e++) x[e] = x[e] + from_lane_up<1>(x[e]);
-    return (x[0] + x[1]) + (x[2] + x[3]);
+    for (int i = 0; i < 2; i++) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, x);
+        const uint2 lo = i ? swap32((uint32_t)u) : swap16((uint32_t)u);
+        const uint2 hi = i ? swap32((uint32_t)(u >> 32)) : swap16((uint32_t)(u >> 32));
+        x = __builtin_bit_cast(double, (uint64_t)lo.x | ((uint64_t)hi.x << 32)) +
+            __builtin_bit_cast(double, (uint64_t)lo.y | ((uint64_t)hi.y << 32));
+    }
+    return x;
 }
 
 // exp of the softmax groups: the polynomial the reference uses there (its
@@ -115,379 +146,602 @@ __device__ inline float expf_poly(float x) {
     return __builtin_fmaf(s2, p, s2) * s1;
 }
 
-constexpr int kAttnBlock = 4096;  // softmax positions per workgroup pass (16 per thread)
-
 // exp of a tail position's shifted score (positions past the last whole
 // 8-group): exp in double, rounded.
 __device__ inline float tail_exp(float x) { return (float)exp((double)x); }
 
-// The softmax of query head h's scores by one wave, for n <= 512 NG (the
-// value launch of the two-launch path): lane l holds the 8-groups of
-// positions 512 g + 8 l .. + 7, g < NG. The max, the exponentials, each
-// group's float sum in the reference's 8-lane order, 1 / total and the f16
-// probabilities are attn_softmax_kernel's; only the order in which the
-// groups' sums are added in double differs (a 64-lane tree instead of a
-// 256-thread one, both within n 2^-53 relative of the reference's
-// sequential sum). The tail [gend, n) is added, and its probabilities
-// written, by the lane whose group holds it, with tail_exp. The
-// probabilities go to pdst[0 .. 512 NG) (positions past n hold values
-// that are not used), and to the caller's probs16 where p16_out.
-constexpr int kAttnFuseMax = 1024;
-
-template <int NG>
-__device__ inline void wave_softmax(const AttnArgs &A, int h, int lane, uint16_t *pdst,
-                                    bool p16_out) {
-    const int n = A.n, gend = n & ~7;
-    const float *row = A.sw + (int64_t)h * A.lw;  // lw >= 512 NG entries
-    float v[NG][8];
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-        if (512 * g < n) {  // wave-uniform
-            const float4 *p = reinterpret_cast<const float4 *>(row + 512 * g + 8 * lane);
-            const float4 a = p[0], b = p[1];
-            v[g][0] = a.x, v[g][1] = a.y, v[g][2] = a.z, v[g][3] = a.w;
-            v[g][4] = b.x, v[g][5] = b.y, v[g][6] = b.z, v[g][7] = b.w;
-        }
-    float mx = -__builtin_inff();
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-        if (512 * g < n)
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                if (512 * g + 8 * lane + e < n && v[g][e] > mx) mx = v[g][e];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const float t = __shfl_xor(mx, o);
-        mx = t > mx ? t : mx;
-    }
-    // the tail's scores, before the exponentials replace them
-    const bool tail_owner = gend < n && lane == (gend % 512) / 8;
-    float tv[8];
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-        if (g == gend / 512)
-#pragma unroll
-            for (int e = 0; e < 8; e++) tv[e] = v[g][e];
-    double part = 0.0;
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-        if (512 * g < n) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[g][e] = expf_poly(v[g][e] - mx);
-            const float *x = v[g];
-            if (512 * g + 8 * lane + 8 <= gend)
-                part += (double)(((x[0] + x[4]) + (x[2] + x[6])) + ((x[1] + x[5]) + (x[3] + x[7])));
-        }
-    if (tail_owner)
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            if (gend + e < n) part += (double)tail_exp(tv[e] - mx);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) part += __shfl_xor(part, o);
-    const float scale = (float)(1.0 / part);
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-        if (512 * g < n) {
-            const int j0 = 512 * g + 8 * lane;
-            uint32_t pk[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                pk[e] = (uint32_t)f32_to_f16_bits(v[g][2 * e] * scale) |
-                        ((uint32_t)f32_to_f16_bits(v[g][2 * e + 1] * scale) << 16);
-            *reinterpret_cast<uint4 *>(pdst + j0) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-            if (A.p16 && p16_out)
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-                    if (j0 + e < n)
-                        A.p16[(int64_t)h * A.ld + j0 + e] = (uint16_t)(pk[e >> 1] >> (16 * (e & 1)));
-        }
-    // the tail's probabilities replace the polynomial's (same lane, later stores)
-    if (tail_owner)
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            if (gend + e < n) {
-                const uint16_t pb = f32_to_f16_bits(tail_exp(tv[e] - mx) * scale);
-                pdst[gend + e] = pb;
-                if (A.p16 && p16_out) A.p16[(int64_t)h * A.ld + gend + e] = pb;
-            }
+// A workgroup's query head and 1D block index: consecutive workgroups take
+// different KV heads, so that where their number is a multiple of 8 the
+// launches of a KV head run on one XCD and find its rows and scores in that
+// XCD's L2.
+struct AttnWg {
+    int hk, h, blk;
+};
+__device__ inline AttnWg attn_wg(const AttnArgs &A) {
+    const int id = (int)blockIdx.x, rest = id / A.n_kv;
+    AttnWg w;
+    w.hk = id % A.n_kv;
+    w.h = w.hk * A.gqa + rest % A.gqa;
+    w.blk = rest / A.gqa;
+    return w;
 }
 
-// Grid (ceil(n / kAttnRows), n_head_kv * ceil(gqa / kAttnHeads)): each
-// workgroup scores kAttnRows cached positions against up to kAttnHeads
-// query heads of one KV head, holding each key row in registers across
-// the heads.
-// VEC: hd % 4 == 0 and k 8-byte aligned (a lane's 4 key elements of a step
-// in one load).
-template <bool VEC>
-__global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(AttnArgs A) {
-    __shared__ uint16_t q16[kAttnHeads * kAttnMaxHd];
-    const int chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
-    const int hk = blockIdx.y / chunks;
-    const int h0 = hk * A.gqa + (blockIdx.y % chunks) * kAttnHeads;
-    const int nh = min(kAttnHeads, hk * A.gqa + A.gqa - h0);
-    const int hd = A.hd;
-    const int L = threadIdx.x & (kAttnRowLanes - 1);
-    const int64_t j = (int64_t)blockIdx.x * kAttnRows + threadIdx.x / kAttnRowLanes;
-    const int64_t jr = j < A.n ? j : A.n - 1;  // rows past n score row n-1, unstored
-    const uint16_t *krow = A.k + ((int64_t)hk * A.n_ctx + jr) * hd;
-    const int body = hd & ~31;
-    float kv[kAttnMaxHd / 32][4];
+// ---- scores ---------------------------------------------------------------------
+//
+// Four lanes score one position: lane L of the quad holds accumulators
+// 8 L .. 8 L + 7, so a 32-element step of the key row is one 16-byte load per
+// lane and a wave's 16 rows are one contiguous span of the cache. T: 32-steps
+// kept in registers (hd / 32 <= T); VEC: 16-byte loads (hd % 8 == 0, keys
+// 16-byte aligned).
+// (lane L < hd % 32 / 8 also holds elements 8 L .. + 7 past the last whole
+// step in tail; without VEC the tail is read where it is added.)
+template <int T>
+struct KeyRow {
+    uint4 w[T];
+    uint4 tail;
+};
+
+template <int T, bool VEC>
+__device__ inline void load_key(const uint16_t *row, int hd, int L, KeyRow<T> &k) {
+    const int steps = hd >> 5;
 #pragma unroll
-    for (int t = 0; t < kAttnMaxHd / 32; t++)
-        if (32 * t < body) {
+    for (int t = 0; t < T; t++)
+        if (t < steps) {
+            const uint16_t *p = row + 32 * t + 8 * L;
             if constexpr (VEC) {
-                const uint2 w = *reinterpret_cast<const uint2 *>(krow + 32 * t + 4 * L);
-                kv[t][0] = f16_bits_to_f32(w.x & 0xffffu);
-                kv[t][1] = f16_bits_to_f32(w.x >> 16);
-                kv[t][2] = f16_bits_to_f32(w.y & 0xffffu);
-                kv[t][3] = f16_bits_to_f32(w.y >> 16);
+                k.w[t] = *reinterpret_cast<const uint4 *>(p);
             } else {
+                uint32_t e[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) kv[t][e] = f16_at(krow, 32 * t + 4 * L + e);
+                for (int i = 0; i < 4; i++) e[i] = (uint32_t)p[2 * i] | ((uint32_t)p[2 * i + 1] << 16);
+                k.w[t] = make_uint4(e[0], e[1], e[2], e[3]);
             }
         }
+    if (VEC && (hd & 31))
+        k.tail = 8 * L < (hd & 31) ? *reinterpret_cast<const uint4 *>(row + 32 * steps + 8 * L)
+                                   : make_uint4(0, 0, 0, 0);
+}
+
+// The scaled score of the quad's row against the f16 query qh (LDS, 16-byte
+// aligned; q: the lane's elements of it, as load_key lays them out); valid in
+// the quad's lane 0. Every lane of the wave takes part.
+template <int T, bool VEC>
+__device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, const uint16_t *row,
+                                  const uint16_t *qh, int hd, int L, float kq_scale) {
+    const int steps = hd >> 5;
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < T; t++)
+        if (t < steps) {
+            const h8_t kk = __builtin_bit_cast(h8_t, k.w[t]);
+            const h8_t qq = __builtin_bit_cast(h8_t, q.w[t]);
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[e] = __builtin_fmaf((float)kk[e], (float)qq[e], acc[e]);
+        }
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = acc[e] + from_lane_up<2>(acc[e]);  // r0 + r2, r1 + r3
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = acc[e] + from_lane_up<1>(acc[e]);  // their sum
+    float t4[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) t4[e] = acc[e] + acc[e + 4];
+    const float res = (t4[0] + t4[1]) + (t4[2] + t4[3]);
+    double total = 0.0;
+    total += (double)res;
+    if (hd & 31) {
+        if constexpr (VEC) {
+            // each lane's products, added in element order (8 per lane)
+            const h8_t kk = __builtin_bit_cast(h8_t, k.tail), qq = __builtin_bit_cast(h8_t, q.tail);
+            float pr[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) pr[e] = (float)kk[e] * (float)qq[e];
+#pragma unroll
+            for (int e = 0; e < 8; e++) total += (double)quad_bcast<0>(pr[e]);
+            if ((hd & 31) > 8)
+#pragma unroll
+                for (int e = 0; e < 8; e++) total += (double)quad_bcast<1>(pr[e]);
+            if ((hd & 31) > 16)
+#pragma unroll
+                for (int e = 0; e < 8; e++) total += (double)quad_bcast<2>(pr[e]);
+        } else if (L == 0) {
+            for (int i = 32 * steps; i < hd; i++)
+                total += (double)(f16_at(row, i) * f16_bits_to_f32(qh[i]));
+        }
+    }
+    return (float)total * kq_scale;
+}
+
+// Grid ceil(n / 64) x ceil(gqa / 4) x n_kv, in one dimension (KV head
+// fastest): a workgroup scores 64 positions against up to 4 query heads of
+// one KV head, each key row kept in registers across the heads, and writes
+// the block's maximum per head. Bound: HBM (the key rows are read once);
+// all workgroups of 16k positions are resident together, so the whole read
+// is in flight at once.
+constexpr int kAttnScoreBlock = 64;
+
+template <int T, bool VEC>
+__global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
+    __shared__ __attribute__((aligned(16))) uint16_t q16[kAttnHeads][kAttnMaxHd];
+    __shared__ float red[kAttnHeads][4];
+    const int chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
+    const int id = (int)blockIdx.x, hk = id % A.n_kv, rest = id / A.n_kv;
+    const int hc = rest % chunks * kAttnHeads, blk = rest / chunks;
+    const int h0 = hk * A.gqa + hc, nh = min(kAttnHeads, A.gqa - hc);
+    const int hd = A.hd;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, L = lane & 3;
+    const int j = blk * kAttnScoreBlock + (int)(threadIdx.x >> 2);
+    // rows past n score row n - 1, unstored
+    const uint16_t *row = A.k + ((int64_t)hk * A.n_ctx + (j < A.n ? j : A.n - 1)) * hd;
+    KeyRow<T> kr;
+    load_key<T, VEC>(row, hd, L, kr);
     // the query heads in f16, staged while the key loads are in flight
-    for (int i = threadIdx.x; i < nh * hd; i += kAttnThreads)
-        q16[i] = f32_to_f16_bits(A.q[(int64_t)h0 * hd + i]);
+    for (int hh = 0; hh < nh; hh++)
+        for (int i = threadIdx.x; i < hd; i += 256)
+            q16[hh][i] = (uint16_t)f32_to_f16_hw(A.q[(int64_t)(h0 + hh) * hd + i]);
     __syncthreads();
     for (int hh = 0; hh < nh; hh++) {
-        const uint16_t *qh = q16 + hh * hd;
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int t = 0; t < kAttnMaxHd / 32; t++)
-            if (32 * t < body)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    acc[e] = __builtin_fmaf(kv[t][e], f16_bits_to_f32(qh[32 * t + 4 * L + e]), acc[e]);
-        const float res = dot_tree(acc);
-        if (L == 0 && j < A.n) {
-            double total = 0.0;
-            total += (double)res;
-            for (int i = body; i < hd; i++)
-                total += (double)(f16_at(krow, i) * f16_bits_to_f32(qh[i]));
-            const float v = (float)total * A.kq_scale;
+        KeyRow<T> qr;
+        load_key<T, true>(q16[hh], hd, L, qr);
+        const float v = key_score<T, VEC>(kr, qr, row, q16[hh], hd, L, A.kq_scale);
+        const bool real = L == 0 && j < A.n;
+        if (real) {
             A.sw[(int64_t)(h0 + hh) * A.lw + j] = v;
             if (A.sc) A.sc[(int64_t)(h0 + hh) * A.ld + j] = v;
         }
+        const float mx = wave_max(real ? max_sel(-__builtin_inff(), v) : -__builtin_inff());
+        if (lane == 0) red[hh][wave] = mx;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nh) {
+        const float *r = red[threadIdx.x];
+        A.pm[(int64_t)(h0 + threadIdx.x) * A.nbs + blk] =
+            max_sel(max_sel(r[0], r[1]), max_sel(r[2], r[3]));
     }
 }
 
-// Positions b + 16t .. b + 16t + 15 of a row for thread t: two 8-groups.
-struct SoftBlock {
-    float v[16];
-};
-
-__device__ inline void load_soft_block(const float *row, int b, SoftBlock &blk) {
-    const float4 *p = reinterpret_cast<const float4 *>(row + b + 16 * threadIdx.x);
+// ---- softmax pieces ---------------------------------------------------------------
+//
+// Four consecutive positions j .. j + 3 (j a multiple of 4) of a head per
+// thread, neighbours (lane ^ 1) sharing an 8-group. x: their scores, on
+// return their exponentials. Returns the thread's share of the total: the
+// 8-group's float sum in the reference's lane order from its even thread,
+// nothing from the tail [gend, n). Every lane of the wave takes part.
+//
+// The tail, at most seven positions, is left to as many lanes of one wave
+// (tail_exp is a double exp: evaluated four times in turn by the thread that
+// holds the positions it cost 2 us of a launch).
+__device__ inline double exp4(float (&x)[4], int j, int gend, float mx) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float4 f = p[i];
-        blk.v[4 * i] = f.x;
-        blk.v[4 * i + 1] = f.y;
-        blk.v[4 * i + 2] = f.z;
-        blk.v[4 * i + 3] = f.w;
+    for (int e = 0; e < 4; e++) x[e] = expf_poly(x[e] - mx);
+    float a[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float o = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x[e]), kDppXor1, 0xf, 0xf, false));
+        a[e] = x[e] + o;
     }
+    return j < gend && !(j & 4) ? (double)((a[0] + a[2]) + (a[1] + a[3])) : 0.0;
 }
 
-// Grid n_head: one workgroup per query head. The max, the total and the
-// f16 probabilities each take one pass over the row in blocks of
-// kAttnBlock positions; with n <= kAttnBlock the block stays in registers
-// and its exponentials are evaluated once.
-__global__ __launch_bounds__(kAttnThreads) void attn_softmax_kernel(AttnArgs A) {
-    __shared__ float redf[kAttnThreads / 64];
-    __shared__ double redd[kAttnThreads / 64];
-    const int h = blockIdx.x;
-    const float *row = A.sw + (int64_t)h * A.lw;
-    const int n = A.n, gend = n & ~7;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const bool one = n <= kAttnBlock;
-    SoftBlock blk;
+// Grid ceil(n / 1024) x n_head in one dimension (attn_wg): the exponentials
+// of a block of 1024 positions of a head, in place of its scores, and their
+// total. The whole softmax in one workgroup per head took 14 us at n = 7000
+// (three passes over the row by 32 workgroups); spread over the positions it
+// takes 2-4.5 us, a launch's latency.
+constexpr int kAttnExpBlock = 1024;
+
+__global__ __launch_bounds__(256) void attn_exp_kernel(AttnArgs A) {
+    __shared__ float redf[4];
+    __shared__ double redd[4];
+    const AttnWg W = attn_wg(A);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int j = W.blk * kAttnExpBlock + 4 * (int)threadIdx.x;
+    float4 *const p = reinterpret_cast<float4 *>(A.sw + (int64_t)W.h * A.lw + j);
+    const float4 f = *p;  // lw is a multiple of the block
+    // tail position gend + tid, where it lies in this block
+    const int gend = A.n & ~7, jt = gend + (int)threadIdx.x;
+    const bool tail = jt < A.n && gend / kAttnExpBlock == W.blk;
+    float *const pt = A.sw + (int64_t)W.h * A.lw + jt;
+    float xt = 0.0f;
+    if (tail) xt = *pt;
     float mx = -__builtin_inff();
-    for (int b = 0; b < n; b += kAttnBlock) {
-        load_soft_block(row, b, blk);
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-            if (b + 16 * (int)threadIdx.x + e < n && blk.v[e] > mx) mx = blk.v[e];
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const float t = __shfl_xor(mx, o);
-        mx = t > mx ? t : mx;
-    }
+    for (int i = threadIdx.x; i < A.nbs; i += 256) mx = max_sel(mx, A.pm[(int64_t)W.h * A.nbs + i]);
+    mx = wave_max(mx);
     if (lane == 0) redf[wave] = mx;
     __syncthreads();
-    mx = redf[0];
-    for (int i = 1; i < kAttnThreads / 64; i++) mx = redf[i] > mx ? redf[i] : mx;
-    // total: the 8-groups (lane order of the reference's 8-wide sum), then
-    // the tail
-    // the thread whose 16 positions hold the tail [gend, n)
-    const int tail_b = gend / kAttnBlock * kAttnBlock;
-    const bool tail_owner = gend < n && (int)threadIdx.x == (gend - tail_b) / 16;
-    double part = 0.0;
-    float ex[16];
-    for (int b = 0; b < n; b += kAttnBlock) {
-        if (!one) load_soft_block(row, b, blk);
-#pragma unroll
-        for (int e = 0; e < 16; e++) ex[e] = expf_poly(blk.v[e] - mx);
-#pragma unroll
-        for (int g = 0; g < 2; g++) {
-            const int j0 = b + 16 * (int)threadIdx.x + 8 * g;
-            const float *v = ex + 8 * g;
-            if (j0 + 8 <= gend)
-                part += (double)(((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7])));
-        }
+    mx = max_sel(max_sel(redf[0], redf[1]), max_sel(redf[2], redf[3]));
+    float x[4] = {f.x, f.y, f.z, f.w};
+    double part = exp4(x, j, gend, mx);
+    if (tail) {
+        xt = tail_exp(xt - mx);
+        part += (double)xt;
+        *pt = xt;
     }
-    if (tail_owner)
-        for (int j = gend; j < n; j++) part += (double)tail_exp(row[j] - mx);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) part += __shfl_xor(part, o);
+    part = wave_sum(part);
+    if (j < gend) *p = make_float4(x[0], x[1], x[2], x[3]);
     if (lane == 0) redd[wave] = part;
     __syncthreads();
-    part = redd[0];
-    for (int i = 1; i < kAttnThreads / 64; i++) part += redd[i];
-    const float scale = (float)(1.0 / part);
-    uint16_t *pw = A.pw + (int64_t)h * A.lw;
-    for (int b = 0; b < n; b += kAttnBlock) {
-        if (!one) {
-            load_soft_block(row, b, blk);
-#pragma unroll
-            for (int e = 0; e < 16; e++) ex[e] = expf_poly(blk.v[e] - mx);
-        }
-        const int j0 = b + 16 * (int)threadIdx.x;
-        uint32_t pk[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            pk[e] = (uint32_t)f32_to_f16_bits(ex[2 * e] * scale) |
-                    ((uint32_t)f32_to_f16_bits(ex[2 * e + 1] * scale) << 16);
-        // whole 32-byte pieces into the workspace row (lw entries)
-        uint4 *dst = reinterpret_cast<uint4 *>(pw + j0);
-        dst[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-        dst[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
-        if (A.p16)
-            for (int e = 0; e < 16 && j0 + e < n; e++)
-                A.p16[(int64_t)h * A.ld + j0 + e] = (uint16_t)(pk[e >> 1] >> (16 * (e & 1)));
-    }
-    // the tail's probabilities replace the polynomial's (same thread, later stores)
-    if (tail_owner)
-        for (int j = gend; j < n; j++) {
-            const uint16_t pb = f32_to_f16_bits(tail_exp(row[j] - mx) * scale);
-            pw[j] = pb;
-            if (A.p16) A.p16[(int64_t)h * A.ld + j] = pb;
-        }
+    if (threadIdx.x == 0)
+        A.ps[(int64_t)W.h * A.nbe + W.blk] = (redd[0] + redd[1]) + (redd[2] + redd[3]);
 }
 
-// Grid (ceil(hd / kAttnPvRows), n_head_kv * ceil(gqa / kAttnHeads)):
-// each workgroup owns kAttnPvRows value rows of one KV head and up to
-// kAttnHeads query heads of it, wave w running head h0 + w. Per chunk of
-// kAttnChunk positions every thread requests its share of the value rows
-// and probability rows at once, stores them to LDS, and each wave runs its
-// accumulator chains over the chunk: lane 8r + L holds accumulators
-// 4L..4L+3 of row r. Then the reduction tree, the tail (inside the last
-// chunk) and the store.
-constexpr int kAttnPvRows = 8;
-constexpr int kAttnChunk = 2048;  // positions per LDS chunk (a multiple of 32, divides kAttnBlock)
-constexpr int kAttnVPieces = kAttnPvRows * kAttnChunk / 8 / kAttnThreads;  // 16-byte pieces
-constexpr int kAttnPPieces = kAttnHeads * kAttnChunk / 8 / kAttnThreads;
+// ---- values -----------------------------------------------------------------------
+//
+// Grid ceil(hd / 16) x n_head in one dimension (attn_wg): a workgroup owns 16
+// value rows of one query head; lane (row r, L < 16) runs accumulators 2 L
+// and 2 L + 1 of row r. The value rows and the head's exponentials stream
+// into LDS by DMA in chunks of 512 positions, three chunks ahead of the
+// chains, so the loads are bound by the memory and not by a round trip per
+// chunk (staged through registers 2048 positions at a time, one chunk's
+// loads after the other's chains, 13.6 us at n = 7000), and each chunk's
+// probabilities are made while the chunk before runs, so that a chunk costs
+// one barrier. Row slots are padded by 64 bytes so that the four rows of a
+// wave read distinct LDS banks.
+constexpr int kAttnPvRows = 16;
+constexpr int kAttnChunk = 512;
+constexpr int kAttnRing = 4;
+constexpr int kAttnRowSlot = kAttnChunk * 2 + 64;
+constexpr int kAttnSlot = kAttnPvRows * kAttnRowSlot;
 
-// VEC: n_ctx % 8 == 0 and v 16-byte aligned (16-byte value pieces).
-// NG > 0 (n <= 512 NG <= kAttnChunk, one chunk): wave w computes the
-// softmax of head h0 + w itself (wave_softmax<NG>, from the scores launch's
-// scores) into its LDS probability row while the value rows load, in place
-// of loading probabilities; the caller's probs16 is written by the
-// workgroups of blockIdx.x == 0.
-template <bool VEC, int NG>
-__global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(AttnArgs A) {
-    __shared__ __attribute__((aligned(16))) uint16_t sv[kAttnPvRows * kAttnChunk];
-    __shared__ __attribute__((aligned(16))) uint16_t sp[kAttnHeads * kAttnChunk];
-    const int chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
-    const int hk = blockIdx.y / chunks;
-    const int h0 = hk * A.gqa + (blockIdx.y % chunks) * kAttnHeads;
-    const int nh = min(kAttnHeads, hk * A.gqa + A.gqa - h0);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bool active = wave < nh;
+typedef int attn_rsrc_t __attribute__((ext_vector_type(4)));
+
+// Copies of 1 KiB (16 bytes per lane) from a buffer straight into LDS, at
+// buffer offset voff (range-checked: zeros past the buffer's end), LDS byte
+// offset lds (wave-uniform). They are in flight until the wave's vmcnt covers
+// them; the compiler does not count them, so every use is behind an explicit
+// wait. The compiler's own m0 is put back.
+__device__ inline void attn_dma(attn_rsrc_t rsrc, uint32_t voff, uint32_t lds) {
+    uint32_t m0;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(m0)
+        : "s"(lds), "v"(voff), "s"(rsrc)
+        : "memory");
+}
+// Four of them at voff[i] + add, the LDS offset advancing by kAttnRowSlot.
+__device__ inline void attn_dma_rows(attn_rsrc_t rsrc, const uint32_t (&voff)[4], uint32_t add,
+                                     uint32_t lds) {
+    uint32_t m0;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %6, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, %7\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %3, %6, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, %7\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %4, %6, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, %7\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %5, %6, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(m0)
+        : "s"(lds), "v"(voff[0] + add), "v"(voff[1] + add), "v"(voff[2] + add), "v"(voff[3] + add),
+          "s"(rsrc), "n"(kAttnRowSlot)
+        : "memory", "scc");
+}
+
+__device__ inline attn_rsrc_t attn_rsrc(const void *p, uint32_t bytes) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    return (attn_rsrc_t){__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                         __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xffff),
+                         __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
+}
+
+// The tree over the 32 accumulators of one row, 32 / NL per lane in lanes
+// L = 0 .. NL - 1 of the row (acc[e] = accumulator 32 / NL * L + e); valid in
+// L == 0. Every lane of the wave takes part.
+__device__ inline float row_tree2(float a0, float a1) {  // 16 lanes, 2 each
+    a0 += from_lane_up<8>(a0), a1 += from_lane_up<8>(a1);  // r0 + r2, r1 + r3
+    a0 += from_lane_up<4>(a0), a1 += from_lane_up<4>(a1);  // their sum
+    a0 += from_lane_up<2>(a0), a1 += from_lane_up<2>(a1);  // l and l + 4
+    const float b = a0 + a1;
+    return b + from_lane_up<1>(b);
+}
+__device__ inline float row_tree1(float a) {  // 32 lanes, 1 each
+    a += __shfl_down(a, 16);
+    a += from_lane_up<8>(a);
+    a += from_lane_up<4>(a);
+    a += from_lane_up<1>(a);
+    return a + from_lane_up<2>(a);
+}
+
+// res plus the tail [body, n) of a dot, added in order in double; v and p:
+// f16 rows of the 32-element block at body (16-byte aligned LDS).
+__device__ inline float add_tail(float res, const uint16_t *v, const uint16_t *p, int cnt) {
+    double total = 0.0;
+    total += (double)res;
+    if (cnt > 0) {
+        h8_t vv[4], pp[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            vv[i] = reinterpret_cast<const h8_t *>(v)[i];
+            pp[i] = reinterpret_cast<const h8_t *>(p)[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 31; i++)
+            if (i < cnt) total += (double)((float)vv[i >> 3][i & 7] * (float)pp[i >> 3][i & 7]);
+    }
+    return (float)total;
+}
+
+// VEC: n_ctx % 8 == 0, v 16-byte aligned and the workgroup's rows within a
+// buffer's 4 GiB; else the value rows are staged by single elements, a chunk
+// at a time.
+template <bool VEC>
+__global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
+    constexpr int kR = VEC ? kAttnRing : 1;
+    __shared__ __attribute__((aligned(16))) uint8_t ring[kR * kAttnSlot];
+    __shared__ __attribute__((aligned(16))) float se[kR][kAttnChunk];
+    __shared__ __attribute__((aligned(16))) uint16_t sp[2][kAttnChunk];
+    const AttnWg W = attn_wg(A);
+    const int tid = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int r = tid >> 4, L = tid & 15;
+    const int rows = min(kAttnPvRows, A.hd - W.blk * kAttnPvRows);
     const int n = A.n, body = n & ~31;
-    const int r = lane >> 3, L = lane & 7;
-    const int c = blockIdx.x * kAttnPvRows + r;
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    int s0 = 0;
-    for (;; s0 += kAttnChunk) {
-        const int cl = min(kAttnChunk, n - s0);
-        const int per_row = (cl + 7) / 8;  // 16-byte pieces of a row in this chunk
-        // probability rows: whole pieces of the workspace (lw >= s0 + kAttnChunk);
-        // heads past nh repeat head nh - 1
-        uint4 pq[kAttnPPieces];
-        if constexpr (NG == 0) {
+    const uint16_t *const vb = A.v + ((int64_t)W.hk * A.hd + W.blk * kAttnPvRows) * A.n_ctx;
+    const float *const eb = A.sw + (int64_t)W.h * A.lw;
+    const int nchunk = (n + kAttnChunk - 1) / kAttnChunk;
+    const uint32_t lds_v = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)ring;
+    const uint32_t lds_e = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)&se[0][0];
+    attn_rsrc_t vr, er;
+    if constexpr (VEC) {
+        vr = attn_rsrc(vb, (uint32_t)(rows * A.n_ctx * 2));
+        er = attn_rsrc(eb, (uint32_t)(A.lw * 4));
+    }
+    // this wave's KiB of chunk ch's exponentials (waves 2 and 3 copy what 0
+    // and 1 copy, the same bytes, so that every wave issues the same number)
+    uint32_t voff[4];
 #pragma unroll
-            for (int i = 0; i < kAttnPPieces; i++) {
-                const int t = threadIdx.x + kAttnThreads * i;
-                const int hh = min(t / (kAttnChunk / 8), nh - 1), pc = t % (kAttnChunk / 8);
-                pq[i] = reinterpret_cast<const uint4 *>(A.pw + (int64_t)(h0 + hh) * A.lw + s0)[pc];
-            }
+    for (int i = 0; i < 4; i++) voff[i] = (uint32_t)(4 * wave + i) * (uint32_t)(A.n_ctx * 2) + lane * 16;
+    const uint32_t voff_e = (uint32_t)(wave & 1) * 1024 + lane * 16;
+    auto uni = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+    auto dma_e = [&](int ch) {
+        const uint32_t cc = (uint32_t)min(ch, nchunk - 1);
+        attn_dma(er, voff_e + cc * (kAttnChunk * 4),
+                 uni(lds_e + (uint32_t)(ch % kR) * (kAttnChunk * 4) + (wave & 1) * 1024));
+    };
+    // value rows 4 wave .. + 3 of chunk ch (rows past hd read zeros), then
+    // the exponentials of chunk ch + 1; chunks past the end copy the last one
+    // again
+    auto dma = [&](int ch) {
+        const uint32_t cc = (uint32_t)min(ch, nchunk - 1);
+        attn_dma_rows(vr, voff, cc * (kAttnChunk * 2),
+                      uni(lds_v + (uint32_t)(ch % kR) * kAttnSlot + 4 * wave * kAttnRowSlot));
+        dma_e(ch + 1);
+    };
+    // 1 / total, the block totals added in a fixed order
+    double part = 0.0;
+    for (int i = lane; i < A.nbe; i += 64) part += A.ps[(int64_t)W.h * A.nbe + i];
+    if constexpr (VEC) {
+        dma_e(0);
+#pragma unroll
+        for (int i = 0; i + 1 < kR; i++) dma(i);
+    }
+    const float scale = (float)(1.0 / wave_sum(part));
+    // the probabilities of chunk ch from its exponentials e
+    auto put_p = [&](int ch, float2 e) {
+        const uint32_t p0 = f32_to_f16_hw(e.x * scale), p1 = f32_to_f16_hw(e.y * scale);
+        reinterpret_cast<uint32_t *>(sp[ch & 1])[tid] = p0 | (p1 << 16);
+        if (A.p16 && W.blk == 0) {
+            const int64_t j = (int64_t)ch * kAttnChunk + 2 * tid;
+            if (j < n) A.p16[(int64_t)W.h * A.ld + j] = (uint16_t)p0;
+            if (j + 1 < n) A.p16[(int64_t)W.h * A.ld + j + 1] = (uint16_t)p1;
         }
-        if constexpr (VEC) {
-            // value rows (rows past hd repeat row hd - 1); pieces past the
-            // chunk's end load the chunk's last piece again (n_ctx % 8 == 0:
-            // it ends inside the row)
-            uint4 vq[kAttnVPieces];
-#pragma unroll
-            for (int i = 0; i < kAttnVPieces; i++) {
-                const int t = threadIdx.x + kAttnThreads * i;
-                const int rr = t / (kAttnChunk / 8), pc = min(t % (kAttnChunk / 8), per_row - 1);
-                const int cr = min(blockIdx.x * kAttnPvRows + rr, A.hd - 1);
-                vq[i] = reinterpret_cast<const uint4 *>(
-                    A.v + ((int64_t)hk * A.hd + cr) * A.n_ctx + s0)[pc];
-            }
-#pragma unroll
-            for (int i = 0; i < kAttnVPieces; i++) {
-                const int t = threadIdx.x + kAttnThreads * i;
-                reinterpret_cast<uint4 *>(sv)[t] = vq[i];
-            }
-        } else {
-#pragma unroll 8
-            for (int t = threadIdx.x; t < kAttnPvRows * cl; t += kAttnThreads) {
-                const int rr = t / cl, i = t - rr * cl;
-                const int cr = min(blockIdx.x * kAttnPvRows + rr, A.hd - 1);
-                sv[rr * kAttnChunk + i] = A.v[((int64_t)hk * A.hd + cr) * A.n_ctx + s0 + i];
-            }
-        }
-        if constexpr (NG > 0) {
-            if (active) wave_softmax<NG>(A, h0 + wave, lane, sp + wave * kAttnChunk, blockIdx.x == 0);
-        } else {
-#pragma unroll
-            for (int i = 0; i < kAttnPPieces; i++)
-                reinterpret_cast<uint4 *>(sp)[threadIdx.x + kAttnThreads * i] = pq[i];
-        }
+    };
+    if constexpr (VEC) {
+        // the first exponentials: 15 younger copies
+        static_assert(kAttnRing == 4, "wait counts");
+        asm volatile("s_waitcnt vmcnt(15)" ::: "memory");
         __syncthreads();
-        // the accumulator chains over the chunk's whole 32-steps
-        if (active) {
-            const uint16_t *vr = sv + r * kAttnChunk;
-            const uint16_t *pr = sp + wave * kAttnChunk;
-            const int steps_end = min(body - s0, cl);
+        put_p(0, reinterpret_cast<const float2 *>(se[0])[tid]);
+    }
+    float a0 = 0.0f, a1 = 0.0f;
+    const uint8_t *slot = ring;
+    for (int ch = 0; ch < nchunk; ch++) {
+        const int s0 = ch * kAttnChunk;
+        if constexpr (VEC) {
+            slot = ring + ch % kR * kAttnSlot;
+            // chunk ch and the next exponentials have arrived (two younger
+            // chunks of five copies in flight), this chunk's probabilities
+            // are written, and every wave is done with chunk ch - 1
+            asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+            __syncthreads();
+            dma(ch + kR - 1);
+        } else {
+            __syncthreads();
+            for (int i = tid; i < kAttnPvRows * kAttnChunk; i += 256) {
+                const int rr = i / kAttnChunk, e = i % kAttnChunk;
+                if (s0 + e < n)
+                    reinterpret_cast<uint16_t *>(ring + rr * kAttnRowSlot)[e] =
+                        vb[(int64_t)min(rr, rows - 1) * A.n_ctx + s0 + e];
+            }
+            put_p(ch, reinterpret_cast<const float2 *>(eb + s0)[tid]);
+            __syncthreads();
+        }
+        const uint32_t *const vs = reinterpret_cast<const uint32_t *>(slot + r * kAttnRowSlot) + L;
+        const uint32_t *const ps = reinterpret_cast<const uint32_t *>(sp[ch & 1]) + L;
+        auto chain = [&](uint32_t vw, uint32_t pw) {
+            a0 = __builtin_fmaf(f16_bits_to_f32(vw & 0xffffu), f16_bits_to_f32(pw & 0xffffu), a0);
+            a1 = __builtin_fmaf(f16_bits_to_f32(vw >> 16), f16_bits_to_f32(pw >> 16), a1);
+        };
+        const int steps = min(body - s0, kAttnChunk) >> 5;
+        if (VEC && steps == kAttnChunk / 32) {
+            // a whole chunk: all its reads go out first
+            uint32_t vw[kAttnChunk / 32], pw[kAttnChunk / 32];
+            const float2 e = reinterpret_cast<const float2 *>(se[(ch + 1) % kR])[tid];
+#pragma unroll
+            for (int t = 0; t < kAttnChunk / 32; t++) vw[t] = vs[16 * t], pw[t] = ps[16 * t];
+            put_p(ch + 1, e);
+#pragma unroll
+            for (int t = 0; t < kAttnChunk / 32; t++) chain(vw[t], pw[t]);
+        } else {
+            if (VEC && ch + 1 < nchunk) put_p(ch + 1, reinterpret_cast<const float2 *>(se[(ch + 1) % kR])[tid]);
 #pragma unroll 4
-            for (int i0 = 0; i0 < steps_end; i0 += 32) {
-                const int i = i0 + 4 * L;
-                const uint2 vw = *reinterpret_cast<const uint2 *>(vr + i);
-                const uint2 pw = *reinterpret_cast<const uint2 *>(pr + i);
-                acc[0] = __builtin_fmaf(f16_bits_to_f32(vw.x & 0xffffu), f16_bits_to_f32(pw.x & 0xffffu), acc[0]);
-                acc[1] = __builtin_fmaf(f16_bits_to_f32(vw.x >> 16), f16_bits_to_f32(pw.x >> 16), acc[1]);
-                acc[2] = __builtin_fmaf(f16_bits_to_f32(vw.y & 0xffffu), f16_bits_to_f32(pw.y & 0xffffu), acc[2]);
-                acc[3] = __builtin_fmaf(f16_bits_to_f32(vw.y >> 16), f16_bits_to_f32(pw.y >> 16), acc[3]);
+            for (int t = 0; t < steps; t++) chain(vs[16 * t], ps[16 * t]);
+        }
+    }
+    const float res = row_tree2(a0, a1);
+    // the tail lies in the last chunk, still in LDS
+    if (L == 0 && r < rows) {
+        const int b0 = body % kAttnChunk;
+        A.out[(int64_t)W.h * A.hd + W.blk * kAttnPvRows + r] =
+            add_tail(res, reinterpret_cast<const uint16_t *>(slot + r * kAttnRowSlot) + b0,
+                     sp[(nchunk - 1) & 1] + b0, n - body);
+    }
+    // no copy may land in the LDS of a workgroup that has ended
+    if constexpr (VEC) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// ---- one launch -------------------------------------------------------------------
+//
+// Grid ceil(hd / 16) x n_head in one dimension (attn_wg), 8 waves: a
+// workgroup scores all n positions of its query head (16 rows per wave and
+// pass, the next pass's key rows in flight), runs the softmax in LDS
+// and the chains of its 16 value rows, one accumulator per thread. Every
+// workgroup of a head repeats the scores (hd / 16 times the score work, n *
+// hd * 2 bytes from the L2 each), which costs less than the launches and
+// round trips through memory that it saves until the rows grow long (8B
+// shape, per layer: n = 600 15.5 -> 8.6 us against a scores launch and a value
+// launch with the softmax in it). What bounds it: 6 us at n = 16, the chain of
+// one launch's start, the key and query loads, three barriers and the store.
+// LDS (dynamic, attn_fused_lds): scores, probabilities, value rows, query.
+constexpr int kAttnFusedThreads = 512;
+constexpr int kAttnFuseMax = 1024;
+constexpr int kAttnFuseCap = 1536;  // the largest the kernel takes (64 KiB of LDS)
+
+__host__ __device__ inline int attn_fused_np(int n) { return (n + 31) / 32 * 32; }
+__host__ __device__ inline int attn_fused_lds(int n) {
+    const int np = attn_fused_np(n);
+    return np * 4 + np * 2 + kAttnPvRows * (np * 2 + 64) + kAttnMaxHd * 2;
+}
+
+template <int T, bool VEC>
+__global__ __launch_bounds__(kAttnFusedThreads)
+__attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(AttnArgs A) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    __shared__ float redf[8];
+    __shared__ double redd[8];
+    const AttnWg W = attn_wg(A);
+    const int n = A.n, np = attn_fused_np(n), hd = A.hd;
+    uint16_t *const sq = reinterpret_cast<uint16_t *>(smem);
+    float *const ss = reinterpret_cast<float *>(smem + kAttnMaxHd * 2);
+    uint16_t *const sp = reinterpret_cast<uint16_t *>(ss + np);
+    uint8_t *const sv = reinterpret_cast<uint8_t *>(sp + np);
+    const int vslot = np * 2 + 64;
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    // scores: 128 positions per pass, four lanes each
+    const int L4 = lane & 3, jr = tid >> 2;
+    const uint16_t *const kb = A.k + (int64_t)W.hk * A.n_ctx * hd;
+    auto key_row = [&](int pass) {
+        const int j = 128 * pass + jr;
+        return kb + (int64_t)(j < n ? j : n - 1) * hd;
+    };
+    const int passes = (n + 127) / 128;
+    constexpr int kD = T <= 4 ? 2 : 1;  // passes of key rows held
+    KeyRow<T> kr[kD];
+    load_key<T, VEC>(key_row(0), hd, L4, kr[0]);
+    float qv = 0.0f;
+    if (tid < hd) qv = A.q[(int64_t)W.h * hd + tid];
+#pragma unroll
+    for (int i = 1; i < kD; i++)
+        if (i < passes) load_key<T, VEC>(key_row(i), hd, L4, kr[i]);
+    // value rows: 32 lanes per row; rows past hd repeat the last, positions
+    // past n are not used
+    const int r = tid >> 5, a = tid & 31;
+    const int c = W.blk * kAttnPvRows + r;
+    const uint16_t *const vrow = A.v + ((int64_t)W.hk * hd + min(c, hd - 1)) * A.n_ctx;
+    constexpr int kVP = kAttnFuseCap / 256;
+    const int per8 = (n + 7) / 8;
+    uint4 vq[kVP];
+    if constexpr (VEC) {
+#pragma unroll
+        for (int i = 0; i < kVP; i++)
+            vq[i] = 32 * i < per8 ? reinterpret_cast<const uint4 *>(vrow)[min(32 * i + a, per8 - 1)]
+                                  : make_uint4(0, 0, 0, 0);
+    }
+    if (tid < hd) sq[tid] = (uint16_t)f32_to_f16_hw(qv);
+    __syncthreads();
+    KeyRow<T> qr;
+    load_key<T, true>(sq, hd, L4, qr);
+    float mx = -__builtin_inff();
+    for (int p0 = 0; p0 < passes; p0 += kD) {
+#pragma unroll
+        for (int u = 0; u < kD; u++) {
+            const int pass = p0 + u;
+            if (pass < passes) {
+                const float v = key_score<T, VEC>(kr[u], qr, key_row(pass), sq, hd, L4, A.kq_scale);
+                if (pass + kD < passes) load_key<T, VEC>(key_row(pass + kD), hd, L4, kr[u]);
+                const int j = 128 * pass + jr;
+                if (L4 == 0 && j < n) {
+                    ss[j] = v;
+                    mx = max_sel(mx, v);
+                    if (A.sc && W.blk == 0) A.sc[(int64_t)W.h * A.ld + j] = v;
+                }
             }
         }
-        if (s0 + cl >= n) break;
-        __syncthreads();  // the next chunk overwrites sv and sp
     }
-    // the tail [body, n) lies in the last chunk, still in LDS
-    const float res = dot_tree(acc);
-    if (active && L == 0 && c < A.hd) {
-        const int h = h0 + wave;
-        double total = 0.0;
-        total += (double)res;
-        for (int j = body; j < n; j++)
-            total += (double)(f16_bits_to_f32(sv[r * kAttnChunk + j - s0]) *
-                              f16_bits_to_f32(sp[wave * kAttnChunk + j - s0]));
-        A.out[(int64_t)h * A.hd + c] = (float)total;
+    if constexpr (VEC) {
+#pragma unroll
+        for (int i = 0; i < kVP; i++)
+            if (32 * i + a < per8) *reinterpret_cast<uint4 *>(sv + r * vslot + (32 * i + a) * 16) = vq[i];
+    } else {
+        for (int i = a; i < n; i += 32) reinterpret_cast<uint16_t *>(sv + r * vslot)[i] = vrow[i];
     }
+    mx = wave_max(mx);
+    if (lane == 0) redf[wave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++) mx = max_sel(mx, redf[i]);
+    const int j = 4 * tid;
+    float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (j < np) {
+        const float4 f = *reinterpret_cast<const float4 *>(ss + j);
+        x[0] = f.x, x[1] = f.y, x[2] = f.z, x[3] = f.w;
+    }
+    // tail position gend + tid
+    const int gend = n & ~7, jt = gend + tid;
+    double part = exp4(x, j, gend, mx);
+    float xt = 0.0f;
+    if (jt < n) {
+        xt = tail_exp(ss[jt] - mx);
+        part += (double)xt;
+    }
+    part = wave_sum(part);
+    if (lane == 0) redd[wave] = part;
+    __syncthreads();
+    part = ((redd[0] + redd[1]) + (redd[2] + redd[3])) + ((redd[4] + redd[5]) + (redd[6] + redd[7]));
+    const float scale = (float)(1.0 / part);
+    auto out_p = [&](int jj, uint32_t p) {
+        if (A.p16 && W.blk == 0) A.p16[(int64_t)W.h * A.ld + jj] = (uint16_t)p;
+    };
+    if (j < gend) {
+        uint32_t p[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            p[e] = f32_to_f16_hw(x[e] * scale);
+            out_p(j + e, p[e]);
+        }
+        *reinterpret_cast<uint2 *>(sp + j) = make_uint2(p[0] | (p[1] << 16), p[2] | (p[3] << 16));
+    }
+    if (jt < n) {
+        const uint32_t p = f32_to_f16_hw(xt * scale);
+        sp[jt] = (uint16_t)p;
+        out_p(jt, p);
+    }
+    __syncthreads();
+    const uint16_t *const vs = reinterpret_cast<const uint16_t *>(sv + r * vslot);
+    const int body = n & ~31;
+    float acc = 0.0f;
+#pragma unroll 8
+    for (int i = a; i < body; i += 32) acc = __builtin_fmaf(f16_bits_to_f32(vs[i]), f16_bits_to_f32(sp[i]), acc);
+    const float res = row_tree1(acc);
+    if (a == 0 && c < hd) A.out[(int64_t)W.h * hd + c] = add_tail(res, vs + body, sp + body, n - body);
 }
 
 }  // namespace sihip

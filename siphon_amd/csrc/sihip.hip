@@ -52,7 +52,7 @@ struct Options {
     int64_t gemmq_xmode = -1;  // Q8_0-pair GEMM record mode 0 or 1 (gemmq_kernel XM; rule: 1 where it fits)
     int64_t gemmq_fuse = -1;   // Q8_0-pair GEMM quantizing X itself (XM 2) at 16-row m blocks, 0: off (rule: on)
     int64_t gemmh_fuse = -1;   // F16 GEMM converting X itself (XF) at 16-row m blocks, 0: off (rule: on)
-    int64_t attn_fuse = -1;    // decode attention in two launches up to 1024 positions (softmax in the value launch), 0: three
+    int64_t attn_fuse = -1;    // decode attention in one launch up to 512 k positions, 0: three (rule: kAttnFuseMax)
     int64_t gemm2s_max_m = -1; // largest M on the small-M Q4_K GEMM, 0: none (rule: 16)
     int64_t gemmks_max_m = -1; // largest M on the small-M K-quant GEMM, 0: none (rule: 16)
     int64_t gemmks_q4k = -1;   // Q4_K small M on gemmks.h (1) or gemm2s.h (0) (rule: 0)
@@ -2383,54 +2383,70 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
     A.n = (int)(pos + 1);
     A.hd = (int)head_dim;
     A.gqa = (int)(n_head / n_head_kv);
-    A.n_head = (int)n_head;
     A.kq_scale = kq_scale;
     A.sc = scores;    // NULL: not written
     A.p16 = probs16;  // NULL: not written
-    // workspace scores (f32) and probabilities (f16): rows of whole
-    // kAttnBlock blocks, so that block loads stay inside the allocation
-    A.lw = (A.n + kAttnBlock - 1) / kAttnBlock * kAttnBlock;
-    const int rc = ensure(ctx, &ctx->d_attn, &ctx->d_attn_cap, (size_t)(n_head * A.lw * 6),
-                          (hipStream_t)stream);
+    A.n_kv = (int)n_head_kv;
+    // workspace: the blocks' totals and maxima, and the scores (later the
+    // exponentials) in rows of whole kAttnWsBlock positions, so that block
+    // loads stay inside the allocation
+    A.lw = (A.n + kAttnWsBlock - 1) / kAttnWsBlock * kAttnWsBlock;
+    const int64_t ps_bytes = (n_head * (A.lw / kAttnExpBlock) * 8 + 255) / 256 * 256;
+    const int64_t sw_bytes = n_head * A.lw * 4;
+    const int64_t pm_bytes = n_head * (A.lw / kAttnScoreBlock) * 4;
+    const int rc = ensure(ctx, &ctx->d_attn, &ctx->d_attn_cap,
+                          (size_t)(ps_bytes + sw_bytes + pm_bytes), (hipStream_t)stream);
     if (rc) return rc;
-    A.sw = (float *)ctx->d_attn;
-    A.pw = (uint16_t *)((uint8_t *)ctx->d_attn + n_head * A.lw * 4);
-    const int chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
-    const dim3 gs((unsigned)((A.n + kAttnRows - 1) / kAttnRows), (unsigned)(n_head_kv * chunks));
-    const dim3 gv((unsigned)((head_dim + kAttnPvRows - 1) / kAttnPvRows),
-                  (unsigned)(n_head_kv * chunks));
-    if (gs.y > 65535) return set_err(ctx, SIHIP_EINVAL, "attn_decode_dev: too many KV heads");
+    A.ps = (double *)ctx->d_attn;
+    A.sw = (float *)((uint8_t *)ctx->d_attn + ps_bytes);
+    A.pm = (float *)((uint8_t *)ctx->d_attn + ps_bytes + sw_bytes);
+    A.nbs = (A.n + kAttnScoreBlock - 1) / kAttnScoreBlock;
+    A.nbe = (A.n + kAttnExpBlock - 1) / kAttnExpBlock;
+    const int64_t chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
+    const int64_t row_blocks = (head_dim + kAttnPvRows - 1) / kAttnPvRows;
+    const int64_t gs = A.nbs * chunks * n_head_kv, ge = A.nbe * n_head, gv = row_blocks * n_head;
+    if (gs > INT32_MAX) return set_err(ctx, SIHIP_EINVAL, "attn_decode_dev: too many KV heads");
     const hipStream_t st = (hipStream_t)stream;
     const int orc = order_before(ctx, ctx->order, st);
     if (orc) return orc;
-    // wide loads where rows stay aligned: keys 8 bytes, value rows 16
-    const bool kvec = head_dim % 4 == 0 && (uintptr_t)k_cache % 8 == 0;
-    const bool vvec = n_ctx % 8 == 0 && (uintptr_t)v_cache % 16 == 0;
-    if (kvec)
-        hipLaunchKernelGGL(attn_scores_kernel<true>, gs, dim3(kAttnThreads), 0, st, A);
-    else
-        hipLaunchKernelGGL(attn_scores_kernel<false>, gs, dim3(kAttnThreads), 0, st, A);
-    // up to kAttnFuseMax positions the value launch's waves compute their
-    // heads' softmax themselves: no softmax launch (8B shape: 11.6 against
-    // 15.1 us per layer at position 511)
-    const int64_t fmax = ctx->opt.attn_fuse > 0 ? std::min<int64_t>(ctx->opt.attn_fuse * 512, 2048)
-                                                : kAttnFuseMax;
-    const int ng = ctx->opt.attn_fuse == 0 || A.n > fmax ? 0 : (A.n + 511) / 512;
-    if (ng == 0)
-        hipLaunchKernelGGL(attn_softmax_kernel, dim3((unsigned)n_head), dim3(kAttnThreads), 0, st, A);
-#define SIHIP_PV(V)                                                                                 \
-    switch (ng) {                                                                                   \
-        case 0: hipLaunchKernelGGL((attn_pv_kernel<V, 0>), gv, dim3(kAttnThreads), 0, st, A); break; \
-        case 1: hipLaunchKernelGGL((attn_pv_kernel<V, 1>), gv, dim3(kAttnThreads), 0, st, A); break; \
-        case 2: hipLaunchKernelGGL((attn_pv_kernel<V, 2>), gv, dim3(kAttnThreads), 0, st, A); break; \
-        default: hipLaunchKernelGGL((attn_pv_kernel<V, 4>), gv, dim3(kAttnThreads), 0, st, A); break; \
-    }
-    if (vvec) {
-        SIHIP_PV(true)
+    // wide loads where rows stay aligned (and, for the streamed value rows,
+    // a workgroup's 16 rows lie within a buffer's 4 GiB)
+    const bool kvec = head_dim % 8 == 0 && (uintptr_t)k_cache % 16 == 0;
+    const bool vvec = n_ctx % 8 == 0 && (uintptr_t)v_cache % 16 == 0 &&
+                      n_ctx * 2 * kAttnPvRows <= (int64_t)UINT32_MAX;
+    const bool narrow = head_dim < 160;  // key rows of at most 4 whole 32-steps
+    // one launch up to kAttnFuseMax positions (the ATTN_FUSE option k: 512 k,
+    // 0: never). One against three launches, us per layer: 32 heads of 128
+    // over 8 KV heads, n = 600 8.6 against 13.0, 1000 11.1 against 13.8, 1300
+    // 13.3 against 14.5, 1536 12.4 against 12.3; 40 heads 1000 14.1 against
+    // 15.1, 1300 17.1 against 16.4; 16 heads of 80 1000 11.7 against 11.9,
+    // 1300 13.8 against 12.7
+    const int64_t fmax = ctx->opt.attn_fuse >= 0
+                             ? std::min<int64_t>(ctx->opt.attn_fuse * 512, kAttnFuseCap)
+                             : kAttnFuseMax;
+    if (A.n <= fmax) {
+        const dim3 g((unsigned)gv), t(kAttnFusedThreads);
+        const size_t lds = (size_t)attn_fused_lds(A.n);
+        if (kvec && vvec && narrow)
+            hipLaunchKernelGGL((attn_fused_kernel<4, true>), g, t, lds, st, A);
+        else if (kvec && vvec)
+            hipLaunchKernelGGL((attn_fused_kernel<16, true>), g, t, lds, st, A);
+        else
+            hipLaunchKernelGGL((attn_fused_kernel<16, false>), g, t, lds, st, A);
     } else {
-        SIHIP_PV(false)
+        const dim3 g((unsigned)gs), t(256);
+        if (kvec && narrow)
+            hipLaunchKernelGGL((attn_scores_kernel<4, true>), g, t, 0, st, A);
+        else if (kvec)
+            hipLaunchKernelGGL((attn_scores_kernel<16, true>), g, t, 0, st, A);
+        else
+            hipLaunchKernelGGL((attn_scores_kernel<16, false>), g, t, 0, st, A);
+        hipLaunchKernelGGL(attn_exp_kernel, dim3((unsigned)ge), t, 0, st, A);
+        if (vvec)
+            hipLaunchKernelGGL(attn_pv_kernel<true>, dim3((unsigned)gv), t, 0, st, A);
+        else
+            hipLaunchKernelGGL(attn_pv_kernel<false>, dim3((unsigned)gv), t, 0, st, A);
     }
-#undef SIHIP_PV
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "attention launch: %s", hipGetErrorString(e));
     return order_after(ctx, ctx->order, st);

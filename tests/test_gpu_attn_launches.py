@@ -1,0 +1,35 @@
+"""The one-launch and three-launch forms of the decode attention at the edges
+of their blocks (16 value rows, 64 scored positions, 128 per scoring pass,
+512 positions per value chunk, 1024 per exponential block), each
+bit-identical to the oracle."""
+import numpy as np
+import pytest
+
+from .test_gpu_attn import bits, check, run_attn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,n_ctx,n", [
+    (4, 2, 128, 1040, 1024),   # the last length of the single launch; whole chunks
+    (4, 2, 128, 1040, 1025),   # a tail of one position in a chunk of its own
+    (4, 1, 64, 1032, 513),     # a chunk of one position
+    (6, 2, 24, 520, 520),      # rows end at the allocation's end; hd below a block of 32
+    (3, 3, 40, 136, 129),      # a second scoring pass of one position, a head tail of 8
+    (5, 1, 120, 2600, 2559),   # five heads on one KV head, a head tail of 24, 31 tail positions
+    (2, 2, 72, 1535, 1533),    # odd n_ctx: narrow value loads
+    (2, 1, 192, 2056, 2049),   # keys wider than four 32-steps, a third exponential block
+])
+@pytest.mark.parametrize("fuse", [0, 3], ids=["three_launches", "one_launch"])
+def test_block_edges(dev, oracle, option, n_head, n_kv, hd, n_ctx, n, fuse):
+    """ATTN_FUSE k: one launch up to 512 k positions, else three."""
+    option("ATTN_FUSE", fuse)
+    rng = np.random.default_rng(hd * 4099 + n)
+    q = rng.standard_normal(n_head * hd).astype(np.float32)
+    k = (rng.standard_normal(n_kv * n_ctx * hd) * 2).astype(np.float16).view(np.uint16)
+    v = rng.standard_normal(n_kv * hd * n_ctx).astype(np.float16).view(np.uint16)
+    kq = float(np.float32(1.0 / np.sqrt(np.float32(hd))))
+    want = oracle.attn_decode(q, k, v, n_head, n_kv, hd, n_ctx, n - 1, kq)
+    args = (dev, q, k, v, n_head, n_kv, hd, n_ctx, n - 1, kq)
+    check(run_attn(*args), want, n, f"hd={hd} n={n} fuse={fuse}")
+    assert np.array_equal(bits(run_attn(*args, caller_buffers=False)[0]), bits(want[0]))
