@@ -61,9 +61,11 @@ constexpr int kG2BN = 128;  // weight rows per workgroup
 //                       64 ks + 16 (l / 16) .. + 15 of the super-block
 //   [256 BM, 288 BM):   f16 group sums, 32 bytes per row
 //   [288 BM, 292 BM):   f32 block scale dx per row
-__host__ __device__ constexpr int g2_rec_bytes(int BM) { return (BM * 292 + 1023) / 1024 * 1024; }
+//   [292 BM, 296 BM):   int32 1152 times the sum of the row's quants (Q5_K)
+__host__ __device__ constexpr int g2_rec_bytes(int BM) { return (BM * 296 + 1023) / 1024 * 1024; }
 __host__ __device__ constexpr int g2_rec_bsum(int BM) { return 256 * BM; }
 __host__ __device__ constexpr int g2_rec_dx(int BM) { return 288 * BM; }
+__host__ __device__ constexpr int g2_rec_sx(int BM) { return 292 * BM; }
 
 // One 16-lane row per Q8_K block (row m, super-block c) of X; rows M..Mp-1
 // are zero. Grid: gemm2_quantize_grid(Mp * nb) workgroups of 256. (A wave
@@ -109,6 +111,12 @@ __global__ __launch_bounds__(kG2Threads) void gemm2_quantize_x(const float *x, i
     *reinterpret_cast<uint4 *>(R + (4 * mt + ks) * 1024 + (16 * g + (mr & 15)) * 16) = r.q;
     reinterpret_cast<_Float16 *>(R + g2_rec_bsum(BM) + mr * 32)[lane16] = (_Float16)(float)r.gsum;
     if (lane16 == 0) reinterpret_cast<float *>(R + g2_rec_dx(BM))[mr] = r.d;
+    int s = r.gsum;
+    s += __builtin_amdgcn_mov_dpp(s, kDppXor1, 0xf, 0xf, false);
+    s += __builtin_amdgcn_mov_dpp(s, kDppXor2, 0xf, 0xf, false);
+    s += __builtin_amdgcn_mov_dpp(s, kDppHalfMirror, 0xf, 0xf, false);
+    s += __builtin_amdgcn_mov_dpp(s, kDppMirror, 0xf, 0xf, false);
+    if (lane16 == 0) reinterpret_cast<int *>(R + g2_rec_sx(BM))[mr] = 1152 * s;
 }
 
 // ---- weight copy in the order of this kernel (Q4_K) ---------------------------

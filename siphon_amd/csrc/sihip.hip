@@ -25,6 +25,8 @@
 #include "gemm2s.h"
 #include "gemmks.h"
 #include "gemmkf.h"
+#include "gemmsk.h"
+#include "gemmx.h"
 #include "gemm6.h"
 #include "gemmh.h"
 #include "gemmq.h"
@@ -59,6 +61,8 @@ struct Options {
     int64_t gemms_waves = -1;  // waves per workgroup of the small-M GEMMs, 4 or 8 (rule: by rows)
     int64_t gemmkf_max_m = -1; // largest M on the fused small-M K-quant launch, 0: none (rule: 8)
     int64_t gemmkf_sbk = -1;   // its K-slice length in super-blocks, 0: fewest slices (rule: by tiles)
+    int64_t gemmsk_max_m = -1; // largest M on the short-prompt K-quant GEMM, 0: none (rule: kGemmSKMaxM)
+    int64_t gemmx_min_m = -1;  // smallest M on the K-quant GEMM of longer prompts, 0: never (rule: past GEMMSK_MAX_M)
     int64_t gemm_group = -1;   // Q4_K matrices over one X in one 16x16 GEMM launch, 0: off (rule: on)
     int64_t q80_scalar = -1;   // Q8_0 activations by the scalar quantizer (reference
                                // kernels.c:542-558, its SI_SCALAR mode), 1: on (rule: off)
@@ -83,7 +87,8 @@ static const OptionName kOptionNames[] = {
     {"GEMMKS_Q4K", &Options::gemmks_q4k},
     {"GEMMS_WAVES", &Options::gemms_waves},
     {"GEMMKF_MAX_M", &Options::gemmkf_max_m}, {"GEMMKF_SBK", &Options::gemmkf_sbk},
-    {"GEMM_GROUP", &Options::gemm_group},
+    {"GEMM_GROUP", &Options::gemm_group}, {"GEMMSK_MAX_M", &Options::gemmsk_max_m},
+    {"GEMMX_MIN_M", &Options::gemmx_min_m},
 };
 
 // Order of launches that share mutable device state across streams: a
@@ -1043,6 +1048,25 @@ static int64_t gemmkf_max_m(const Options &o) {
     return o.gemmkf_max_m >= 0 ? (o.gemmkf_max_m < kKFMaxM ? o.gemmkf_max_m : kKFMaxM) : kKFMaxM;
 }
 
+// Smallest M that takes the 16x16 Q4_K GEMM (gemm2.h); option GEMM2_MIN_M.
+// It needs two of its 128-row workgroups per CU to hide latency: at the
+// 14336 x 4096 shape it is faster from M = 512 (83 against 95 us per call;
+// M = 2048: 323 against 357 us) and slower at M = 256 (67 against 50 us).
+constexpr int64_t kGemm2MinM = 384;
+static int64_t gemm2_min_m(const Options &o) { return o.gemm2_min_m > 0 ? o.gemm2_min_m : kGemm2MinM; }
+
+// The short-prompt K-quant GEMM (gemmsk.h) takes M from 9 to kGemmSKMaxM, and
+// longer ones, short of kGemm2MinM, of small products: up to kGemmSKTiles
+// 32 x 16 output tiles with rows of at most kGemmSKMaxK (option GEMMSK_MAX_M: up to that M instead,
+// 0: never). 8B Q4_K_M layer, us per layer on the kernels before / gemmsk.h /
+// gemmx.h: M = 16 79 / 60 / 78, 37 123 / 79 / 94, 64 127 / 87 / 104, 96 155 /
+// 104 / 133, 130 197 / 140 / 144, 300 282 / 267 / 224; its q/k/v (192 blocks
+// of 32 rows) at M = 200 56 / 29 / 33 and 300 60 / 38 / 37, gate + up (896) at
+// M = 130 78 / 57 / 54, ffn_down (14336 long) at M = 130 43 / 44 / 41.
+constexpr int64_t kGemmSKMaxM = 112;
+constexpr int64_t kGemmSKTiles = 3600, kGemmSKMaxK = 8192;
+static int64_t gemmsk_max_m(const Options &o) { return o.gemmsk_max_m >= 0 ? o.gemmsk_max_m : kGemmSKMaxM; }
+
 // The near-GGUF-size K-quant copy of the small-M GEMM (gemmks.h).
 static int build_gemmks_copy(sihip_ctx *ctx, sihip_weight *w, hipStream_t st) {
     if (capturing(st))
@@ -1090,7 +1114,7 @@ extern "C" int sihip_weight_prepare_gemm(sihip_ctx *ctx, sihip_weight *w) {
         if (rc) return rc;
     }
     if (is_kquant(w->L.type) && !w->gsmall &&
-        (gemmkf_max_m(ctx->opt) > 0 ||
+        (gemmkf_max_m(ctx->opt) > 0 || gemmsk_max_m(ctx->opt) > 0 ||
          (gemmks_max_m(ctx->opt, w->L.type) > 0 &&
           !(w->L.type == T_Q4_K && ctx->opt.gemmks_q4k != 1)))) {
         const int rc = build_gemmks_copy(ctx, w, ctx->stream);
@@ -1100,12 +1124,6 @@ extern "C" int sihip_weight_prepare_gemm(sihip_ctx *ctx, sihip_weight *w) {
     return SIHIP_OK;
 }
 
-// Smallest M that takes the 16x16 Q4_K GEMM (gemm2.h); option GEMM2_MIN_M.
-// It needs two of its 128-row workgroups per CU to hide latency: at the
-// 14336 x 4096 shape it is faster from M = 512 (83 against 95 us per call;
-// M = 2048: 323 against 357 us) and slower at M = 256 (67 against 50 us).
-constexpr int64_t kGemm2MinM = 384;
-static int64_t gemm2_min_m(const Options &o) { return o.gemm2_min_m > 0 ? o.gemm2_min_m : kGemm2MinM; }
 // Largest M that takes the small-M Q4_K GEMM (gemm2s.h; at most its 16-row
 // m tile); option GEMM2S_MAX_M, 0 turns it off.
 static int64_t gemm2s_max_m(const Options &o) {
@@ -1981,6 +1999,387 @@ static int run_gemmkf(sihip_ctx *ctx, int count, const sihip_weight *const *wc, 
     return order_after(ctx, ctx->order, st);
 }
 
+// The activation planes of a K-quant product of M rows: `need` bytes, and
+// outside capture as much as any of its kernels asks for at any smaller M (at
+// most 320 bytes per row and super-block, and a third or seven more 16-row
+// tiles than M has), so that a capture of such a call finds them whichever
+// kernel each of the two takes.
+static int ensure_planes(sihip_ctx *ctx, const Layout &L, int64_t M, size_t need, hipStream_t st) {
+    if (is_kquant(L.type) && M >= 9 && L.n_in % 256 == 0 && !capturing(st)) {
+        const int64_t tiles = (M + 15) / 16;
+        need = std::max(need, (size_t)((tiles + std::max<int64_t>(7, tiles / 3 + 1)) *
+                                       (L.n_in / 256) * g2_rec_bytes(16)));
+    }
+    return ensure(ctx, &ctx->d_ws, &ctx->d_ws_cap, need, st);
+}
+
+// ---- the short-prompt K-quant launch (gemmsk.h) -------------------------------
+
+// m blocks of 16 mt rows, mt at most 3 (what the registers hold), as few as
+// cover M's 16-row tiles, as even as they go.
+struct SKPlan {
+    int mt, MB;
+    int64_t Mp, ws_bytes;
+};
+static SKPlan plan_gemmsk(int64_t M, int64_t nb) {
+    const int64_t tiles = (M + 15) / 16;
+    SKPlan p;
+    p.MB = (int)((tiles + 2) / 3);
+    p.mt = (int)((tiles + p.MB - 1) / p.MB);
+    p.Mp = (int64_t)p.MB * p.mt * 16;
+    p.ws_bytes = p.Mp / 16 * nb * g2_rec_bytes(16);
+    return p;
+}
+
+// Whether weights over one X take this launch: K-quants of one row length
+// and M in its range, unless an option sets the tiling of the other GEMMs.
+// Under graph capture, where a missing weight copy cannot be built, the
+// kernel whose copies exist is taken.
+static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w,
+                            int64_t M, hipStream_t st) {
+    if (count < 1 || count > kSKMaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
+    if (gemmsk_max_m(ctx->opt) <= 0 || M < 9 || M < gemm_min_m(ctx->opt)) return false;
+    bool here = true, other = true;
+    for (int i = 0; i < count; i++) {
+        const Layout &L = w[i]->L;
+        if (!is_kquant(L.type) || L.n_in != w[0]->L.n_in || L.n_in % 256) return false;
+        // a buffer's 32-bit offsets: a row block's chunks, an m block's records
+        if (L.n_in / 256 * g2_rec_bytes(16) * 3 > INT32_MAX) return false;
+        here = here && w[i]->gsmall;
+        other = other && plan_copy(w[i], plan_gemm(ctx, L, M));
+    }
+    if (here != other && capturing(st)) return here;
+    if (ctx->opt.gemmsk_max_m >= 0) return M <= ctx->opt.gemmsk_max_m;
+    int64_t blocks = 0;
+    for (int i = 0; i < count; i++) blocks += (w[i]->L.n_out + 31) / 32;
+    return M <= kGemmSKMaxM || (M < kGemm2MinM && blocks * ((M + 15) / 16) <= kGemmSKTiles &&
+                                w[0]->L.n_in <= kGemmSKMaxK);
+}
+
+template <int MT, int NT, int KW>
+static bool launch_gemmsk(uint32_t t0, uint32_t t1, dim3 grid, hipStream_t st, const GSKArgs &A) {
+    if (t0 > t1) std::swap(t0, t1);
+    constexpr size_t lds = sk_lds_bytes(MT, NT, KW);
+#define SIHIP_SK(F0, F1)                                                                         \
+    if (t0 == F0 && t1 == F1) {                                                                  \
+        hipLaunchKernelGGL((gemmsk_kernel<F0, F1, MT, NT, KW>), grid, dim3(64 * KW), lds, st, A); \
+        return true;                                                                             \
+    }
+    SIHIP_SK(T_Q4_K, T_Q4_K)
+    SIHIP_SK(T_Q4_K, T_Q6_K)
+    SIHIP_SK(T_Q6_K, T_Q6_K)
+    SIHIP_SK(T_Q5_K, T_Q5_K)
+    SIHIP_SK(T_Q5_K, T_Q6_K)
+    SIHIP_SK(T_Q3_K, T_Q3_K)
+    SIHIP_SK(T_Q2_K, T_Q2_K)
+#undef SIHIP_SK
+    return false;
+}
+
+// Weights over one X (every gemmks.h copy exists, ws holds plan.ws_bytes):
+// the records once, then one launch where the formats have an instance, else
+// one per format.
+static int launch_gemmsk_group(sihip_ctx *ctx, int count, const sihip_weight *const *w,
+                               const SKPlan &p, const float *X, int64_t M, float *const *Y,
+                               uint8_t *ws, hipStream_t st) {
+    const int64_t n_in = w[0]->L.n_in, nb = n_in / 256;
+    hipLaunchKernelGGL(gemm2_quantize_x<16>, dim3((unsigned)gemm2_quantize_grid(p.Mp * nb)),
+                       dim3(kG2Threads), 0, st, X, n_in, M, p.Mp, nb, ws);
+    auto launch = [&](uint32_t t0, uint32_t t1) {  // the weights of these types
+        GSKArgs A{};
+        A.x = ws;
+        A.M = M;
+        A.nb = (int)nb;
+        A.MB = p.MB;
+        int64_t blocks = 0;
+        for (int i = 0; i < count; i++)
+            if (w[i]->L.type == t0 || w[i]->L.type == t1) blocks += (w[i]->L.n_out + 31) / 32 * p.MB;
+        // few 32-row blocks: half a block per workgroup and eight waves
+        // instead of four (M = 37: ffn_down 4096 x 14336, 128 blocks, 27.8 ->
+        // 24.5 us, 2048 x 5632, 64 blocks, 15.4 -> 12.4, 4096 x 4096 11.4 ->
+        // 10.9; q/k/v, 192 blocks, 13.4 against 16.6); the GEMMS_WAVES option
+        // 4 or 8 sets it
+        const int64_t ow = ctx->opt.gemms_waves;
+        const bool narrow = ow == 4 || ow == 8 ? ow == 8 : 8 * blocks <= 5 * (int64_t)ctx->n_cu;
+        const int rows = narrow ? 16 : 32;
+        int64_t wg = 0;
+        for (int i = 0; i < count; i++) {
+            const Layout &L = w[i]->L;
+            if (L.type != t0 && L.type != t1) continue;
+            GSKSeg &g = A.seg[A.nseg++];
+            g.w = w[i]->gsmall;
+            g.y = Y[i];
+            g.ldy = L.n_out;
+            g.n_out = L.n_out;
+            g.type = L.type;
+            g.nblk = (int)((L.n_out + rows - 1) / rows);
+            g.wg0 = (int)wg;
+            wg += (int64_t)((g.nblk + 7) / 8) * 8 * p.MB;
+        }
+        const dim3 grid((unsigned)wg);
+        switch (p.mt) {
+            case 1: return narrow ? launch_gemmsk<1, 1, 8>(t0, t1, grid, st, A) : launch_gemmsk<1, 2, 4>(t0, t1, grid, st, A);
+            case 2: return narrow ? launch_gemmsk<2, 1, 8>(t0, t1, grid, st, A) : launch_gemmsk<2, 2, 4>(t0, t1, grid, st, A);
+            default: return narrow ? launch_gemmsk<3, 1, 8>(t0, t1, grid, st, A) : launch_gemmsk<3, 2, 4>(t0, t1, grid, st, A);
+        }
+    };
+    uint32_t t0 = w[0]->L.type, t1 = t0;
+    bool two = true;  // at most two formats
+    for (int i = 1; i < count; i++) {
+        const uint32_t t = w[i]->L.type;
+        if (t == t0 || t == t1) continue;
+        two = two && t0 == t1;
+        t1 = t;
+    }
+    if (!two || !launch(t0, t1)) {
+        for (int i = 0; i < count; i++) {
+            bool seen = false;
+            for (int j = 0; j < i; j++) seen = seen || w[j]->L.type == w[i]->L.type;
+            if (!seen && !launch(w[i]->L.type, w[i]->L.type))
+                return set_err(ctx, SIHIP_EINVAL, "gemm: no instance for a format");
+        }
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "gemm launch: %s", hipGetErrorString(e));
+    return SIHIP_OK;
+}
+
+static int run_gemmsk(sihip_ctx *ctx, int count, const sihip_weight *const *wc, const float *X,
+                      int64_t M, float *const *Y, hipStream_t st) {
+    for (int i = 0; i < count; i++) {
+        sihip_weight *w = const_cast<sihip_weight *>(wc[i]);  // the GEMM copies are caches of w
+        if (!w->gsmall) {
+            const int rc = build_gemmks_copy(ctx, w, st);
+            if (rc) return rc;
+        }
+    }
+    const SKPlan p = plan_gemmsk(M, wc[0]->L.n_in / 256);
+    int rc = ensure_planes(ctx, wc[0]->L, M, (size_t)p.ws_bytes, st);
+    if (rc) return rc;
+    rc = order_before(ctx, ctx->order, st);
+    if (rc) return rc;
+    rc = launch_gemmsk_group(ctx, count, wc, p, X, M, Y, (uint8_t *)ctx->d_ws, st);
+    if (rc) return rc;
+    return order_after(ctx, ctx->order, st);
+}
+
+// ---- the K-quant launch of longer prompts (gemmx.h) ---------------------------
+
+// m blocks of 16 mt rows and K slices for NB n blocks of 128 rows: the pair
+// with the least estimated time. A workgroup's super-block costs a decode
+// (about two m tiles' worth) and mt m tiles; one, two, three and four
+// workgroups per CU take 0.72, 1, 1.57 and 1.95 of the time of two (two run
+// at a time: 51, 71, 111 and 138 us at 16 super-blocks and mt = 8); and the
+// slices' partial sums cost about 0.4 us per megabyte, two units of half an m
+// tile (q/k/v of the 8B shapes at M = 512 in 4 blocks of 8 tiles: 50 us
+// unsliced, one per CU, 43 in 2 slices).
+static GemmPlan plan_gemmx(const sihip_ctx *ctx, int64_t M, int64_t nb, int64_t NB) {
+    const int64_t tiles = (M + 15) / 16, slots = 2 * ctx->n_cu;
+    auto rounds = [&](int64_t wgs) {
+        const int64_t k = (wgs + ctx->n_cu - 1) / ctx->n_cu;
+        return k == 1 ? 0.72 : k / 2 + (k % 2 ? 0.57 : 0.0);
+    };
+    GemmPlan p;
+    p.v2 = true;
+    p.steps = nb;
+    double best = -1.0;
+    for (int mt : {2, 3, 4, 5, 6, 8}) {
+        const int64_t MB = (tiles + mt - 1) / mt;
+        for (int64_t S = 1; S <= std::max<int64_t>(nb / 2, 1); S++) {
+            const int64_t wgs = MB * NB * S;
+            if (S > 1 && (wgs > slots || MB * NB > kGemmCounters)) break;
+            const int64_t sbk = (nb + S - 1) / S;
+            if (S > 1 && sbk == (nb + S - 2) / (S - 1)) continue;  // the same slices as S - 1
+            const double part = S > 1 ? 4.0 * S * MB * 16 * mt * NB * kG2BN : 0.0;
+            const double cost = rounds(wgs) * sbk * (4 + 2 * mt) + 2e-6 * part;
+            if (best >= 0.0 && cost >= best) continue;
+            best = cost;
+            p.mt = mt;
+            p.S = (int)((nb + sbk - 1) / sbk);
+            p.SBK = (int)sbk;
+            p.Mp = MB * 16 * mt;
+            p.ws_bytes = MB * nb * g2_rec_bytes(16 * mt);
+            p.part_bytes = p.S > 1 ? (int64_t)p.S * p.Mp * NB * kG2BN * (int64_t)sizeof(float) : 0;
+        }
+    }
+    return p;
+}
+
+static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M,
+                           hipStream_t st) {
+    if (count < 1 || count > kG2MaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
+    if (ctx->opt.gemmx_min_m == 0 || M < 9 || M < gemm_min_m(ctx->opt)) return false;
+    bool here = true, other = true;
+    for (int i = 0; i < count; i++) {
+        const Layout &L = w[i]->L;
+        if (!is_kquant(L.type) || L.n_in != w[0]->L.n_in || L.n_in % 256) return false;
+        // 32-bit buffer offsets: a row block's chunks, an m block's records
+        if (L.n_in / 256 * g2_rec_bytes(128) > INT32_MAX) return false;
+        here = here && w[i]->gsmall;
+        other = other && plan_copy(w[i], plan_gemm(ctx, L, M));
+    }
+    if (here != other && capturing(st)) return here;
+    if (ctx->opt.gemmx_min_m > 0) return M >= ctx->opt.gemmx_min_m;
+    // Q4_K from M = kGemm2MinM runs on gemm2.h, whose copy holds the scales
+    // and mins split beforehand (8B gate + up at M = 2048 502 us against 520
+    // here, wo at M = 512 33.5 against 38.1); other types' single matrices of
+    // few rows on the kernels whose m tiles need fewer K slices and, for
+    // Q6_K, no decode (M = 512, wo: Q6_K 33.3 against 50.8, Q3_K 32.4 against
+    // 41.7, Q2_K 30.1 against 32.9; M = 2048: 90.6 / 81.0 / 72.3 against 93.4
+    // / 71.7 / 68.9). Everything else is faster here (M = 512, 8B gate + up:
+    // Q5_K 264 -> 162 us, Q3_K 142 -> 116, Q6_K 179 -> 159).
+    // (A Q6_K matrix beside Q4_K ones there keeps the launch, and the bits, of
+    // a call of its own.)
+    const uint32_t t = w[0]->L.type;
+    for (int i = 0; i < count; i++)
+        if (w[i]->L.type == T_Q4_K && M >= gemm2_min_m(ctx->opt)) return false;
+    if (count == 1 && w[0]->L.n_out <= 8192 && M >= 128 &&
+        (t == T_Q6_K || ((t == T_Q2_K || t == T_Q3_K) && M < 1024)))
+        return false;
+    return true;
+}
+
+template <int MT>
+static bool launch_gemmx(uint32_t t0, uint32_t t1, dim3 grid, hipStream_t st, const GXArgs &A) {
+    if (t0 > t1) std::swap(t0, t1);
+#define SIHIP_GX(F0, F1)                                                                \
+    if (t0 == F0 && t1 == F1) {                                                         \
+        hipLaunchKernelGGL((gemmx_kernel<F0, F1, MT>), grid, dim3(kG2Threads), 0, st, A); \
+        return true;                                                                    \
+    }
+    SIHIP_GX(T_Q4_K, T_Q4_K)
+    SIHIP_GX(T_Q4_K, T_Q6_K)
+    SIHIP_GX(T_Q6_K, T_Q6_K)
+    SIHIP_GX(T_Q5_K, T_Q5_K)
+    SIHIP_GX(T_Q5_K, T_Q6_K)
+    SIHIP_GX(T_Q3_K, T_Q3_K)
+    SIHIP_GX(T_Q2_K, T_Q2_K)
+#undef SIHIP_GX
+    return false;
+}
+
+template <int BM>
+static void launch_gx_quantize(const float *X, int64_t ldx, int64_t M, int64_t Mp, int64_t nb,
+                               uint8_t *ws, hipStream_t st) {
+    hipLaunchKernelGGL(gemm2_quantize_x<BM>, dim3((unsigned)gemm2_quantize_grid(Mp * nb)),
+                       dim3(kG2Threads), 0, st, X, ldx, M, Mp, nb, ws);
+}
+
+// n blocks of the weights of types t0 and t1.
+static int64_t gemmx_blocks(int count, const sihip_weight *const *w, uint32_t t0, uint32_t t1) {
+    int64_t NB = 0;
+    for (int i = 0; i < count; i++)
+        if (w[i]->L.type == t0 || w[i]->L.type == t1) NB += (w[i]->L.n_out + kG2BN - 1) / kG2BN;
+    return NB;
+}
+
+static int64_t gemmx_all_blocks(int count, const sihip_weight *const *w) {
+    int64_t NB = 0;
+    for (int i = 0; i < count; i++) NB += (w[i]->L.n_out + kG2BN - 1) / kG2BN;
+    return NB;
+}
+
+// Weights over one X (every gemmks.h copy exists): the records once, then one
+// launch where the formats have an instance, else one per format. slices:
+// false runs every launch without K slices.
+static int launch_gemmx_group(sihip_ctx *ctx, int count, const sihip_weight *const *w, const float *X,
+                              int64_t M, float *const *Y, const GemmBufs &B, bool slices,
+                              hipStream_t st) {
+    const int64_t n_in = w[0]->L.n_in, nb = n_in / 256;
+    const GemmPlan q = plan_gemmx(ctx, M, nb, gemmx_all_blocks(count, w));
+    switch (q.mt) {
+        case 2: launch_gx_quantize<32>(X, n_in, M, q.Mp, nb, B.ws, st); break;
+        case 3: launch_gx_quantize<48>(X, n_in, M, q.Mp, nb, B.ws, st); break;
+        case 4: launch_gx_quantize<64>(X, n_in, M, q.Mp, nb, B.ws, st); break;
+        case 5: launch_gx_quantize<80>(X, n_in, M, q.Mp, nb, B.ws, st); break;
+        case 6: launch_gx_quantize<96>(X, n_in, M, q.Mp, nb, B.ws, st); break;
+        default: launch_gx_quantize<128>(X, n_in, M, q.Mp, nb, B.ws, st); break;
+    }
+    auto launch = [&](uint32_t t0, uint32_t t1) {  // the weights of these types
+        // a launch of part of the group keeps the records' m blocks and the
+        // slices of the whole
+        const GemmPlan &p = q;
+        GXArgs A{};
+        A.x = B.ws;
+        A.M = M;
+        A.nb = (int)nb;
+        A.MB = (int)(p.Mp / (16 * p.mt));
+        A.S = slices ? p.S : 1;
+        A.SBK = slices ? p.SBK : (int)nb;
+        A.part = B.part;
+        A.cnt = B.cnt;
+        int64_t NB = 0;
+        for (int i = 0; i < count; i++) {
+            const Layout &L = w[i]->L;
+            if (L.type != t0 && L.type != t1) continue;
+            GXSeg &g = A.seg[A.nseg++];
+            g.w = w[i]->gsmall;
+            g.y = Y[i];
+            g.ldy = L.n_out;
+            g.n_out = L.n_out;
+            g.type = L.type;
+            g.nblk32 = (int)((L.n_out + 31) / 32);
+            g.nb0 = (int)NB;
+            NB += (L.n_out + kG2BN - 1) / kG2BN;
+        }
+        A.NB = (int)NB;
+        const dim3 grid((unsigned)((NB + 7) / 8 * 8 * A.MB * A.S));
+        switch (p.mt) {
+            case 2: return launch_gemmx<2>(t0, t1, grid, st, A);
+            case 3: return launch_gemmx<3>(t0, t1, grid, st, A);
+            case 4: return launch_gemmx<4>(t0, t1, grid, st, A);
+            case 5: return launch_gemmx<5>(t0, t1, grid, st, A);
+            case 6: return launch_gemmx<6>(t0, t1, grid, st, A);
+            default: return launch_gemmx<8>(t0, t1, grid, st, A);
+        }
+    };
+    uint32_t t0 = w[0]->L.type, t1 = t0;
+    bool two = true;  // at most two formats
+    for (int i = 1; i < count; i++) {
+        const uint32_t t = w[i]->L.type;
+        if (t == t0 || t == t1) continue;
+        two = two && t0 == t1;
+        t1 = t;
+    }
+    if (!two || !launch(t0, t1)) {
+        for (int i = 0; i < count; i++) {
+            bool seen = false;
+            for (int j = 0; j < i; j++) seen = seen || w[j]->L.type == w[i]->L.type;
+            if (!seen && !launch(w[i]->L.type, w[i]->L.type))
+                return set_err(ctx, SIHIP_EINVAL, "gemm: no instance for a format");
+        }
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "gemm launch: %s", hipGetErrorString(e));
+    return SIHIP_OK;
+}
+
+static int run_gemmx(sihip_ctx *ctx, int count, const sihip_weight *const *wc, const float *X,
+                     int64_t M, float *const *Y, hipStream_t st) {
+    for (int i = 0; i < count; i++) {
+        sihip_weight *w = const_cast<sihip_weight *>(wc[i]);  // the GEMM copies are caches of w
+        if (!w->gsmall) {
+            const int rc = build_gemmks_copy(ctx, w, st);
+            if (rc) return rc;
+        }
+    }
+    const GemmPlan p = plan_gemmx(ctx, M, wc[0]->L.n_in / 256, gemmx_all_blocks(count, wc));
+    int rc = ensure_planes(ctx, wc[0]->L, M, (size_t)p.ws_bytes, st);
+    if (rc) return rc;
+    // a capture that cannot have the slices' partial sums goes without slices
+    const bool slices = p.S > 1 && (!capturing(st) || ctx->d_gpart_cap >= (size_t)p.part_bytes);
+    if (slices) {
+        rc = ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, (size_t)p.part_bytes, st);
+        if (rc) return rc;
+    }
+    rc = order_before(ctx, ctx->order, st);
+    if (rc) return rc;
+    const GemmBufs B{(uint8_t *)ctx->d_ws, (float *)ctx->d_gpart, ctx->d_gcnt};
+    rc = launch_gemmx_group(ctx, count, wc, X, M, Y, B, slices, st);
+    if (rc) return rc;
+    return order_after(ctx, ctx->order, st);
+}
+
 // The MFMA GEMM on the context's workspaces (grown as needed, outside
 // graph capture) and the weight's GEMM copy (built on first use). The
 // activation planes live in the context, so calls on one context must not
@@ -1989,11 +2388,15 @@ static int run_gemm_mfma(sihip_ctx *ctx, const sihip_weight *wc, const float *X,
                          int64_t M, float *Y, int64_t ldy, hipStream_t st) {
     if (ldx == wc->L.n_in && ldy == wc->L.n_out && gemmkf_eligible(ctx, 1, &wc, M))
         return run_gemmkf(ctx, 1, &wc, X, M, &Y, st);
+    if (ldx == wc->L.n_in && ldy == wc->L.n_out && gemmsk_eligible(ctx, 1, &wc, M, st))
+        return run_gemmsk(ctx, 1, &wc, X, M, &Y, st);
+    if (ldx == wc->L.n_in && ldy == wc->L.n_out && gemmx_eligible(ctx, 1, &wc, M, st))
+        return run_gemmx(ctx, 1, &wc, X, M, &Y, st);
     sihip_weight *w = const_cast<sihip_weight *>(wc);  // the GEMM copies are caches of w
     const GemmPlan p = plan_gemm(ctx, w->L, M);
     int rc = build_plan_copy(ctx, w, p, st);
     if (rc) return rc;
-    rc = ensure(ctx, &ctx->d_ws, &ctx->d_ws_cap, (size_t)p.ws_bytes, st);
+    rc = ensure_planes(ctx, w->L, M, (size_t)p.ws_bytes, st);
     if (rc) return rc;
     if (p.S > 1) {
         rc = ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, (size_t)p.part_bytes, st);
@@ -2034,6 +2437,8 @@ static int run_gemm_multi(sihip_ctx *ctx, int count, const sihip_weight *const *
                           const float *X, int64_t M, float *const *Y, hipStream_t st) {
     if (count <= kKFMaxSegs && gemmkf_eligible(ctx, count, wc, M))
         return run_gemmkf(ctx, count, wc, X, M, Y, st);
+    if (gemmsk_eligible(ctx, count, wc, M, st)) return run_gemmsk(ctx, count, wc, X, M, Y, st);
+    if (gemmx_eligible(ctx, count, wc, M, st)) return run_gemmx(ctx, count, wc, X, M, Y, st);
     // the Q4_K weights on the 16x16 kernel (M >= gemm2_min_m) share one
     // launch, planned as one matrix of their n blocks together (the
     // GEMM_GROUP option at 0 turns this off)
@@ -2113,7 +2518,7 @@ static int run_gemm_multi(sihip_ctx *ctx, int count, const sihip_weight *const *
         const int rc = build_plan_copy(ctx, w, plan[i], st);
         if (rc) return rc;
     }
-    int rc = ensure(ctx, &ctx->d_ws, &ctx->d_ws_cap, total, st);
+    int rc = ensure_planes(ctx, wc[0]->L, M, total, st);
     if (rc) return rc;
     if (part) {
         rc = ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, part, st);
@@ -2331,6 +2736,22 @@ extern "C" int sihip_gemm_dev_noalloc(sihip_ctx *ctx, const sihip_weight *w, con
                                            (uint32_t *)(ctx->scratch + room), st, done);
         if (rc) return rc;
         return done ? SIHIP_OK : set_err(ctx, SIHIP_EINVAL, "gemm_dev_noalloc: no fused instance");
+    }
+    if (w->gsmall && gemmsk_eligible(ctx, 1, &w, M, st)) {
+        const SKPlan sp = plan_gemmsk(M, w->L.n_in / 256);
+        float *Yp = Y;
+        if ((size_t)sp.ws_bytes <= room)  // else the kernels below, whose planes are smaller
+            return launch_gemmsk_group(ctx, 1, &w, sp, X, M, &Yp, ctx->scratch, st);
+    }
+    if (w->gsmall && gemmx_eligible(ctx, 1, &w, M, st)) {
+        const GemmPlan gp = plan_gemmx(ctx, M, w->L.n_in / 256, gemmx_blocks(1, &w, w->L.type, w->L.type));
+        const size_t off = ((size_t)gp.ws_bytes + 255) & ~(size_t)255;
+        float *Yp = Y;
+        if ((size_t)gp.ws_bytes <= room) {
+            const bool slices = gp.S > 1 && off + (size_t)gp.part_bytes <= room;
+            const GemmBufs GB{ctx->scratch, (float *)(ctx->scratch + off), (uint32_t *)(ctx->scratch + room)};
+            return launch_gemmx_group(ctx, 1, &w, X, M, &Yp, GB, slices, st);
+        }
     }
     GemmPlan p = plan_gemm(ctx, w->L, M);
     if (!plan_copy(w, p))
