@@ -27,6 +27,7 @@
 #include "gemmkf.h"
 #include "gemmsk.h"
 #include "gemmx.h"
+#include "gemmd.h"
 #include "gemm6.h"
 #include "gemmh.h"
 #include "gemmq.h"
@@ -62,6 +63,7 @@ struct Options {
     int64_t gemmkf_max_m = -1; // largest M on the fused small-M K-quant launch, 0: none (rule: 8)
     int64_t gemmkf_sbk = -1;   // its K-slice length in super-blocks, 0: fewest slices (rule: by tiles)
     int64_t gemmsk_max_m = -1; // largest M on the short-prompt K-quant GEMM, 0: none (rule: kGemmSKMaxM)
+    int64_t gemmd_min_m = -1;  // smallest M on the F16 and Q8_0-pair GEMM of prompts, 0: never (rule: kGemmDMinM)
     int64_t gemmx_min_m = -1;  // smallest M on the K-quant GEMM of longer prompts, 0: never (rule: past GEMMSK_MAX_M)
     int64_t gemm_group = -1;   // Q4_K matrices over one X in one 16x16 GEMM launch, 0: off (rule: on)
     int64_t q80_scalar = -1;   // Q8_0 activations by the scalar quantizer (reference
@@ -88,7 +90,7 @@ static const OptionName kOptionNames[] = {
     {"GEMMS_WAVES", &Options::gemms_waves},
     {"GEMMKF_MAX_M", &Options::gemmkf_max_m}, {"GEMMKF_SBK", &Options::gemmkf_sbk},
     {"GEMM_GROUP", &Options::gemm_group}, {"GEMMSK_MAX_M", &Options::gemmsk_max_m},
-    {"GEMMX_MIN_M", &Options::gemmx_min_m},
+    {"GEMMX_MIN_M", &Options::gemmx_min_m}, {"GEMMD_MIN_M", &Options::gemmd_min_m},
 };
 
 // Order of launches that share mutable device state across streams: a
@@ -1999,18 +2001,35 @@ static int run_gemmkf(sihip_ctx *ctx, int count, const sihip_weight *const *wc, 
     return order_after(ctx, ctx->order, st);
 }
 
-// The activation planes of a K-quant product of M rows: `need` bytes, and
-// outside capture as much as any of its kernels asks for at any smaller M (at
-// most 320 bytes per row and super-block, and a third or seven more 16-row
-// tiles than M has), so that a capture of such a call finds them whichever
-// kernel each of the two takes.
-static int ensure_planes(sihip_ctx *ctx, const Layout &L, int64_t M, size_t need, hipStream_t st) {
-    if (is_kquant(L.type) && M >= 9 && L.n_in % 256 == 0 && !capturing(st)) {
+// The workspaces of a product of M rows of weights over one X: `ws` bytes of
+// activation planes, `part` of partial sums. Outside capture the planes are
+// kept as large as any kernel asks for at any smaller M (K-quants: at most 320
+// bytes per row and super-block, and a third or seven more 16-row tiles than M
+// has; the others: 256 or 160 per row and step, seven more tiles) and both as
+// large as the single plans (plan_gemm), so that a capture of such a call
+// finds them whichever kernel each of the two takes.
+static int ensure_bufs(sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M, size_t ws,
+                       size_t part, hipStream_t st) {
+    if (M >= 9 && !capturing(st)) {
         const int64_t tiles = (M + 15) / 16;
-        need = std::max(need, (size_t)((tiles + std::max<int64_t>(7, tiles / 3 + 1)) *
-                                       (L.n_in / 256) * g2_rec_bytes(16)));
+        size_t sum = 0;
+        for (int i = 0; i < count; i++) {
+            const Layout &L = w[i]->L;
+            const GemmPlan p = plan_gemm(ctx, L, M);
+            bool first = true;
+            for (int j = 0; j < i; j++) first = first && w[j]->L.type != L.type;
+            if (first) sum += ((size_t)p.ws_bytes + 255) & ~(size_t)255;
+            if (p.S > 1) part = std::max(part, (size_t)p.part_bytes);
+            const int64_t bound =
+                is_kquant(L.type) ? (tiles + std::max<int64_t>(7, tiles / 3 + 1)) * (L.n_in / 256) * g2_rec_bytes(16)
+                                  : (tiles + 7) * (L.n_in / 128) * (L.type == T_F16 ? gh_rec_bytes(16) : gq_rec_bytes(16));
+            ws = std::max(ws, (size_t)bound);
+        }
+        ws = std::max(ws, sum);
     }
-    return ensure(ctx, &ctx->d_ws, &ctx->d_ws_cap, need, st);
+    int rc = ensure(ctx, &ctx->d_ws, &ctx->d_ws_cap, ws, st);
+    if (rc || !part) return rc;
+    return ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, part, st);
 }
 
 // ---- the short-prompt K-quant launch (gemmsk.h) -------------------------------
@@ -2154,7 +2173,7 @@ static int run_gemmsk(sihip_ctx *ctx, int count, const sihip_weight *const *wc, 
         }
     }
     const SKPlan p = plan_gemmsk(M, wc[0]->L.n_in / 256);
-    int rc = ensure_planes(ctx, wc[0]->L, M, (size_t)p.ws_bytes, st);
+    int rc = ensure_bufs(ctx, count, wc, M, (size_t)p.ws_bytes, 0, st);
     if (rc) return rc;
     rc = order_before(ctx, ctx->order, st);
     if (rc) return rc;
@@ -2166,42 +2185,58 @@ static int run_gemmsk(sihip_ctx *ctx, int count, const sihip_weight *const *wc, 
 // ---- the K-quant launch of longer prompts (gemmx.h) ---------------------------
 
 // m blocks of 16 mt rows and K slices for NB n blocks of 128 rows: the pair
-// with the least estimated time. A workgroup's super-block costs a decode
-// (about two m tiles' worth) and mt m tiles; one, two, three and four
-// workgroups per CU take 0.72, 1, 1.57 and 1.95 of the time of two (two run
-// at a time: 51, 71, 111 and 138 us at 16 super-blocks and mt = 8); and the
+// with the least estimated time. A workgroup's step costs `fixed` and
+// `per_tile` for each m tile; `share` is what k workgroups on one CU take over
+// what two take (n blocks go round-robin over the 8 XCDs, so the XCD with the
+// most sets k); a sliced launch pays `slice` and `byte` for each byte of
+// partial sums.
+struct TileCost {
+    double fixed, per_tile, slice, byte;
+    double (*share)(int64_t k);
+    int max_mt;
+};
+
+// One, two, three and four workgroups per CU take 0.72, 1, 1.57 and 1.95 of
+// the time of two (two run at a time: the 8B gate + up in gemmx.h at 16
+// super-blocks and mt = 8: 51, 71, 111 and 138 us).
+static double share_paired(int64_t k) { return k == 1 ? 0.72 : (double)(k / 2) + (k % 2 ? 0.57 : 0.0); }
+
+static GemmPlan plan_tiles(const sihip_ctx *ctx, int64_t M, int64_t steps, int64_t NB, const TileCost &C) {
+    const int64_t tiles = (M + 15) / 16, slots = 2 * ctx->n_cu;
+    GemmPlan p;
+    p.v2 = true;
+    p.steps = steps;
+    double best = -1.0;
+    for (int mt : {2, 3, 4, 5, 6, 8}) {
+        if (mt > C.max_mt) break;
+        const int64_t MB = (tiles + mt - 1) / mt;
+        for (int64_t S = 1; S <= std::max<int64_t>(steps / 2, 1); S++) {
+            const int64_t wgs = MB * ((NB + 7) / 8 * 8) * S;
+            if (S > 1 && (wgs > slots || MB * NB > kGemmCounters)) break;
+            const int64_t sbk = (steps + S - 1) / S;
+            if (S > 1 && sbk == (steps + S - 2) / (S - 1)) continue;  // the same slices as S - 1
+            const double part = S > 1 ? 4.0 * S * MB * 16 * mt * NB * kG2BN : 0.0;
+            const double cost = C.share((wgs + ctx->n_cu - 1) / ctx->n_cu) * sbk * (C.fixed + C.per_tile * mt) +
+                                (S > 1 ? C.slice : 0.0) + C.byte * part;
+            if (best >= 0.0 && cost >= best) continue;
+            best = cost;
+            p.mt = mt;
+            p.S = (int)((steps + sbk - 1) / sbk);
+            p.SBK = (int)sbk;
+            p.Mp = MB * 16 * mt;
+            p.part_bytes = p.S > 1 ? (int64_t)p.S * p.Mp * NB * kG2BN * (int64_t)sizeof(float) : 0;
+        }
+    }
+    return p;
+}
+
+// A super-block costs a decode (about two m tiles' worth) and mt m tiles; the
 // slices' partial sums cost about 0.4 us per megabyte, two units of half an m
 // tile (q/k/v of the 8B shapes at M = 512 in 4 blocks of 8 tiles: 50 us
 // unsliced, one per CU, 43 in 2 slices).
 static GemmPlan plan_gemmx(const sihip_ctx *ctx, int64_t M, int64_t nb, int64_t NB) {
-    const int64_t tiles = (M + 15) / 16, slots = 2 * ctx->n_cu;
-    auto rounds = [&](int64_t wgs) {
-        const int64_t k = (wgs + ctx->n_cu - 1) / ctx->n_cu;
-        return k == 1 ? 0.72 : k / 2 + (k % 2 ? 0.57 : 0.0);
-    };
-    GemmPlan p;
-    p.v2 = true;
-    p.steps = nb;
-    double best = -1.0;
-    for (int mt : {2, 3, 4, 5, 6, 8}) {
-        const int64_t MB = (tiles + mt - 1) / mt;
-        for (int64_t S = 1; S <= std::max<int64_t>(nb / 2, 1); S++) {
-            const int64_t wgs = MB * NB * S;
-            if (S > 1 && (wgs > slots || MB * NB > kGemmCounters)) break;
-            const int64_t sbk = (nb + S - 1) / S;
-            if (S > 1 && sbk == (nb + S - 2) / (S - 1)) continue;  // the same slices as S - 1
-            const double part = S > 1 ? 4.0 * S * MB * 16 * mt * NB * kG2BN : 0.0;
-            const double cost = rounds(wgs) * sbk * (4 + 2 * mt) + 2e-6 * part;
-            if (best >= 0.0 && cost >= best) continue;
-            best = cost;
-            p.mt = mt;
-            p.S = (int)((nb + sbk - 1) / sbk);
-            p.SBK = (int)sbk;
-            p.Mp = MB * 16 * mt;
-            p.ws_bytes = MB * nb * g2_rec_bytes(16 * mt);
-            p.part_bytes = p.S > 1 ? (int64_t)p.S * p.Mp * NB * kG2BN * (int64_t)sizeof(float) : 0;
-        }
-    }
+    GemmPlan p = plan_tiles(ctx, M, nb, NB, TileCost{4, 2, 0, 2e-6, share_paired, 8});
+    p.ws_bytes = p.Mp / (16 * p.mt) * nb * g2_rec_bytes(16 * p.mt);
     return p;
 }
 
@@ -2265,15 +2300,8 @@ static void launch_gx_quantize(const float *X, int64_t ldx, int64_t M, int64_t M
                        dim3(kG2Threads), 0, st, X, ldx, M, Mp, nb, ws);
 }
 
-// n blocks of the weights of types t0 and t1.
-static int64_t gemmx_blocks(int count, const sihip_weight *const *w, uint32_t t0, uint32_t t1) {
-    int64_t NB = 0;
-    for (int i = 0; i < count; i++)
-        if (w[i]->L.type == t0 || w[i]->L.type == t1) NB += (w[i]->L.n_out + kG2BN - 1) / kG2BN;
-    return NB;
-}
-
-static int64_t gemmx_all_blocks(int count, const sihip_weight *const *w) {
+// n blocks of the weights.
+static int64_t gemm_blocks(int count, const sihip_weight *const *w) {
     int64_t NB = 0;
     for (int i = 0; i < count; i++) NB += (w[i]->L.n_out + kG2BN - 1) / kG2BN;
     return NB;
@@ -2286,7 +2314,7 @@ static int launch_gemmx_group(sihip_ctx *ctx, int count, const sihip_weight *con
                               int64_t M, float *const *Y, const GemmBufs &B, bool slices,
                               hipStream_t st) {
     const int64_t n_in = w[0]->L.n_in, nb = n_in / 256;
-    const GemmPlan q = plan_gemmx(ctx, M, nb, gemmx_all_blocks(count, w));
+    const GemmPlan q = plan_gemmx(ctx, M, nb, gemm_blocks(count, w));
     switch (q.mt) {
         case 2: launch_gx_quantize<32>(X, n_in, M, q.Mp, nb, B.ws, st); break;
         case 3: launch_gx_quantize<48>(X, n_in, M, q.Mp, nb, B.ws, st); break;
@@ -2363,15 +2391,11 @@ static int run_gemmx(sihip_ctx *ctx, int count, const sihip_weight *const *wc, c
             if (rc) return rc;
         }
     }
-    const GemmPlan p = plan_gemmx(ctx, M, wc[0]->L.n_in / 256, gemmx_all_blocks(count, wc));
-    int rc = ensure_planes(ctx, wc[0]->L, M, (size_t)p.ws_bytes, st);
-    if (rc) return rc;
+    const GemmPlan p = plan_gemmx(ctx, M, wc[0]->L.n_in / 256, gemm_blocks(count, wc));
     // a capture that cannot have the slices' partial sums goes without slices
     const bool slices = p.S > 1 && (!capturing(st) || ctx->d_gpart_cap >= (size_t)p.part_bytes);
-    if (slices) {
-        rc = ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, (size_t)p.part_bytes, st);
-        if (rc) return rc;
-    }
+    int rc = ensure_bufs(ctx, count, wc, M, (size_t)p.ws_bytes, slices ? (size_t)p.part_bytes : 0, st);
+    if (rc) return rc;
     rc = order_before(ctx, ctx->order, st);
     if (rc) return rc;
     const GemmBufs B{(uint8_t *)ctx->d_ws, (float *)ctx->d_gpart, ctx->d_gcnt};
@@ -2384,6 +2408,211 @@ static int run_gemmx(sihip_ctx *ctx, int count, const sihip_weight *const *wc, c
 // graph capture) and the weight's GEMM copy (built on first use). The
 // activation planes live in the context, so calls on one context must not
 // overlap.
+static bool gemm_on_mfma(const sihip_ctx *ctx, const sihip_weight *w, int64_t M);
+
+// ---- the F16 and Q8_0-pair launch of prompts (gemmd.h) ------------------------
+
+// Smallest M on this launch, of a group and of a single matrix; option
+// GEMMD_MIN_M for both. Up to 16 rows the kernels that quantize or convert X
+// themselves need no launch before them. A single matrix of up to 128 rows is
+// as fast there (M = 20, Q8_0 2048 x 5632 14.3 us against 15.8 here, M = 64
+// Q5_0 16.7 against 19.2, M = 100 Q8_0 21.1 against 21.2; M = 200 30.3 against
+// 24.7, F16 M = 500 40.1 against 28 to 31).
+constexpr int64_t kGemmDMinM = 17, kGemmDMinM1 = 129;
+
+// Small products (plan.small) in the workgroups of gemmds_kernel where each
+// gets a CU of its own (1.1B q/k/v in 240 workgroups: Q8_0 M = 100 16.0 us
+// against 17.1 in tiles, F16 M = 40 in 80 9.8 against 11.7; wo of the 0.5B
+// shapes at M = 300 in 224 12.4 against 13.8; q/k/v in 400 equal, gate + up of
+// F16 at M = 200 in 1760 36.7 against 24.9) and the Q8_0 pairs' rows are not
+// long (0.5B ffn_down, 38 steps of three m tiles: 26.7 against 22.4), the rest
+// in tiles. Costs: F16 0.13
+// us per step and 0.12 per m tile whether a CU has one workgroup or more (LDS
+// reads), the Q8_0 pairs 0.25 and 0.26 (the epilogue's VALU work), two in 1.4
+// of the time of one; slices about 1 us and 0.5 per megabyte.
+static GemmPlan plan_gemmd(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M) {
+    const Layout &L = w[0]->L;
+    const bool f16 = L.type == T_F16;
+    const int64_t nk = L.n_in / 128;
+    const SKPlan q = plan_gemmsk(M, 1);
+    int64_t wgs = 0;
+    for (int i = 0; i < count; i++) wgs += (w[i]->L.n_out + 255) / 256 * 8 * q.MB;
+    GemmPlan p;
+    if (wgs <= ctx->n_cu && (f16 || nk * q.mt <= 64)) {
+        p.v2 = p.small = true;
+        p.mt = q.mt;
+        p.Mp = q.Mp;
+        p.S = 1;
+        p.SBK = (int)nk;
+        p.steps = nk;
+        p.part_bytes = 0;
+    } else {
+        p = plan_tiles(ctx, M, nk, gemm_blocks(count, w),
+                       f16 ? TileCost{2.2, 2, 16, 8e-6, [](int64_t k) { return (double)k; }, 6}
+                           : TileCost{2, 2, 5.5, 2.8e-6, share_paired, 5});
+    }
+    p.ws_bytes = p.Mp / 16 * nk * (f16 ? gh_rec_bytes(16) : gq_rec_bytes(16));
+    return p;
+}
+
+// Whether weights over one X take this launch: one format of these, unless an
+// option sets the tiling of the other kernels.
+static bool gemmd_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M) {
+    if (count < 1 || count > kG2MaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
+    if (ctx->opt.gemmd_min_m == 0 || ctx->opt.gemmq_xmode >= 0) return false;
+    const int64_t min_m = ctx->opt.gemmd_min_m > 0 ? ctx->opt.gemmd_min_m : count > 1 ? kGemmDMinM : kGemmDMinM1;
+    if (M < 2 || M < min_m) return false;
+    for (int i = 0; i < count; i++) {
+        const Layout &L = w[i]->L;
+        if (L.type != w[0]->L.type || L.n_in != w[0]->L.n_in || !gemm_on_mfma(ctx, w[i], M)) return false;
+        if (L.type != T_F16 && !is_q80_pair(L.type)) return false;
+        // 32-bit buffer offsets: a 128-row block's chunks, an m block's records
+        if (L.n_in / 128 * 4 * kGHChunk > INT32_MAX) return false;
+    }
+    if (ctx->opt.gemmd_min_m > 0) return true;
+    const Layout &L = w[0]->L;
+    // F16 matrices with work for the chip each run as fast in the 128-row
+    // tiles of gemmh.h (32B at M = 700, 51840 tile steps a matrix: gate + up
+    // 522 us there against 554, ffn_down 269 against 307; 1.1B gate + up at
+    // M = 1500, 8448 each: 119 against 94 here, 8B at M = 300, 10752: 143
+    // against 110)
+    if (L.type == T_F16)
+        return gemm_blocks(count, w) * ((M + 127) / 128) * (L.n_in / 128) < (int64_t)32768 * count;
+    // a single Q8_0-pair matrix of few rows from 512: no faster here (2048 x
+    // 2048 at M = 600: Q4_0 29.4 us there, 33.0 here; M = 500: 27.9 and 21.1)
+    return count > 1 || M <= 512 || L.n_out >= 4096;
+}
+
+template <uint32_t FMT, int BM>
+static void launch_gemmd_x(const float *X, int64_t n_in, int64_t M, int64_t Mp, int q80s, uint8_t *ws,
+                           hipStream_t st) {
+    const int64_t threads = Mp * n_in / (FMT == T_F16 ? 8 : 32);
+    const dim3 qg((unsigned)((threads + 255) / 256));
+    if constexpr (FMT == T_F16)
+        hipLaunchKernelGGL(gemmh_convert_x<BM>, qg, dim3(256), 0, st, X, n_in, M, Mp, n_in, ws);
+    else
+        hipLaunchKernelGGL((gemmq_quantize_x<BM, FMT == T_Q4_0 ? 8 : FMT == T_Q5_0 ? 16 : 0>), qg,
+                           dim3(256), 0, st, X, n_in, M, Mp, n_in, ws, q80s);
+}
+
+template <uint32_t FMT, int MT>
+static void launch_gemmd(const float *X, int64_t n_in, int64_t M, int64_t Mp, int q80s, uint8_t *ws,
+                         dim3 grid, hipStream_t st, const GDArgs &A) {
+    launch_gemmd_x<FMT, 16 * MT>(X, n_in, M, Mp, q80s, ws, st);
+    hipLaunchKernelGGL((gemmd_kernel<FMT, MT>), grid, dim3(kG2Threads), 0, st, A);
+}
+
+// A small product (plan.small): the records, then one launch.
+static int launch_gemmds_group(sihip_ctx *ctx, int count, const sihip_weight *const *w, const GemmPlan &p,
+                               const float *X, int64_t M, float *const *Y, uint8_t *ws, hipStream_t st) {
+    const int64_t n_in = w[0]->L.n_in;
+    GDSArgs A{};
+    A.x = ws;
+    A.M = M;
+    A.nk = (int)(n_in / 128);
+    A.MB = (int)(p.Mp / (16 * p.mt));
+    int64_t wg = 0;
+    for (int i = 0; i < count; i++) {
+        GDSSeg &g = A.seg[A.nseg++];
+        g.w = w[i]->gemm2;
+        g.y = Y[i];
+        g.ldy = g.n_out = w[i]->L.n_out;
+        g.nblk = (int)((g.n_out + 31) / 32);
+        g.wg0 = (int)wg;
+        wg += (int64_t)((g.nblk + 7) / 8) * 8 * A.MB;
+    }
+    const dim3 grid((unsigned)wg);
+    const int q80s = ctx->opt.q80_scalar > 0;
+#define SIHIP_GDS(F)                                                  \
+    case F:                                                           \
+        launch_gemmd_x<F, 16>(X, n_in, M, p.Mp, q80s, ws, st);        \
+        if (p.mt == 1) hipLaunchKernelGGL((gemmds_kernel<F, 1>), grid, dim3(kG2Threads), 0, st, A); \
+        else if (p.mt == 2) hipLaunchKernelGGL((gemmds_kernel<F, 2>), grid, dim3(kG2Threads), 0, st, A); \
+        else hipLaunchKernelGGL((gemmds_kernel<F, 3>), grid, dim3(kG2Threads), 0, st, A); \
+        break;
+    switch (w[0]->L.type) {
+        SIHIP_GDS(T_F16)
+        SIHIP_GDS(T_Q4_0)
+        SIHIP_GDS(T_Q5_0)
+        SIHIP_GDS(T_Q8_0)
+    }
+#undef SIHIP_GDS
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "gemm launch: %s", hipGetErrorString(e));
+    return SIHIP_OK;
+}
+
+// Weights over one X (every gemm2 copy exists): the records, then one launch.
+// slices: false runs it without K slices.
+static int launch_gemmd_group(sihip_ctx *ctx, int count, const sihip_weight *const *w, const GemmPlan &p,
+                              const float *X, int64_t M, float *const *Y, const GemmBufs &B,
+                              bool slices, hipStream_t st) {
+    if (p.small) return launch_gemmds_group(ctx, count, w, p, X, M, Y, B.ws, st);
+    const int64_t n_in = w[0]->L.n_in, nk = n_in / 128;
+    GDArgs A{};
+    A.x = B.ws;
+    A.M = M;
+    A.nk = (int)nk;
+    A.MB = (int)(p.Mp / (16 * p.mt));
+    A.S = slices ? p.S : 1;
+    A.SBK = slices ? p.SBK : (int)nk;
+    A.part = B.part;
+    A.cnt = B.cnt;
+    int64_t NB = 0;
+    for (int i = 0; i < count; i++) {
+        GDSeg &g = A.seg[A.nseg++];
+        g.w = w[i]->gemm2;
+        g.y = Y[i];
+        g.ldy = g.n_out = w[i]->L.n_out;
+        g.nb0 = (int)NB;
+        NB += (w[i]->L.n_out + kG2BN - 1) / kG2BN;
+    }
+    A.NB = (int)NB;
+    const dim3 grid((unsigned)((NB + 7) / 8 * 8 * A.MB * A.S));
+    const int q80s = ctx->opt.q80_scalar > 0;
+#define SIHIP_GD(F, MT)                                                           \
+    case MT: launch_gemmd<F, MT>(X, n_in, M, p.Mp, q80s, B.ws, grid, st, A); break;
+#define SIHIP_GDF(F, MORE)                                                        \
+    case F:                                                                       \
+        switch (p.mt) {                                                           \
+            SIHIP_GD(F, 2) SIHIP_GD(F, 3) SIHIP_GD(F, 4) SIHIP_GD(F, 5) MORE      \
+        }                                                                         \
+        break;
+    switch (w[0]->L.type) {
+        SIHIP_GDF(T_F16, SIHIP_GD(T_F16, 6))
+        SIHIP_GDF(T_Q4_0, )
+        SIHIP_GDF(T_Q5_0, )
+        SIHIP_GDF(T_Q8_0, )
+    }
+#undef SIHIP_GDF
+#undef SIHIP_GD
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "gemm launch: %s", hipGetErrorString(e));
+    return SIHIP_OK;
+}
+
+static int run_gemmd(sihip_ctx *ctx, int count, const sihip_weight *const *wc, const float *X,
+                     int64_t M, float *const *Y, hipStream_t st) {
+    for (int i = 0; i < count; i++) {
+        sihip_weight *w = const_cast<sihip_weight *>(wc[i]);  // the GEMM copies are caches of w
+        if (!w->gemm2) {
+            const int rc = build_gemm2_copy(ctx, w, st);
+            if (rc) return rc;
+        }
+    }
+    const GemmPlan p = plan_gemmd(ctx, count, wc, M);
+    // a capture that cannot have the slices' partial sums goes without slices
+    const bool slices = p.S > 1 && (!capturing(st) || ctx->d_gpart_cap >= (size_t)p.part_bytes);
+    int rc = ensure_bufs(ctx, count, wc, M, (size_t)p.ws_bytes, slices ? (size_t)p.part_bytes : 0, st);
+    if (rc) return rc;
+    rc = order_before(ctx, ctx->order, st);
+    if (rc) return rc;
+    const GemmBufs B{(uint8_t *)ctx->d_ws, (float *)ctx->d_gpart, ctx->d_gcnt};
+    rc = launch_gemmd_group(ctx, count, wc, p, X, M, Y, B, slices, st);
+    if (rc) return rc;
+    return order_after(ctx, ctx->order, st);
+}
+
 static int run_gemm_mfma(sihip_ctx *ctx, const sihip_weight *wc, const float *X, int64_t ldx,
                          int64_t M, float *Y, int64_t ldy, hipStream_t st) {
     if (ldx == wc->L.n_in && ldy == wc->L.n_out && gemmkf_eligible(ctx, 1, &wc, M))
@@ -2392,16 +2621,14 @@ static int run_gemm_mfma(sihip_ctx *ctx, const sihip_weight *wc, const float *X,
         return run_gemmsk(ctx, 1, &wc, X, M, &Y, st);
     if (ldx == wc->L.n_in && ldy == wc->L.n_out && gemmx_eligible(ctx, 1, &wc, M, st))
         return run_gemmx(ctx, 1, &wc, X, M, &Y, st);
+    if (ldx == wc->L.n_in && ldy == wc->L.n_out && gemmd_eligible(ctx, 1, &wc, M))
+        return run_gemmd(ctx, 1, &wc, X, M, &Y, st);
     sihip_weight *w = const_cast<sihip_weight *>(wc);  // the GEMM copies are caches of w
     const GemmPlan p = plan_gemm(ctx, w->L, M);
     int rc = build_plan_copy(ctx, w, p, st);
     if (rc) return rc;
-    rc = ensure_planes(ctx, w->L, M, (size_t)p.ws_bytes, st);
+    rc = ensure_bufs(ctx, 1, &wc, M, (size_t)p.ws_bytes, p.S > 1 ? (size_t)p.part_bytes : 0, st);
     if (rc) return rc;
-    if (p.S > 1) {
-        rc = ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, (size_t)p.part_bytes, st);
-        if (rc) return rc;
-    }
     rc = order_before(ctx, ctx->order, st);
     if (rc) return rc;
     const GemmBufs B{(uint8_t *)ctx->d_ws, (float *)ctx->d_gpart, ctx->d_gcnt};
@@ -2439,6 +2666,7 @@ static int run_gemm_multi(sihip_ctx *ctx, int count, const sihip_weight *const *
         return run_gemmkf(ctx, count, wc, X, M, Y, st);
     if (gemmsk_eligible(ctx, count, wc, M, st)) return run_gemmsk(ctx, count, wc, X, M, Y, st);
     if (gemmx_eligible(ctx, count, wc, M, st)) return run_gemmx(ctx, count, wc, X, M, Y, st);
+    if (gemmd_eligible(ctx, count, wc, M)) return run_gemmd(ctx, count, wc, X, M, Y, st);
     // the Q4_K weights on the 16x16 kernel (M >= gemm2_min_m) share one
     // launch, planned as one matrix of their n blocks together (the
     // GEMM_GROUP option at 0 turns this off)
@@ -2518,12 +2746,8 @@ static int run_gemm_multi(sihip_ctx *ctx, int count, const sihip_weight *const *
         const int rc = build_plan_copy(ctx, w, plan[i], st);
         if (rc) return rc;
     }
-    int rc = ensure_planes(ctx, wc[0]->L, M, total, st);
+    int rc = ensure_bufs(ctx, count, wc, M, total, part, st);
     if (rc) return rc;
-    if (part) {
-        rc = ensure(ctx, &ctx->d_gpart, &ctx->d_gpart_cap, part, st);
-        if (rc) return rc;
-    }
     rc = order_before(ctx, ctx->order, st);
     if (rc) return rc;
     bool grp_done = false;
@@ -2744,13 +2968,23 @@ extern "C" int sihip_gemm_dev_noalloc(sihip_ctx *ctx, const sihip_weight *w, con
             return launch_gemmsk_group(ctx, 1, &w, sp, X, M, &Yp, ctx->scratch, st);
     }
     if (w->gsmall && gemmx_eligible(ctx, 1, &w, M, st)) {
-        const GemmPlan gp = plan_gemmx(ctx, M, w->L.n_in / 256, gemmx_blocks(1, &w, w->L.type, w->L.type));
+        const GemmPlan gp = plan_gemmx(ctx, M, w->L.n_in / 256, gemm_blocks(1, &w));
         const size_t off = ((size_t)gp.ws_bytes + 255) & ~(size_t)255;
         float *Yp = Y;
         if ((size_t)gp.ws_bytes <= room) {
             const bool slices = gp.S > 1 && off + (size_t)gp.part_bytes <= room;
             const GemmBufs GB{ctx->scratch, (float *)(ctx->scratch + off), (uint32_t *)(ctx->scratch + room)};
             return launch_gemmx_group(ctx, 1, &w, X, M, &Yp, GB, slices, st);
+        }
+    }
+    if (w->gemm2 && gemmd_eligible(ctx, 1, &w, M)) {
+        const GemmPlan gp = plan_gemmd(ctx, 1, &w, M);
+        const size_t off = ((size_t)gp.ws_bytes + 255) & ~(size_t)255;
+        float *Yp = Y;
+        if ((size_t)gp.ws_bytes <= room) {
+            const bool slices = gp.S > 1 && off + (size_t)gp.part_bytes <= room;
+            const GemmBufs GB{ctx->scratch, (float *)(ctx->scratch + off), (uint32_t *)(ctx->scratch + room)};
+            return launch_gemmd_group(ctx, 1, &w, gp, X, M, &Yp, GB, slices, st);
         }
     }
     GemmPlan p = plan_gemm(ctx, w->L, M);
