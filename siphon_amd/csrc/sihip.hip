@@ -11,6 +11,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <mutex>
 #include <utility>
@@ -122,6 +124,10 @@ struct sihip_ctx {
     size_t d_in_cap = 0;
     void *d_out = nullptr;
     size_t d_out_cap = 0;
+    uint8_t *h_stage = nullptr;  // pinned staging of sihip_gemv (kStageBytes), made on first use
+    uint8_t *h_stage_dev = nullptr;  // its device address
+    bool h_stage_tried = false;
+    uint32_t h_seq = 0;  // calls that used it
     void *d_aux = nullptr;
     size_t d_aux_cap = 0;
     void *d_ws = nullptr;  // prefill GEMM: quantized activation planes
@@ -336,6 +342,7 @@ extern "C" void sihip_shutdown(sihip_ctx *ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
+    if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
     for (void *p : {ctx->d_in, ctx->d_out, ctx->d_aux, ctx->d_ws, ctx->d_gpart,
                     (void *)ctx->d_gcnt, ctx->d_attn})
         if (p) (void)hipFree(p);
@@ -3213,6 +3220,51 @@ extern "C" int sihip_synchronize(sihip_ctx *ctx) {
     return SIHIP_OK;
 }
 
+// ---- host vectors -----------------------------------------------------------------
+//
+// sihip_gemv's vectors are a few tens of KB, so a call is bound by round trips:
+// with two hipMemcpyAsync of pageable memory and a stream synchronization it
+// took 33 us, 8 to 15 of them the matvec (the 7 matrices of an 8B Q4_K_M layer
+// 235 us; so 193). Vectors up to kStageVec floats go
+// through pinned memory that small kernels read and write across the bus, and
+// the call waits for a word that the last of them stores. Longer ones keep the
+// copy engines.
+constexpr int64_t kStageVec = 65536;
+constexpr size_t kStageIn = 64, kStageOut = kStageIn + kStageVec * 4, kStageBytes = kStageOut + kStageVec * 4;
+constexpr int kStageThreads = 1024;
+
+// dst, src: 16-byte aligned with room for whole float4s. flag: NULL, or (one
+// workgroup) the word set to seq when every store before it is visible to the
+// host.
+__global__ __launch_bounds__(kStageThreads) void stage_copy_kernel(const float4 *src, float4 *dst, int n4,
+                                                                   uint32_t *flag, uint32_t seq) {
+    for (int i = (int)(blockIdx.x * kStageThreads + threadIdx.x); i < n4; i += (int)(gridDim.x * kStageThreads))
+        dst[i] = src[i];
+    if (!flag) return;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The context's staging memory, or NULL where pinned memory is not to be had.
+static uint8_t *host_stage(sihip_ctx *ctx) {
+    if (!ctx->h_stage_tried) {
+        ctx->h_stage_tried = true;
+        void *h = nullptr, *d = nullptr;
+        if (hipHostMalloc(&h, kStageBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+            (void)hipGetLastError();
+        } else if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipHostFree(h);
+        } else {
+            *(uint32_t *)h = 0;
+            ctx->h_stage = (uint8_t *)h;
+            ctx->h_stage_dev = (uint8_t *)d;
+        }
+    }
+    return ctx->h_stage;
+}
+
 extern "C" int sihip_gemv(sihip_ctx *ctx, const sihip_weight *w, const float *x, float *y,
                           int64_t n_out) {
     if (!ctx || !w || !x || !y) return set_err(ctx, SIHIP_EINVAL, "gemv: NULL argument");
@@ -3221,14 +3273,45 @@ extern "C" int sihip_gemv(sihip_ctx *ctx, const sihip_weight *w, const float *x,
                        (long long)w->L.n_out);
     HIP_OK(ctx, hipSetDevice(ctx->device));
     const size_t xb = (size_t)w->L.n_in * 4, yb = (size_t)n_out * 4;
-    int rc = ensure(ctx, &ctx->d_in, &ctx->d_in_cap, xb);
+    int rc = ensure(ctx, &ctx->d_in, &ctx->d_in_cap, (xb + 15) / 16 * 16);
     if (rc) return rc;
-    rc = ensure(ctx, &ctx->d_out, &ctx->d_out_cap, yb);
+    rc = ensure(ctx, &ctx->d_out, &ctx->d_out_cap, (yb + 15) / 16 * 16);
     if (rc) return rc;
-    HIP_OK(ctx, hipMemcpyAsync(ctx->d_in, x, xb, hipMemcpyHostToDevice, ctx->stream));
+    uint8_t *const h = w->L.n_in <= kStageVec && n_out <= kStageVec ? host_stage(ctx) : nullptr;
+    if (h) {
+        memcpy(h + kStageIn, x, xb);
+        const int n4 = (int)((xb + 15) / 16);
+        hipLaunchKernelGGL(stage_copy_kernel, dim3((unsigned)((n4 + kStageThreads - 1) / kStageThreads)),
+                           dim3(kStageThreads), 0, ctx->stream, (const float4 *)(ctx->h_stage_dev + kStageIn),
+                           (float4 *)ctx->d_in, n4, (uint32_t *)nullptr, 0u);
+        HIP_OK(ctx, hipGetLastError());
+    } else {
+        HIP_OK(ctx, hipMemcpyAsync(ctx->d_in, x, xb, hipMemcpyHostToDevice, ctx->stream));
+    }
     rc = run_matvec(ctx, w, (const float *)ctx->d_in, w->L.n_in, nullptr, 0, 1,
                     (float *)ctx->d_out, n_out, n_out, ctx->stream);
-    if (rc) return rc;
+    if (rc) {
+        if (h) (void)hipStreamSynchronize(ctx->stream);  // the copy reads the staging memory
+        return rc;
+    }
+    if (h) {
+        const uint32_t seq = ++ctx->h_seq;
+        hipLaunchKernelGGL(stage_copy_kernel, dim3(1), dim3(kStageThreads), 0, ctx->stream,
+                           (const float4 *)ctx->d_out, (float4 *)(ctx->h_stage_dev + kStageOut),
+                           (int)((yb + 15) / 16), (uint32_t *)ctx->h_stage_dev, seq);
+        HIP_OK(ctx, hipGetLastError());
+        // the word, for a bounded time; past it (a long queue, an error) the
+        // stream's own synchronization
+        const volatile uint32_t *flag = (const volatile uint32_t *)h;
+        const auto t0 = std::chrono::steady_clock::now();
+        bool done = false;
+        while (!(done = *flag == seq))
+            if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(300)) break;
+        std::atomic_thread_fence(std::memory_order_acquire);
+        if (!done) HIP_OK(ctx, hipStreamSynchronize(ctx->stream));
+        memcpy(y, h + kStageOut, yb);
+        return SIHIP_OK;
+    }
     HIP_OK(ctx, hipMemcpyAsync(y, ctx->d_out, yb, hipMemcpyDeviceToHost, ctx->stream));
     HIP_OK(ctx, hipStreamSynchronize(ctx->stream));
     return SIHIP_OK;
