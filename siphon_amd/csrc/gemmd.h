@@ -258,8 +258,9 @@ __attribute__((amdgpu_waves_per_eu(2))) void gemmd_kernel(GDArgs A) {
     auto step = [&](int c, const uint8_t *X, uint8_t *Xn, GDRaw<FMT> &rw) {
         // the record has arrived: issued after it were the weights of its own
         // step and, for each of the R - 2 later steps, a record and weights
-        // (at most; a shallower weight ring issued fewer)
-        wait_vm<(R - 2) * kD + (R - 1 < DW ? R - 1 : DW) * kW>();
+        // (at most; a shallower weight ring issued fewer); and this wave's reads
+        // of the slot before have returned, which the copy below overwrites
+        wait_vm_lds<(R - 2) * kD + (R - 1 < DW ? R - 1 : DW) * kW>();
         __builtin_amdgcn_s_barrier();
         fence();
         dma(clamp(c + R - 1), Xn);

@@ -147,6 +147,13 @@ __device__ inline void wait_vm() {
     static_assert(N >= 0 && N < 64, "vmcnt field");
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// The same, and until its LDS reads have returned: what a wave has to wait for
+// before a bare s_barrier after which others overwrite what it has read.
+template <int N>
+__device__ inline void wait_vm_lds() {
+    static_assert(N >= 0 && N < 64, "vmcnt field");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
 
 // The stored quants of K-step ks, n tile nt (16 slots, byte b of word i = slot
 // 4 i + b).

@@ -117,8 +117,9 @@ __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int m
     auto step = [&](int c, const uint8_t *X, uint8_t *Xn, SKRaw<FMT, 2> &rw) {
         // the record has arrived: issued after it were the weights of its own
         // step and, for each of the R - 2 later steps, a record and weights
-        // (at most; a shallower weight ring issued fewer)
-        wait_vm<(R - 2) * kD + (R - 1 < DW ? R - 1 : DW) * kW>();
+        // (at most; a shallower weight ring issued fewer); and this wave's reads
+        // of the slot before have returned, which the copy below overwrites
+        wait_vm_lds<(R - 2) * kD + (R - 1 < DW ? R - 1 : DW) * kW>();
         __builtin_amdgcn_s_barrier();
         fence();
         SKOps<FMT, 2> o;

@@ -1,0 +1,35 @@
+"""The order of copies, LDS reads and barriers in the compiled ring-buffered
+prompt GEMMs (pipeline_asm.py states it), on the CPU: a step that broke it
+would read a slot while it is written, which a GPU run shows only by chance."""
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+from . import pipeline_asm
+
+# (instance, ring slots): a ring of two and of more, weights as deep as the
+# ring and shallower, both segments of a pair, each record size class. Types:
+# F16 1, Q5_0 6, Q8_0 8, Q2_K 10, Q4_K 12, Q5_K 13, Q6_K 14
+INSTANCES = [
+    ("gemmx_kernel<10, 10, 2>(GXArgs)", 3),
+    ("gemmx_kernel<12, 14, 3>(GXArgs)", 3),
+    ("gemmx_kernel<13, 13, 5>(GXArgs)", 3),
+    ("gemmx_kernel<12, 12, 8>(GXArgs)", 2),
+    ("gemmd_kernel<1, 2>(GDArgs)", 4),
+    ("gemmd_kernel<1, 5>(GDArgs)", 3),
+    ("gemmd_kernel<6, 5>(GDArgs)", 4),
+    ("gemmd_kernel<8, 3>(GDArgs)", 4),
+]
+
+
+@pytest.fixture(scope="module")
+def broken():
+    """(instance) -> what its compiled code breaks."""
+    with ThreadPoolExecutor(4) as ex:
+        code = list(ex.map(lambda c: pipeline_asm.compile_kernel(c[0]), INSTANCES))
+    return {c[0]: pipeline_asm.violations(k, c[1]) for c, k in zip(INSTANCES, code)}
+
+
+@pytest.mark.parametrize("instance", [i for i, _ in INSTANCES])
+def test_no_copy_over_a_slot_being_read(broken, instance):
+    assert not broken[instance]["reads"]
