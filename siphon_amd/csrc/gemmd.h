@@ -255,12 +255,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void gemmd_kernel(GDArgs A) {
         fence();
     });
     constexpr int kW = gd_loads<FMT>();
-    auto step = [&](int c, const uint8_t *X, uint8_t *Xn, GDRaw<FMT> &rw) {
-        // the record has arrived: issued after it were the weights of its own
-        // step and, for each of the R - 2 later steps, a record and weights
-        // (at most; a shallower weight ring issued fewer); and this wave's reads
-        // of the slot before have returned, which the copy below overwrites
-        wait_vm_lds<(R - 2) * kD + (R - 1 < DW ? R - 1 : DW) * kW>();
+    auto step = [&](int c, auto younger, const uint8_t *X, uint8_t *Xn, GDRaw<FMT> &rw) {
+        // the record has arrived, and this wave's reads of the slot before have
+        // returned, which the copy below overwrites
+        wait_vm_lds<decltype(younger)::value>();
         __builtin_amdgcn_s_barrier();
         fence();
         dma(clamp(c + R - 1), Xn);
@@ -273,12 +271,14 @@ __attribute__((amdgpu_waves_per_eu(2))) void gemmd_kernel(GDArgs A) {
     // the last partial round
     constexpr int U = R % DW == 0 ? R : R * DW;
     int c = c0;
-    auto run = [&](auto u) {
-        step(c + u, slot(u), slot(std::integral_constant<int, (decltype(u)::value + R - 1) % R>()), raw[u % DW]);
+    auto run = [&](auto u, auto last) {
+        constexpr int v = decltype(u)::value, kY = gx_younger(R, DW, kD, kW, U, decltype(last)::value ? v : -1);
+        step(c + v, std::integral_constant<int, kY>(), slot(u), slot(std::integral_constant<int, (v + R - 1) % R>()),
+             raw[v % DW]);
     };
-    for (; c + U <= c1; c += U) gx_unroll<U>(run);
+    for (; c + U <= c1; c += U) gx_unroll<U>([&](auto u) { run(u, std::false_type()); });
     gx_unroll<U - 1>([&](auto u) {
-        if (c + u < c1) run(u);
+        if (c + u < c1) run(u, std::true_type());
     });
     v4f2_t(&y)[MT][2] = ys[0];
     if constexpr (gd_sums<FMT>() == 2) {

@@ -65,6 +65,18 @@ __device__ inline void gx_unroll(F f) {
     }
 }
 
+// The wave's operations younger than a step's record when the step waits for
+// it, at least: the records of the R - 2 later steps (kD copies each) and the
+// weights (kW loads a step) issued since, which are min(R - 1, DW) steps' worth
+// from the prologue on. Step u of the last partial round of U (u < 0: any step
+// of a whole one) counts only weights that a later step uses: the compiler may
+// drop the loads issued for steps U - 1 and beyond, one step's worth for each
+// step from U - 1 - DW on.
+__host__ __device__ constexpr int gx_younger(int R, int DW, int kD, int kW, int U, int u) {
+    const int kept = R - 1 < DW ? R - 1 : DW, dropped = u > U - 1 - DW ? u - (U - 1 - DW) : 0;
+    return (R - 2) * kD + (kept > dropped ? kept - dropped : 0) * kW;
+}
+
 template <uint32_t FMT, int MT>
 __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int mblk, int slice,
                                uint8_t *s0, uint8_t *s1, uint8_t *s2) {
@@ -114,12 +126,10 @@ __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int m
         fence();
     });
     constexpr int kW = sk_loads<FMT>();  // weight loads of a super-block
-    auto step = [&](int c, const uint8_t *X, uint8_t *Xn, SKRaw<FMT, 2> &rw) {
-        // the record has arrived: issued after it were the weights of its own
-        // step and, for each of the R - 2 later steps, a record and weights
-        // (at most; a shallower weight ring issued fewer); and this wave's reads
-        // of the slot before have returned, which the copy below overwrites
-        wait_vm_lds<(R - 2) * kD + (R - 1 < DW ? R - 1 : DW) * kW>();
+    auto step = [&](int c, auto younger, const uint8_t *X, uint8_t *Xn, SKRaw<FMT, 2> &rw) {
+        // the record has arrived, and this wave's reads of the slot before have
+        // returned, which the copy below overwrites
+        wait_vm_lds<decltype(younger)::value>();
         __builtin_amdgcn_s_barrier();
         fence();
         SKOps<FMT, 2> o;
@@ -143,12 +153,14 @@ __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int m
     };
     constexpr int U = R * DW;  // steps per round: ring slot and weight set static
     int c = c0;
-    auto run = [&](auto u) {
-        step(c + u, slot(u), slot(std::integral_constant<int, (decltype(u)::value + R - 1) % R>()), raw[u % DW]);
+    auto run = [&](auto u, auto last) {
+        constexpr int v = decltype(u)::value, kY = gx_younger(R, DW, kD, kW, U, decltype(last)::value ? v : -1);
+        step(c + v, std::integral_constant<int, kY>(), slot(u), slot(std::integral_constant<int, (v + R - 1) % R>()),
+             raw[v % DW]);
     };
-    for (; c + U <= c1; c += U) gx_unroll<U>(run);
+    for (; c + U <= c1; c += U) gx_unroll<U>([&](auto u) { run(u, std::false_type()); });
     gx_unroll<U - 1>([&](auto u) {
-        if (c + u < c1) run(u);
+        if (c + u < c1) run(u, std::true_type());
     });
     wait_vm<0>();  // no copy may land in the LDS of a workgroup that has ended
     const int64_t n0 = (int64_t)lblk * kG2BN + 32 * wave;

@@ -33,3 +33,8 @@ def broken():
 @pytest.mark.parametrize("instance", [i for i, _ in INSTANCES])
 def test_no_copy_over_a_slot_being_read(broken, instance):
     assert not broken[instance]["reads"]
+
+
+@pytest.mark.parametrize("instance", [i for i, _ in INSTANCES])
+def test_a_step_waits_for_its_record(broken, instance):
+    assert not broken[instance]["copies"]
