@@ -251,6 +251,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void gemmd_kernel(GDArgs A) {
     GDRaw<FMT> raw[DW];
     gx_unroll<(R - 1 > DW ? R - 1 : DW)>([&](auto i) {
         if constexpr (i < R - 1) dma(clamp(c0 + i), slot(i));
+        fence();
         if constexpr (i < DW) gd_load_w<FMT>(wr, clamp(c0 + i) * kStep, lane, raw[i]);
         fence();
     });

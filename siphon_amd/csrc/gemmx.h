@@ -109,6 +109,8 @@ __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int m
                 c * kRec + i * 1024, 0, 0);
         }
     };
+    // keep the order of issue: the counted waits rest on a record's copies coming
+    // before the weights of its step
     auto fence = [] {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -122,6 +124,7 @@ __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int m
     SKRaw<FMT, 2> raw[DW];
     gx_unroll<(R - 1 > DW ? R - 1 : DW)>([&](auto i) {
         if constexpr (i < R - 1) dma(clamp(c0 + i), slot(i));
+        fence();
         if constexpr (i < DW) sk_load_w<FMT, 2>(wr, clamp(c0 + i), 0, lane, raw[i]);
         fence();
     });
@@ -135,6 +138,7 @@ __device__ inline void gx_body(const GXArgs &A, const GXSeg &sg, int nblk, int m
         SKOps<FMT, 2> o;
         sk_decode<FMT, 2>(rw, 0, lane, o);
         dma(clamp(c + R - 1), Xn);
+        fence();
         sk_load_w<FMT, 2>(wr, clamp(c + DW), 0, lane, rw);
         fence();
 #pragma unroll
