@@ -3278,28 +3278,37 @@ extern "C" int sihip_gemv(sihip_ctx *ctx, const sihip_weight *w, const float *x,
     rc = ensure(ctx, &ctx->d_out, &ctx->d_out_cap, (yb + 15) / 16 * 16);
     if (rc) return rc;
     uint8_t *const h = w->L.n_in <= kStageVec && n_out <= kStageVec ? host_stage(ctx) : nullptr;
+    // on an error after a staged launch: what is queued reads and writes the
+    // staging memory, which the next call fills
+    auto drained = [&](int e) {
+        if (e && h) (void)hipStreamSynchronize(ctx->stream);
+        return e;
+    };
+    auto staged = [&]() -> int {
+        HIP_OK(ctx, hipGetLastError());
+        return SIHIP_OK;
+    };
     if (h) {
         memcpy(h + kStageIn, x, xb);
         const int n4 = (int)((xb + 15) / 16);
         hipLaunchKernelGGL(stage_copy_kernel, dim3((unsigned)((n4 + kStageThreads - 1) / kStageThreads)),
                            dim3(kStageThreads), 0, ctx->stream, (const float4 *)(ctx->h_stage_dev + kStageIn),
                            (float4 *)ctx->d_in, n4, (uint32_t *)nullptr, 0u);
-        HIP_OK(ctx, hipGetLastError());
+        rc = drained(staged());
+        if (rc) return rc;
     } else {
         HIP_OK(ctx, hipMemcpyAsync(ctx->d_in, x, xb, hipMemcpyHostToDevice, ctx->stream));
     }
-    rc = run_matvec(ctx, w, (const float *)ctx->d_in, w->L.n_in, nullptr, 0, 1,
-                    (float *)ctx->d_out, n_out, n_out, ctx->stream);
-    if (rc) {
-        if (h) (void)hipStreamSynchronize(ctx->stream);  // the copy reads the staging memory
-        return rc;
-    }
+    rc = drained(run_matvec(ctx, w, (const float *)ctx->d_in, w->L.n_in, nullptr, 0, 1,
+                            (float *)ctx->d_out, n_out, n_out, ctx->stream));
+    if (rc) return rc;
     if (h) {
         const uint32_t seq = ++ctx->h_seq;
         hipLaunchKernelGGL(stage_copy_kernel, dim3(1), dim3(kStageThreads), 0, ctx->stream,
                            (const float4 *)ctx->d_out, (float4 *)(ctx->h_stage_dev + kStageOut),
                            (int)((yb + 15) / 16), (uint32_t *)ctx->h_stage_dev, seq);
-        HIP_OK(ctx, hipGetLastError());
+        rc = drained(staged());
+        if (rc) return rc;
         // the word, for a bounded time; past it (a long queue, an error) the
         // stream's own synchronization
         const volatile uint32_t *flag = (const volatile uint32_t *)h;
