@@ -2057,8 +2057,19 @@ static SKPlan plan_gemmsk(int64_t M, int64_t nb) {
     return p;
 }
 
+// Whether an option puts M rows of a K-quant on one of the other GEMMs
+// (GEMMKS_MAX_M, GEMM2S_MAX_M, GEMM2_MIN_M, GEMM6_MIN_M): what it names keeps
+// its range, and gemmsk.h and gemmx.h, by their built-in rules, the rest.
+static bool placed_by_option(const Options &o, uint32_t type, int64_t M) {
+    if (o.gemmks_max_m >= 0 && M <= gemmks_max_m(o, type) && !(type == T_Q4_K && o.gemmks_q4k != 1)) return true;
+    if (type == T_Q4_K)
+        return (o.gemm2s_max_m >= 0 && M <= gemm2s_max_m(o)) || (o.gemm2_min_m > 0 && M >= o.gemm2_min_m);
+    return type == T_Q6_K && o.gemm6_min_m > 0 && M >= o.gemm6_min_m;
+}
+
 // Whether weights over one X take this launch: K-quants of one row length
-// and M in its range, unless an option sets the tiling of the other GEMMs.
+// and M in its range, unless an option sets the tiling of the other GEMMs or
+// puts M on one of them.
 // Under graph capture, where a missing weight copy cannot be built, the
 // kernel whose copies exist is taken.
 static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w,
@@ -2069,6 +2080,7 @@ static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight 
     for (int i = 0; i < count; i++) {
         const Layout &L = w[i]->L;
         if (!is_kquant(L.type) || L.n_in != w[0]->L.n_in || L.n_in % 256) return false;
+        if (ctx->opt.gemmsk_max_m < 0 && placed_by_option(ctx->opt, L.type, M)) return false;
         // a buffer's 32-bit offsets: a row block's chunks, an m block's records
         if (L.n_in / 256 * g2_rec_bytes(16) * 3 > INT32_MAX) return false;
         here = here && w[i]->gsmall;
@@ -2255,6 +2267,7 @@ static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *
     for (int i = 0; i < count; i++) {
         const Layout &L = w[i]->L;
         if (!is_kquant(L.type) || L.n_in != w[0]->L.n_in || L.n_in % 256) return false;
+        if (ctx->opt.gemmx_min_m < 0 && placed_by_option(ctx->opt, L.type, M)) return false;
         // 32-bit buffer offsets: a row block's chunks, an m block's records
         if (L.n_in / 256 * g2_rec_bytes(128) > INT32_MAX) return false;
         here = here && w[i]->gsmall;

@@ -1,0 +1,43 @@
+"""Which GEMM a call takes, on the CPU (host/fake_hip.cpp records the
+launches)."""
+import pytest
+
+from . import fake_hip
+
+
+def gemms(options, types, n_out, n_in, Ms):
+    """M -> the GEMM kernels of a call with one matrix per type."""
+    got = fake_hip.run(f"""
+        for name, value in {options!r}.items():
+            dev.set_option(name, value)
+        ws = [upload(getattr(sa, t), {n_out}, {n_in}) for t in {types!r}]
+        for w in ws:
+            w.prepare_gemm()
+        result = []
+        for M in {Ms!r}:
+            fake.fake_reset(0)
+            dev.gemm_multi_dev(ws, X, M, [X] * len(ws))
+            result.append([k[0] for k in launched() if "quantize" not in k[0] and "convert" not in k[0]])
+    """)
+    return dict(zip(Ms, got))
+
+
+@pytest.mark.parametrize("options,wt,want", [
+    ({"GEMMKS_MAX_M": 16}, "Q5_K", {9: "gemmks", 16: "gemmks", 17: "gemmsk"}),
+    ({"GEMMKS_MAX_M": 16}, "Q4_K", {9: "gemmsk", 16: "gemmsk"}),
+    ({"GEMMKS_MAX_M": 16, "GEMMKS_Q4K": 1}, "Q4_K", {9: "gemmks", 16: "gemmks", 17: "gemmsk"}),
+    ({"GEMMKS_MAX_M": 12}, "Q2_K", {12: "gemmks", 13: "gemmsk"}),
+    ({"GEMM2S_MAX_M": 16}, "Q4_K", {9: "gemm2s_q4k", 16: "gemm2s_q4k", 17: "gemmsk"}),
+    ({"GEMM2S_MAX_M": 16}, "Q5_K", {9: "gemmsk"}),
+    ({"GEMM2_MIN_M": 40}, "Q4_K", {39: "gemmsk", 40: "gemm2_q4k", 200: "gemm2_q4k"}),
+    ({"GEMM6_MIN_M": 20}, "Q6_K", {20: "gemm6_q6k", 64: "gemm6_q6k", 300: "gemm6_q6k"}),
+    ({"GEMM6_MIN_M": 1, "GEMMSK_MAX_M": 40}, "Q6_K", {40: "gemmsk", 41: "gemm6_q6k"}),
+    ({}, "Q6_K", {9: "gemmsk", 112: "gemmsk"}),
+    ({}, "Q4_K", {9: "gemmsk", 200: "gemmsk", 384: "gemm2_q4k"}),
+])
+def test_options_place_their_kernels(options, wt, want):
+    """An option that names one of the older K-quant GEMMs keeps the M it
+    names on it; the built-in rule has the rest, and the newer GEMMs' own
+    options go first."""
+    got = gemms(options, [wt], 1024, 2048, list(want))
+    assert {M: [k.split("_kernel")[0] for k in v] for M, v in got.items()} == {M: [k] for M, k in want.items()}
