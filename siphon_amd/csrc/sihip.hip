@@ -2070,10 +2070,10 @@ static bool placed_by_option(const Options &o, uint32_t type, int64_t M) {
 // Whether weights over one X take this launch: K-quants of one row length
 // and M in its range, unless an option sets the tiling of the other GEMMs or
 // puts M on one of them.
-// Under graph capture, where a missing weight copy cannot be built, the
-// kernel whose copies exist is taken.
+// Where a missing weight copy cannot be built (under graph capture, and with
+// noalloc), the kernel whose copies exist is taken.
 static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w,
-                            int64_t M, hipStream_t st) {
+                            int64_t M, hipStream_t st, bool noalloc = false) {
     if (count < 1 || count > kSKMaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
     if (gemmsk_max_m(ctx->opt) <= 0 || M < 9 || M < gemm_min_m(ctx->opt)) return false;
     bool here = true, other = true;
@@ -2086,7 +2086,7 @@ static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight 
         here = here && w[i]->gsmall;
         other = other && plan_copy(w[i], plan_gemm(ctx, L, M));
     }
-    if (here != other && capturing(st)) return here;
+    if (here != other && (noalloc || capturing(st))) return here;
     if (ctx->opt.gemmsk_max_m >= 0) return M <= ctx->opt.gemmsk_max_m;
     int64_t blocks = 0;
     for (int i = 0; i < count; i++) blocks += (w[i]->L.n_out + 31) / 32;
@@ -2260,7 +2260,7 @@ static GemmPlan plan_gemmx(const sihip_ctx *ctx, int64_t M, int64_t nb, int64_t 
 }
 
 static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M,
-                           hipStream_t st) {
+                           hipStream_t st, bool noalloc = false) {
     if (count < 1 || count > kG2MaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
     if (ctx->opt.gemmx_min_m == 0 || M < 9 || M < gemm_min_m(ctx->opt)) return false;
     bool here = true, other = true;
@@ -2273,7 +2273,7 @@ static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *
         here = here && w[i]->gsmall;
         other = other && plan_copy(w[i], plan_gemm(ctx, L, M));
     }
-    if (here != other && capturing(st)) return here;
+    if (here != other && (noalloc || capturing(st))) return here;
     if (ctx->opt.gemmx_min_m > 0) return M >= ctx->opt.gemmx_min_m;
     // Q4_K from M = kGemm2MinM runs on gemm2.h, whose copy holds the scales
     // and mins split beforehand (8B gate + up at M = 2048 502 us against 520
@@ -2981,13 +2981,29 @@ extern "C" int sihip_gemm_dev_noalloc(sihip_ctx *ctx, const sihip_weight *w, con
         if (rc) return rc;
         return done ? SIHIP_OK : set_err(ctx, SIHIP_EINVAL, "gemm_dev_noalloc: no fused instance");
     }
-    if (w->gsmall && gemmsk_eligible(ctx, 1, &w, M, st)) {
-        const SKPlan sp = plan_gemmsk(M, w->L.n_in / 256);
+    GemmPlan p = plan_gemm(ctx, w->L, M);
+    const bool planned = plan_copy(w, p) != nullptr;
+    if (w->gsmall && gemmsk_eligible(ctx, 1, &w, M, st, true)) {
+        const int64_t nb = w->L.n_in / 256;
         float *Yp = Y;
-        if ((size_t)sp.ws_bytes <= room)  // else the kernels below, whose planes are smaller
+        SKPlan sp = plan_gemmsk(M, nb);
+        if ((size_t)sp.ws_bytes <= room)  // else the kernels below
             return launch_gemmsk_group(ctx, 1, &w, sp, X, M, &Yp, ctx->scratch, st);
+        // planes that only the plan's kernel fits into the scratch, whose copy
+        // is missing: pieces of whole m blocks of three 16-row tiles
+        const int64_t piece = (int64_t)(room / (size_t)(nb * g2_rec_bytes(16))) / 3 * 48;
+        if (!planned && (size_t)p.ws_bytes <= room && piece > 0) {
+            for (int64_t m = 0; m < M; m += piece) {
+                const int64_t n = std::min(piece, M - m);
+                Yp = Y + m * w->L.n_out;
+                sp = plan_gemmsk(n, nb);
+                const int rc = launch_gemmsk_group(ctx, 1, &w, sp, X + m * w->L.n_in, n, &Yp, ctx->scratch, st);
+                if (rc) return rc;
+            }
+            return SIHIP_OK;
+        }
     }
-    if (w->gsmall && gemmx_eligible(ctx, 1, &w, M, st)) {
+    if (w->gsmall && gemmx_eligible(ctx, 1, &w, M, st, true)) {
         const GemmPlan gp = plan_gemmx(ctx, M, w->L.n_in / 256, gemm_blocks(1, &w));
         const size_t off = ((size_t)gp.ws_bytes + 255) & ~(size_t)255;
         float *Yp = Y;
@@ -3007,8 +3023,7 @@ extern "C" int sihip_gemm_dev_noalloc(sihip_ctx *ctx, const sihip_weight *w, con
             return launch_gemmd_group(ctx, 1, &w, gp, X, M, &Yp, GB, slices, st);
         }
     }
-    GemmPlan p = plan_gemm(ctx, w->L, M);
-    if (!plan_copy(w, p))
+    if (!planned)
         return set_err(ctx, SIHIP_EINVAL,
                        "gemm_dev_noalloc: the weight has no GEMM copy; call "
                        "sihip_weight_prepare_gemm first");

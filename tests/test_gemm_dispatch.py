@@ -41,3 +41,23 @@ def test_options_place_their_kernels(options, wt, want):
     options go first."""
     got = gemms(options, [wt], 1024, 2048, list(want))
     assert {M: [k.split("_kernel")[0] for k in v] for M, v in got.items()} == {M: [k] for M, k in want.items()}
+
+
+@pytest.mark.parametrize("wt,n_out,n_in,M,launches", [
+    *[(wt, *c, 1) for wt in ("Q2_K", "Q3_K", "Q5_K", "Q6_K")
+      for c in ((256, 2048, 600), (1024, 4096, 2000), (4096, 14336, 300))],
+    # the planes of 1000 rows exceed the scratch: two pieces
+    *[(wt, 4096, 14336, 1000, 2) for wt in ("Q2_K", "Q3_K", "Q5_K")],
+])
+def test_noalloc_after_a_short_prompt(wt, n_out, n_in, M, launches):
+    """A weight whose first GEMM call was a short prompt holds the copy of that
+    prompt's kernel alone; sihip_gemm_dev_noalloc takes it for a longer one
+    rather than refuse a call that only lacks the other copy."""
+    got = fake_hip.run(f"""
+        w = upload(sa.{wt}, {n_out}, {n_in})
+        dev.gemm_dev(w, X, 40, X)
+        fake.fake_reset(0)
+        dev.gemm_dev_noalloc(w, X, {M}, X)
+        result = [k[0] for k in launched() if "quantize" not in k[0]]
+    """)
+    assert len(got) == launches and all(k.startswith(("gemmsk", "gemmx", "gemm6", "gemm_kq")) for k in got), got

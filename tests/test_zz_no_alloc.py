@@ -139,3 +139,28 @@ def test_noalloc_graph_replays(dev):
         for b in (xd, x2, ye, yg, y2):
             b.free()
         w.free()
+
+
+@pytest.mark.parametrize("wt,n_out,n_in,M", [
+    (sa.Q5_K, 48, 14336, 1000),  # two pieces, the second of 40 rows
+    (sa.Q6_K, 70, 2048, 600),
+])
+def test_noalloc_on_the_copy_of_a_shorter_call(dev, oracle, wt, n_out, n_in, M):
+    """The weight holds the copy of a 40-row call's kernel alone; a longer
+    noalloc call runs on it, in pieces where its planes exceed the scratch."""
+    rng = np.random.default_rng(n_out + M)
+    W = synth.make_weights(wt, n_out, n_in, rng)
+    X = rng.standard_normal((M, n_in)).astype(np.float32)
+    w = dev.upload(wt, n_out, n_in, W)
+    xd, yd = dev.to_device(X), dev.to_device(np.full(M * n_out, np.nan, np.float32))
+    try:
+        dev.gemm_dev(w, xd.ptr, 40, yd.ptr)
+        dev.gemm_dev_noalloc(w, xd.ptr, M, yd.ptr)
+        dev.synchronize()
+        ref, L1 = oracle.gemm(wt, W, n_out, n_in, X)
+        assert_close(yd.to_host(np.float32, M * n_out), ref.reshape(-1).astype(np.float64), L1.reshape(-1),
+                     f"{sa.NAMES[wt]} M={M}")
+    finally:
+        xd.free()
+        yd.free()
+        w.free()
