@@ -36,6 +36,7 @@
 namespace sihip {
 
 constexpr int kAttnMaxHd = 512;
+constexpr int64_t kAttnMaxN = (int64_t)1 << 29;  // positions, so that indexes stay ints
 constexpr int kAttnHeads = 4;  // query heads per workgroup of the scores launch
 constexpr int64_t kAttnWsBlock = 4096;  // positions that workspace rows are a multiple of
 
@@ -52,8 +53,16 @@ struct AttnArgs {
     int64_t n_ctx, ld, lw;
     int n, hd, gqa, n_kv;
     int nbs, nbe;
+    int gx;                // blocks per row of the grid (attn_block)
     float kq_scale;
 };
+
+// The scores and exponential launches have a block per piece of a head's
+// positions, which can be more than one grid dimension takes (2^32 work items:
+// 32 heads over 1 KV head at 2^27 positions): past kAttnGridX blocks the grid
+// has further rows, the last one with blocks to spare.
+constexpr int64_t kAttnGridX = (int64_t)1 << 22;
+__device__ inline int attn_block(const AttnArgs &A) { return (int)blockIdx.y * A.gx + (int)blockIdx.x; }
 
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 
@@ -157,8 +166,8 @@ __device__ inline float tail_exp(float x) { return (float)exp((double)x); }
 struct AttnWg {
     int hk, h, blk;
 };
-__device__ inline AttnWg attn_wg(const AttnArgs &A) {
-    const int id = (int)blockIdx.x, rest = id / A.n_kv;
+__device__ inline AttnWg attn_wg(const AttnArgs &A, int id) {
+    const int rest = id / A.n_kv;
     AttnWg w;
     w.hk = id % A.n_kv;
     w.h = w.hk * A.gqa + rest % A.gqa;
@@ -264,8 +273,9 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
     __shared__ __attribute__((aligned(16))) uint16_t q16[kAttnHeads][kAttnMaxHd];
     __shared__ float red[kAttnHeads][4];
     const int chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
-    const int id = (int)blockIdx.x, hk = id % A.n_kv, rest = id / A.n_kv;
+    const int id = attn_block(A), hk = id % A.n_kv, rest = id / A.n_kv;
     const int hc = rest % chunks * kAttnHeads, blk = rest / chunks;
+    if (blk >= A.nbs) return;
     const int h0 = hk * A.gqa + hc, nh = min(kAttnHeads, A.gqa - hc);
     const int hd = A.hd;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, L = lane & 3;
@@ -332,7 +342,8 @@ constexpr int kAttnExpBlock = 1024;
 __global__ __launch_bounds__(256) void attn_exp_kernel(AttnArgs A) {
     __shared__ float redf[4];
     __shared__ double redd[4];
-    const AttnWg W = attn_wg(A);
+    const AttnWg W = attn_wg(A, attn_block(A));
+    if (W.blk >= A.nbe) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int j = W.blk * kAttnExpBlock + 4 * (int)threadIdx.x;
     float4 *const p = reinterpret_cast<float4 *>(A.sw + (int64_t)W.h * A.lw + j);
@@ -479,7 +490,7 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
     __shared__ __attribute__((aligned(16))) uint8_t ring[kR * kAttnSlot];
     __shared__ __attribute__((aligned(16))) float se[kR][kAttnChunk];
     __shared__ __attribute__((aligned(16))) uint16_t sp[2][kAttnChunk];
-    const AttnWg W = attn_wg(A);
+    const AttnWg W = attn_wg(A, (int)blockIdx.x);
     const int tid = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r = tid >> 4, L = tid & 15;
     const int rows = min(kAttnPvRows, A.hd - W.blk * kAttnPvRows);
@@ -627,7 +638,7 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ float redf[8];
     __shared__ double redd[8];
-    const AttnWg W = attn_wg(A);
+    const AttnWg W = attn_wg(A, (int)blockIdx.x);
     const int n = A.n, np = attn_fused_np(n), hd = A.hd;
     uint16_t *const sq = reinterpret_cast<uint16_t *>(smem);
     float *const ss = reinterpret_cast<float *>(smem + kAttnMaxHd * 2);

@@ -3062,6 +3062,9 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
     if (n_ctx < 1 || n_ctx > (int64_t)INT32_MAX || pos < 0 || pos >= n_ctx)
         return set_err(ctx, SIHIP_EINVAL, "attn_decode_dev: pos %lld outside 0..n_ctx-1 (n_ctx %lld)",
                        (long long)pos, (long long)n_ctx);
+    if (pos >= kAttnMaxN)
+        return set_err(ctx, SIHIP_EINVAL, "attn_decode_dev: pos %lld past %lld positions", (long long)pos,
+                       (long long)kAttnMaxN);
     HIP_OK(ctx, hipSetDevice(ctx->device));
     AttnArgs A;
     A.q = q;
@@ -3124,14 +3127,20 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
         else
             hipLaunchKernelGGL((attn_fused_kernel<16, false>), g, t, lds, st, A);
     } else {
-        const dim3 g((unsigned)gs), t(256);
+        const dim3 t(256);
+        auto rows = [&](int64_t blocks) {
+            A.gx = (int)std::min(blocks, kAttnGridX);
+            return dim3((unsigned)A.gx, (unsigned)((blocks + A.gx - 1) / A.gx));
+        };
+        const dim3 g = rows(gs);
         if (kvec && narrow)
             hipLaunchKernelGGL((attn_scores_kernel<4, true>), g, t, 0, st, A);
         else if (kvec)
             hipLaunchKernelGGL((attn_scores_kernel<16, true>), g, t, 0, st, A);
         else
             hipLaunchKernelGGL((attn_scores_kernel<16, false>), g, t, 0, st, A);
-        hipLaunchKernelGGL(attn_exp_kernel, dim3((unsigned)ge), t, 0, st, A);
+        const dim3 eg = rows(ge);
+        hipLaunchKernelGGL(attn_exp_kernel, eg, t, 0, st, A);
         if (vvec)
             hipLaunchKernelGGL(attn_pv_kernel<true>, dim3((unsigned)gv), t, 0, st, A);
         else

@@ -33,3 +33,22 @@ def test_block_edges(dev, oracle, option, n_head, n_kv, hd, n_ctx, n, fuse):
     args = (dev, q, k, v, n_head, n_kv, hd, n_ctx, n - 1, kq)
     check(run_attn(*args), want, n, f"hd={hd} n={n} fuse={fuse}")
     assert np.array_equal(bits(run_attn(*args, caller_buffers=False)[0]), bits(want[0]))
+
+
+def test_more_blocks_than_one_grid_row(dev):
+    """1025 heads of 2^18 positions: 4 198 400 score blocks, past the 2^22 of
+    a grid row. Equal scores give probabilities of 2^-18 exactly, so each
+    head's output is its (constant) value."""
+    nh, n = 1025, 1 << 18
+    one = np.float16(1).view(np.uint16)
+    c = np.arange(1, nh + 1).astype(np.float16)
+    bufs = [dev.to_device(a) for a in (np.ones(nh, np.float32), np.full(nh * n, one, np.uint16),
+                                       np.repeat(c.view(np.uint16), n), np.full(nh, np.nan, np.float32))]
+    try:
+        q, k, v, out = (b.ptr for b in bufs)
+        dev.attn_decode_dev(q, k, v, nh, nh, 1, n, n - 1, 1.0, out)
+        dev.synchronize()
+        assert np.array_equal(bufs[3].to_host(np.float32, nh), c.astype(np.float32))
+    finally:
+        for b in bufs:
+            b.free()
