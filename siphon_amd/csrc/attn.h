@@ -463,7 +463,9 @@ __device__ inline float row_tree1(float a) {  // 32 lanes, 1 each
 }
 
 // res plus the tail [body, n) of a dot, added in order in double; v and p:
-// f16 rows of the 32-element block at body (16-byte aligned LDS).
+// f16 rows of the 32-element block at body (LDS, 16-byte aligned, v with
+// ALIGNED).
+template <bool ALIGNED>
 __device__ inline float add_tail(float res, const uint16_t *v, const uint16_t *p, int cnt) {
     double total = 0.0;
     total += (double)res;
@@ -471,7 +473,12 @@ __device__ inline float add_tail(float res, const uint16_t *v, const uint16_t *p
         h8_t vv[4], pp[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            vv[i] = reinterpret_cast<const h8_t *>(v)[i];
+            if constexpr (ALIGNED) {
+                vv[i] = reinterpret_cast<const h8_t *>(v)[i];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) vv[i][e] = reinterpret_cast<const _Float16 *>(v)[8 * i + e];
+            }
             pp[i] = reinterpret_cast<const h8_t *>(p)[i];
         }
 #pragma unroll
@@ -482,8 +489,12 @@ __device__ inline float add_tail(float res, const uint16_t *v, const uint16_t *p
 }
 
 // VEC: n_ctx % 8 == 0, v 16-byte aligned and the workgroup's rows within a
-// buffer's 4 GiB; else the value rows are staged by single elements, a chunk
-// at a time.
+// buffer's 4 GiB. Else the rows start anywhere in a 16-byte granule of memory:
+// a row's 16 lanes, which alone read it, load the whole granules that hold
+// its chunk (65 of them; a granule with an element of the row lies in the
+// row's pages, and what else it holds is not used) a chunk ahead into registers
+// and put them into its LDS slot, and the chains read at the row's shift. (By single elements, a
+// chunk at a time: 8B shape at n = 4000, n_ctx 4001, 59.5 us per layer; so 14.9.)
 template <bool VEC>
 __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
     constexpr int kR = VEC ? kAttnRing : 1;
@@ -535,6 +546,22 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
         for (int i = 0; i + 1 < kR; i++) dma(i);
     }
     const float scale = (float)(1.0 / wave_sum(part));
+    // without VEC: the granules of this lane's row, 64 a chunk and one more
+    const uint16_t *const vrow = vb + (int64_t)min(r, rows - 1) * A.n_ctx;
+    const int shift = VEC ? 0 : (int)((uintptr_t)vrow & 15) / 2, last = (shift + n - 1) >> 3;
+    const uint4 *const gran = reinterpret_cast<const uint4 *>(vrow - shift);
+    struct Staged {
+        uint4 v0, v1, v2, v3, v4;
+        float2 e;
+    };
+    auto load_v = [&](int ch) {
+        const int g = ch * (kAttnChunk / 8) + L;
+        return Staged{gran[min(g, last)], gran[min(g + 16, last)], gran[min(g + 32, last)], gran[min(g + 48, last)],
+                      L == 0 ? gran[min(g + 64, last)] : make_uint4(0, 0, 0, 0),
+                      reinterpret_cast<const float2 *>(eb + (int64_t)ch * kAttnChunk)[tid]};
+    };
+    Staged st{};
+    if constexpr (!VEC) st = load_v(0);
     // the probabilities of chunk ch from its exponentials e
     auto put_p = [&](int ch, float2 e) {
         const uint32_t p0 = f32_to_f16_hw(e.x * scale), p1 = f32_to_f16_hw(e.y * scale);
@@ -565,36 +592,40 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
             __syncthreads();
             dma(ch + kR - 1);
         } else {
-            __syncthreads();
-            for (int i = tid; i < kAttnPvRows * kAttnChunk; i += 256) {
-                const int rr = i / kAttnChunk, e = i % kAttnChunk;
-                if (s0 + e < n)
-                    reinterpret_cast<uint16_t *>(ring + rr * kAttnRowSlot)[e] =
-                        vb[(int64_t)min(rr, rows - 1) * A.n_ctx + s0 + e];
-            }
-            put_p(ch, reinterpret_cast<const float2 *>(eb + s0)[tid]);
+            uint4 *const dst = reinterpret_cast<uint4 *>(ring + r * kAttnRowSlot) + L;
+            dst[0] = st.v0, dst[16] = st.v1, dst[32] = st.v2, dst[48] = st.v3;
+            if (L == 0) dst[64] = st.v4;
+            put_p(ch, st.e);
+            st = load_v(min(ch + 1, nchunk - 1));
             __syncthreads();
         }
-        const uint32_t *const vs = reinterpret_cast<const uint32_t *>(slot + r * kAttnRowSlot) + L;
+        const uint32_t *const vs = reinterpret_cast<const uint32_t *>(slot + r * kAttnRowSlot) + (shift >> 1) + L;
         const uint32_t *const ps = reinterpret_cast<const uint32_t *>(sp[ch & 1]) + L;
+        // elements 2 L and 2 L + 1 of step t (across two words where the row's
+        // shift is odd: an unaligned LDS read of a word took 4 times as long)
+        auto pair = [&](int t) -> uint32_t {
+            if constexpr (VEC) return vs[16 * t];
+            else return __builtin_amdgcn_alignbit(vs[16 * t + 1], vs[16 * t], (uint32_t)(shift & 1) * 16);
+        };
         auto chain = [&](uint32_t vw, uint32_t pw) {
             a0 = __builtin_fmaf(f16_bits_to_f32(vw & 0xffffu), f16_bits_to_f32(pw & 0xffffu), a0);
             a1 = __builtin_fmaf(f16_bits_to_f32(vw >> 16), f16_bits_to_f32(pw >> 16), a1);
         };
         const int steps = min(body - s0, kAttnChunk) >> 5;
-        if (VEC && steps == kAttnChunk / 32) {
+        if (steps == kAttnChunk / 32) {
             // a whole chunk: all its reads go out first
             uint32_t vw[kAttnChunk / 32], pw[kAttnChunk / 32];
-            const float2 e = reinterpret_cast<const float2 *>(se[(ch + 1) % kR])[tid];
+            float2 e;
+            if constexpr (VEC) e = reinterpret_cast<const float2 *>(se[(ch + 1) % kR])[tid];
 #pragma unroll
-            for (int t = 0; t < kAttnChunk / 32; t++) vw[t] = vs[16 * t], pw[t] = ps[16 * t];
-            put_p(ch + 1, e);
+            for (int t = 0; t < kAttnChunk / 32; t++) vw[t] = pair(t), pw[t] = ps[16 * t];
+            if constexpr (VEC) put_p(ch + 1, e);
 #pragma unroll
             for (int t = 0; t < kAttnChunk / 32; t++) chain(vw[t], pw[t]);
         } else {
             if (VEC && ch + 1 < nchunk) put_p(ch + 1, reinterpret_cast<const float2 *>(se[(ch + 1) % kR])[tid]);
 #pragma unroll 4
-            for (int t = 0; t < steps; t++) chain(vs[16 * t], ps[16 * t]);
+            for (int t = 0; t < steps; t++) chain(pair(t), ps[16 * t]);
         }
     }
     const float res = row_tree2(a0, a1);
@@ -602,8 +633,8 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
     if (L == 0 && r < rows) {
         const int b0 = body % kAttnChunk;
         A.out[(int64_t)W.h * A.hd + W.blk * kAttnPvRows + r] =
-            add_tail(res, reinterpret_cast<const uint16_t *>(slot + r * kAttnRowSlot) + b0,
-                     sp[(nchunk - 1) & 1] + b0, n - body);
+            add_tail<VEC>(res, reinterpret_cast<const uint16_t *>(slot + r * kAttnRowSlot) + shift + b0,
+                          sp[(nchunk - 1) & 1] + b0, n - body);
     }
     // no copy may land in the LDS of a workgroup that has ended
     if constexpr (VEC) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -752,7 +783,7 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
 #pragma unroll 8
     for (int i = a; i < body; i += 32) acc = __builtin_fmaf(f16_bits_to_f32(vs[i]), f16_bits_to_f32(sp[i]), acc);
     const float res = row_tree1(acc);
-    if (a == 0 && c < hd) A.out[(int64_t)W.h * hd + c] = add_tail(res, vs + body, sp + body, n - body);
+    if (a == 0 && c < hd) A.out[(int64_t)W.h * hd + c] = add_tail<true>(res, vs + body, sp + body, n - body);
 }
 
 }  // namespace sihip

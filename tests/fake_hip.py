@@ -40,7 +40,7 @@ def run(code, lib=None):
 def kernel(text):
     """"sihip::gemmx_kernel<12u, 14u, 5>(...)" -> "gemmx_kernel<12,14,5>"."""
     m = re.match(r"(?:void )?sihip::(\w+)(<[^>]*>)?", text)
-    return m.group(1) + re.sub(r"[u ]", "", m.group(2) or "")
+    return m.group(1) + re.sub(r"(?<=\d)u| ", "", m.group(2) or "")
 
 
 def _main():
