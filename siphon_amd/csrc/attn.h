@@ -31,6 +31,8 @@
 // survives the f16 rounding of its probability only rarely.
 #pragma once
 
+#include <type_traits>
+
 #include "quant.h"
 
 namespace sihip {
@@ -180,43 +182,49 @@ __device__ inline AttnWg attn_wg(const AttnArgs &A, int id) {
 // Four lanes score one position: lane L of the quad holds accumulators
 // 8 L .. 8 L + 7, so a 32-element step of the key row is one 16-byte load per
 // lane and a wave's 16 rows are one contiguous span of the cache. T: 32-steps
-// kept in registers (hd / 32 <= T); VEC: 16-byte loads (hd % 8 == 0, keys
-// 16-byte aligned).
+// kept in registers (hd / 32 <= T); W: elements per load, 8 (hd % 8 == 0, keys
+// 16-byte aligned), 4 (hd % 4 == 0, 8-byte aligned) or 1.
 // (lane L < hd % 32 / 8 also holds elements 8 L .. + 7 past the last whole
-// step in tail; without VEC the tail is read where it is added.)
+// step in tail, zeros past hd.)
 template <int T>
 struct KeyRow {
     uint4 w[T];
     uint4 tail;
 };
 
-template <int T, bool VEC>
+// Elements p[0 .. cnt) of eight, zeros behind (cnt > 0; with W = 8 all of
+// them, with W = 4 the first four or all).
+template <int W>
+__device__ inline uint4 load_key8(const uint16_t *p, int cnt) {
+    if constexpr (W == 8) {
+        return *reinterpret_cast<const uint4 *>(p);
+    } else if constexpr (W == 4) {
+        const uint2 a = *reinterpret_cast<const uint2 *>(p);
+        const uint2 b = cnt > 4 ? *reinterpret_cast<const uint2 *>(p + 4) : make_uint2(0, 0);
+        return make_uint4(a.x, a.y, b.x, b.y);
+    } else {
+        uint32_t e[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) e[i] = i < cnt ? p[i] : 0u;
+        return make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
+    }
+}
+
+template <int T, int W>
 __device__ inline void load_key(const uint16_t *row, int hd, int L, KeyRow<T> &k) {
     const int steps = hd >> 5;
 #pragma unroll
     for (int t = 0; t < T; t++)
-        if (t < steps) {
-            const uint16_t *p = row + 32 * t + 8 * L;
-            if constexpr (VEC) {
-                k.w[t] = *reinterpret_cast<const uint4 *>(p);
-            } else {
-                uint32_t e[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) e[i] = (uint32_t)p[2 * i] | ((uint32_t)p[2 * i + 1] << 16);
-                k.w[t] = make_uint4(e[0], e[1], e[2], e[3]);
-            }
-        }
-    if (VEC && (hd & 31))
-        k.tail = 8 * L < (hd & 31) ? *reinterpret_cast<const uint4 *>(row + 32 * steps + 8 * L)
-                                   : make_uint4(0, 0, 0, 0);
+        if (t < steps) k.w[t] = load_key8<W>(row + 32 * t + 8 * L, 8);
+    if (hd & 31)
+        k.tail = 8 * L < (hd & 31) ? load_key8<W>(row + 32 * steps + 8 * L, (hd & 31) - 8 * L) : make_uint4(0, 0, 0, 0);
 }
 
-// The scaled score of the quad's row against the f16 query qh (LDS, 16-byte
-// aligned; q: the lane's elements of it, as load_key lays them out); valid in
-// the quad's lane 0. Every lane of the wave takes part.
-template <int T, bool VEC>
-__device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, const uint16_t *row,
-                                  const uint16_t *qh, int hd, int L, float kq_scale) {
+// The scaled score of the quad's row against the f16 query (q: the lane's
+// elements of it, as load_key lays them out; in its tail anything past hd);
+// valid in the quad's lane 0. Every lane of the wave takes part.
+template <int T, int W>
+__device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, int hd, float kq_scale) {
     const int steps = hd >> 5;
     float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -238,24 +246,23 @@ __device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, const 
     double total = 0.0;
     total += (double)res;
     if (hd & 31) {
-        if constexpr (VEC) {
-            // each lane's products, added in element order (8 per lane)
-            const h8_t kk = __builtin_bit_cast(h8_t, k.tail), qq = __builtin_bit_cast(h8_t, q.tail);
-            float pr[8];
+        // each lane's products, added in element order (8 per lane)
+        const h8_t kk = __builtin_bit_cast(h8_t, k.tail), qq = __builtin_bit_cast(h8_t, q.tail);
+        float pr[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) pr[e] = (float)kk[e] * (float)qq[e];
+        for (int e = 0; e < 8; e++) pr[e] = (float)kk[e] * (float)qq[e];
+        auto add = [&](auto from, int cnt) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) total += (double)quad_bcast<0>(pr[e]);
-            if ((hd & 31) > 8)
-#pragma unroll
-                for (int e = 0; e < 8; e++) total += (double)quad_bcast<1>(pr[e]);
-            if ((hd & 31) > 16)
-#pragma unroll
-                for (int e = 0; e < 8; e++) total += (double)quad_bcast<2>(pr[e]);
-        } else if (L == 0) {
-            for (int i = 32 * steps; i < hd; i++)
-                total += (double)(f16_at(row, i) * f16_bits_to_f32(qh[i]));
-        }
+            for (int e = 0; e < 8; e++) {
+                if (e % W == 0 && e >= cnt) break;
+                total += (double)quad_bcast<decltype(from)::value>(pr[e]);
+            }
+        };
+        const int cnt = hd & 31;
+        add(std::integral_constant<int, 0>(), cnt);
+        if (cnt > 8) add(std::integral_constant<int, 1>(), cnt - 8);
+        if (cnt > 16) add(std::integral_constant<int, 2>(), cnt - 16);
+        if (W < 8 && cnt > 24) add(std::integral_constant<int, 3>(), cnt - 24);
     }
     return (float)total * kq_scale;
 }
@@ -268,7 +275,7 @@ __device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, const 
 // is in flight at once.
 constexpr int kAttnScoreBlock = 64;
 
-template <int T, bool VEC>
+template <int T, int W>
 __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
     __shared__ __attribute__((aligned(16))) uint16_t q16[kAttnHeads][kAttnMaxHd];
     __shared__ float red[kAttnHeads][4];
@@ -283,7 +290,7 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
     // rows past n score row n - 1, unstored
     const uint16_t *row = A.k + ((int64_t)hk * A.n_ctx + (j < A.n ? j : A.n - 1)) * hd;
     KeyRow<T> kr;
-    load_key<T, VEC>(row, hd, L, kr);
+    load_key<T, W>(row, hd, L, kr);
     // the query heads in f16, staged while the key loads are in flight
     for (int hh = 0; hh < nh; hh++)
         for (int i = threadIdx.x; i < hd; i += 256)
@@ -291,8 +298,8 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
     __syncthreads();
     for (int hh = 0; hh < nh; hh++) {
         KeyRow<T> qr;
-        load_key<T, true>(q16[hh], hd, L, qr);
-        const float v = key_score<T, VEC>(kr, qr, row, q16[hh], hd, L, A.kq_scale);
+        load_key<T, 8>(q16[hh], hd, L, qr);
+        const float v = key_score<T, W>(kr, qr, hd, A.kq_scale);
         const bool real = L == 0 && j < A.n;
         if (real) {
             A.sw[(int64_t)(h0 + hh) * A.lw + j] = v;
@@ -663,7 +670,8 @@ __host__ __device__ inline int attn_fused_lds(int n) {
     return np * 4 + np * 2 + kAttnPvRows * (np * 2 + 64) + kAttnMaxHd * 2;
 }
 
-template <int T, bool VEC>
+// VEC: value rows by 16-byte loads (n_ctx % 8 == 0, v 16-byte aligned).
+template <int T, int KW, bool VEC>
 __global__ __launch_bounds__(kAttnFusedThreads)
 __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(AttnArgs A) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -687,12 +695,12 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
     const int passes = (n + 127) / 128;
     constexpr int kD = T <= 4 ? 2 : 1;  // passes of key rows held
     KeyRow<T> kr[kD];
-    load_key<T, VEC>(key_row(0), hd, L4, kr[0]);
+    load_key<T, KW>(key_row(0), hd, L4, kr[0]);
     float qv = 0.0f;
     if (tid < hd) qv = A.q[(int64_t)W.h * hd + tid];
 #pragma unroll
     for (int i = 1; i < kD; i++)
-        if (i < passes) load_key<T, VEC>(key_row(i), hd, L4, kr[i]);
+        if (i < passes) load_key<T, KW>(key_row(i), hd, L4, kr[i]);
     // value rows: 32 lanes per row; rows past hd repeat the last, positions
     // past n are not used
     const int r = tid >> 5, a = tid & 31;
@@ -710,15 +718,15 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
     if (tid < hd) sq[tid] = (uint16_t)f32_to_f16_hw(qv);
     __syncthreads();
     KeyRow<T> qr;
-    load_key<T, true>(sq, hd, L4, qr);
+    load_key<T, 8>(sq, hd, L4, qr);
     float mx = -__builtin_inff();
     for (int p0 = 0; p0 < passes; p0 += kD) {
 #pragma unroll
         for (int u = 0; u < kD; u++) {
             const int pass = p0 + u;
             if (pass < passes) {
-                const float v = key_score<T, VEC>(kr[u], qr, key_row(pass), sq, hd, L4, A.kq_scale);
-                if (pass + kD < passes) load_key<T, VEC>(key_row(pass + kD), hd, L4, kr[u]);
+                const float v = key_score<T, KW>(kr[u], qr, hd, A.kq_scale);
+                if (pass + kD < passes) load_key<T, KW>(key_row(pass + kD), hd, L4, kr[u]);
                 const int j = 128 * pass + jr;
                 if (L4 == 0 && j < n) {
                     ss[j] = v;

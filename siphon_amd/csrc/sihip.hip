@@ -3103,8 +3103,10 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
     const int orc = order_before(ctx, ctx->order, st);
     if (orc) return orc;
     // wide loads where rows stay aligned (and, for the streamed value rows,
-    // a workgroup's 16 rows lie within a buffer's 4 GiB)
-    const bool kvec = head_dim % 8 == 0 && (uintptr_t)k_cache % 16 == 0;
+    // a workgroup's 16 rows lie within a buffer's 4 GiB); keys and values each
+    // by their own
+    const int kw = head_dim % 8 == 0 && (uintptr_t)k_cache % 16 == 0 ? 8
+                   : head_dim % 4 == 0 && (uintptr_t)k_cache % 8 == 0 ? 4 : 1;
     const bool vvec = n_ctx % 8 == 0 && (uintptr_t)v_cache % 16 == 0 &&
                       n_ctx * 2 * kAttnPvRows <= (int64_t)UINT32_MAX;
     const bool narrow = head_dim < 160;  // key rows of at most 4 whole 32-steps
@@ -3117,15 +3119,23 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
     const int64_t fmax = ctx->opt.attn_fuse >= 0
                              ? std::min<int64_t>(ctx->opt.attn_fuse * 512, kAttnFuseCap)
                              : kAttnFuseMax;
+#define SIHIP_BY_KEYS(LAUNCH)               \
+    switch (narrow ? kw : -kw) {            \
+        case 8: { LAUNCH(4, 8) } break;     \
+        case 4: { LAUNCH(4, 4) } break;     \
+        case 1: { LAUNCH(4, 1) } break;     \
+        case -8: { LAUNCH(16, 8) } break;   \
+        case -4: { LAUNCH(16, 4) } break;   \
+        default: { LAUNCH(16, 1) } break;   \
+    }
     if (A.n <= fmax) {
         const dim3 g((unsigned)gv), t(kAttnFusedThreads);
         const size_t lds = (size_t)attn_fused_lds(A.n);
-        if (kvec && vvec && narrow)
-            hipLaunchKernelGGL((attn_fused_kernel<4, true>), g, t, lds, st, A);
-        else if (kvec && vvec)
-            hipLaunchKernelGGL((attn_fused_kernel<16, true>), g, t, lds, st, A);
-        else
-            hipLaunchKernelGGL((attn_fused_kernel<16, false>), g, t, lds, st, A);
+#define SIHIP_AF(T, W)                                                                               \
+    if (vvec) hipLaunchKernelGGL((attn_fused_kernel<T, W, true>), g, t, lds, st, A);                 \
+    else hipLaunchKernelGGL((attn_fused_kernel<T, W, false>), g, t, lds, st, A);
+        SIHIP_BY_KEYS(SIHIP_AF)
+#undef SIHIP_AF
     } else {
         const dim3 t(256);
         auto rows = [&](int64_t blocks) {
@@ -3133,12 +3143,9 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
             return dim3((unsigned)A.gx, (unsigned)((blocks + A.gx - 1) / A.gx));
         };
         const dim3 g = rows(gs);
-        if (kvec && narrow)
-            hipLaunchKernelGGL((attn_scores_kernel<4, true>), g, t, 0, st, A);
-        else if (kvec)
-            hipLaunchKernelGGL((attn_scores_kernel<16, true>), g, t, 0, st, A);
-        else
-            hipLaunchKernelGGL((attn_scores_kernel<16, false>), g, t, 0, st, A);
+#define SIHIP_AS(T, W) hipLaunchKernelGGL((attn_scores_kernel<T, W>), g, t, 0, st, A);
+        SIHIP_BY_KEYS(SIHIP_AS)
+#undef SIHIP_AS
         const dim3 eg = rows(ge);
         hipLaunchKernelGGL(attn_exp_kernel, eg, t, 0, st, A);
         if (vvec)
@@ -3146,6 +3153,7 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
         else
             hipLaunchKernelGGL(attn_pv_kernel<false>, dim3((unsigned)gv), t, 0, st, A);
     }
+#undef SIHIP_BY_KEYS
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "attention launch: %s", hipGetErrorString(e));
     return order_after(ctx, ctx->order, st);

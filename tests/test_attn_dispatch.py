@@ -34,3 +34,20 @@ def test_any_number_of_blocks_has_a_grid(n_head, n_kv, n):
 
 def test_refuses_more_positions_than_it_indexes():
     assert "positions" in launches(1, 1, 8, (1 << 29) + 1)
+
+
+@pytest.mark.parametrize("hd,n_ctx,k_offset,want", [
+    (128, 512, 0, "4,8,true"),
+    (128, 515, 0, "4,8,false"),  # value rows at any alignment, key rows still by 16 bytes
+    (128, 512, 8, "4,4,true"),
+    (128, 512, 2, "4,1,true"),
+    (100, 512, 0, "4,4,true"),
+    (66, 515, 0, "4,1,false"),
+    (300, 512, 0, "16,4,true"),
+])
+def test_keys_and_values_load_by_their_own_alignment(hd, n_ctx, k_offset, want):
+    got = launches(8, 8, hd, 300, n_ctx, k_offset)
+    assert [k for k, *_ in got] == [f"attn_fused_kernel<{want}>"]
+    got = launches(8, 8, hd, 1300, n_ctx + 1024, k_offset)
+    keys, values = want.rsplit(",", 1)
+    assert [k for k, *_ in got] == [f"attn_scores_kernel<{keys}>", "attn_exp_kernel", f"attn_pv_kernel<{values}>"]
