@@ -3,9 +3,9 @@
 // f16 dot (kernels_avx2.c:118-148), softmax (kernels.c:855-885) and the
 // softmax's exp polynomial (kernels.c:820-850).
 //
-// Up to kAttnFuseMax positions one launch, attn_fused_kernel: a workgroup per
-// query head and 16 value rows scores every position itself. Beyond, three
-// launches on one stream:
+// Up to about a thousand positions (the host's rule) one launch,
+// attn_fused_kernel: a workgroup per query head and a few blocks of 16 value
+// rows scores every position itself. Beyond, three launches on one stream:
 //   attn_scores_kernel   s[h][j] = dot(K[hk][j], f16(q_h)) * kq_scale, and the
 //                        maximum of each block of positions
 //   attn_exp_kernel      e[h][j] = exp(s[h][j] - max), and each block's total
@@ -56,6 +56,7 @@ struct AttnArgs {
     int n, hd, gqa, n_kv;
     int nbs, nbe;
     int gx;                // blocks per row of the grid (attn_block)
+    int rb;                // 16-row blocks of values per workgroup of the single launch
     float kq_scale;
 };
 
@@ -222,9 +223,11 @@ __device__ inline void load_key(const uint16_t *row, int hd, int L, KeyRow<T> &k
 
 // The scaled score of the quad's row against the f16 query (q: the lane's
 // elements of it, as load_key lays them out; in its tail anything past hd);
-// valid in the quad's lane 0. Every lane of the wave takes part.
-template <int T, int W>
-__device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, int hd, float kq_scale) {
+// valid in the quad's lane 0. Every lane of the wave takes part. NEXT: the row
+// `next` is loaded into k, each piece as soon as it is used.
+template <int T, int W, bool NEXT = false>
+__device__ inline float key_score(KeyRow<T> &k, const KeyRow<T> &q, int hd, float kq_scale,
+                                  const uint16_t *next = nullptr, int L = 0) {
     const int steps = hd >> 5;
     float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -234,6 +237,7 @@ __device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, int hd
             const h8_t qq = __builtin_bit_cast(h8_t, q.w[t]);
 #pragma unroll
             for (int e = 0; e < 8; e++) acc[e] = __builtin_fmaf((float)kk[e], (float)qq[e], acc[e]);
+            if constexpr (NEXT) k.w[t] = load_key8<W>(next + 32 * t + 8 * L, 8);
         }
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[e] = acc[e] + from_lane_up<2>(acc[e]);  // r0 + r2, r1 + r3
@@ -251,6 +255,8 @@ __device__ inline float key_score(const KeyRow<T> &k, const KeyRow<T> &q, int hd
         float pr[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) pr[e] = (float)kk[e] * (float)qq[e];
+        if constexpr (NEXT)
+            if (8 * L < (hd & 31)) k.tail = load_key8<W>(next + 32 * steps + 8 * L, (hd & 31) - 8 * L);
         auto add = [&](auto from, int cnt) {
 #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -649,19 +655,20 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
 
 // ---- one launch -------------------------------------------------------------------
 //
-// Grid ceil(hd / 16) x n_head in one dimension (attn_wg), 8 waves: a
+// Grid ceil(row blocks / rb) x n_head in one dimension (attn_wg), 8 waves: a
 // workgroup scores all n positions of its query head (16 rows per wave and
-// pass, the next pass's key rows in flight), runs the softmax in LDS
-// and the chains of its 16 value rows, one accumulator per thread. Every
-// workgroup of a head repeats the scores (hd / 16 times the score work, n *
-// hd * 2 bytes from the L2 each), which costs less than the launches and
-// round trips through memory that it saves until the rows grow long (8B
-// shape, per layer: n = 600 15.5 -> 8.6 us against a scores launch and a value
-// launch with the softmax in it). What bounds it: 6 us at n = 16, the chain of
-// one launch's start, the key and query loads, three barriers and the store.
+// pass, the next pass's key rows in flight), runs the softmax in LDS and the
+// chains of its rb blocks of 16 value rows, one block after another, one
+// accumulator per thread. Every workgroup of a head repeats the scores (n * hd *
+// 2 bytes from the L2 each), which costs less than the launches and round trips
+// through memory that it saves until the rows grow long (8B shape, per layer:
+// n = 600 15.5 -> 8.5 us against a scores launch and a value launch with the
+// softmax in it) or the workgroups many: the host chooses rb for one workgroup
+// per CU. What bounds it: 6 us at n = 16, the chain of one launch's start, the
+// key and query loads, three barriers and the store; about 1.5 us for each
+// further block, a round trip for its value rows.
 // LDS (dynamic, attn_fused_lds): scores, probabilities, value rows, query.
 constexpr int kAttnFusedThreads = 512;
-constexpr int kAttnFuseMax = 1024;
 constexpr int kAttnFuseCap = 1536;  // the largest the kernel takes (64 KiB of LDS)
 
 __host__ __device__ inline int attn_fused_np(int n) { return (n + 31) / 32 * 32; }
@@ -693,7 +700,9 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
         return kb + (int64_t)(j < n ? j : n - 1) * hd;
     };
     const int passes = (n + 127) / 128;
-    constexpr int kD = T <= 4 ? 2 : 1;  // passes of key rows held
+    // passes of key rows held; with one, a pass's row is replaced piece by
+    // piece (8 heads of 512 at n = 800: 14.3 us against 15.9 loaded after it)
+    constexpr int kD = T <= 8 ? 2 : 1;
     KeyRow<T> kr[kD];
     load_key<T, KW>(key_row(0), hd, L4, kr[0]);
     float qv = 0.0f;
@@ -701,20 +710,37 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
 #pragma unroll
     for (int i = 1; i < kD; i++)
         if (i < passes) load_key<T, KW>(key_row(i), hd, L4, kr[i]);
-    // value rows: 32 lanes per row; rows past hd repeat the last, positions
-    // past n are not used
+    // value rows, a block of 16 after another: 32 lanes per row; rows past hd
+    // repeat the last, positions past n are not used
     const int r = tid >> 5, a = tid & 31;
-    const int c = W.blk * kAttnPvRows + r;
-    const uint16_t *const vrow = A.v + ((int64_t)W.hk * hd + min(c, hd - 1)) * A.n_ctx;
+    const int b1 = min((W.blk + 1) * A.rb, (hd + kAttnPvRows - 1) / kAttnPvRows);
     constexpr int kVP = kAttnFuseCap / 256;
     const int per8 = (n + 7) / 8;
     uint4 vq[kVP];
-    if constexpr (VEC) {
+    uint8_t *const svr = sv + r * vslot;
+    auto value_row = [&](int b) {
+        return A.v + ((int64_t)W.hk * hd + min(b * kAttnPvRows + r, hd - 1)) * A.n_ctx;
+    };
+    auto load_v = [&](int b) {
+        if constexpr (VEC) {
+            const uint4 *const p = reinterpret_cast<const uint4 *>(value_row(b));
 #pragma unroll
-        for (int i = 0; i < kVP; i++)
-            vq[i] = 32 * i < per8 ? reinterpret_cast<const uint4 *>(vrow)[min(32 * i + a, per8 - 1)]
-                                  : make_uint4(0, 0, 0, 0);
-    }
+            for (int i = 0; i < kVP; i++) vq[i] = 32 * i < per8 ? p[min(32 * i + a, per8 - 1)] : make_uint4(0, 0, 0, 0);
+        }
+    };
+    // block b (VEC: loaded before) to LDS: its row's lanes alone read it
+    auto put_v = [&](int b) {
+        if constexpr (VEC) {
+#pragma unroll
+            for (int i = 0; i < kVP; i++)
+                if (32 * i + a < per8) *reinterpret_cast<uint4 *>(svr + (32 * i + a) * 16) = vq[i];
+        } else {
+            const uint16_t *const p = value_row(b);
+            for (int i = a; i < n; i += 32) reinterpret_cast<uint16_t *>(svr)[i] = p[i];
+        }
+    };
+    int b = W.blk * A.rb;
+    load_v(b);
     if (tid < hd) sq[tid] = (uint16_t)f32_to_f16_hw(qv);
     __syncthreads();
     KeyRow<T> qr;
@@ -725,8 +751,9 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
         for (int u = 0; u < kD; u++) {
             const int pass = p0 + u;
             if (pass < passes) {
-                const float v = key_score<T, KW>(kr[u], qr, hd, A.kq_scale);
-                if (pass + kD < passes) load_key<T, KW>(key_row(pass + kD), hd, L4, kr[u]);
+                const uint16_t *const next = key_row(min(pass + kD, passes - 1));
+                const float v = key_score<T, KW, kD == 1>(kr[u], qr, hd, A.kq_scale, next, L4);
+                if (kD > 1 && pass + kD < passes) load_key<T, KW>(next, hd, L4, kr[u]);
                 const int j = 128 * pass + jr;
                 if (L4 == 0 && j < n) {
                     ss[j] = v;
@@ -736,13 +763,8 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
             }
         }
     }
-    if constexpr (VEC) {
-#pragma unroll
-        for (int i = 0; i < kVP; i++)
-            if (32 * i + a < per8) *reinterpret_cast<uint4 *>(sv + r * vslot + (32 * i + a) * 16) = vq[i];
-    } else {
-        for (int i = a; i < n; i += 32) reinterpret_cast<uint16_t *>(sv + r * vslot)[i] = vrow[i];
-    }
+    put_v(b);
+    if (b + 1 < b1) load_v(b + 1);
     mx = wave_max(mx);
     if (lane == 0) redf[wave] = mx;
     __syncthreads();
@@ -785,13 +807,24 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
         out_p(jt, p);
     }
     __syncthreads();
-    const uint16_t *const vs = reinterpret_cast<const uint16_t *>(sv + r * vslot);
+    const uint16_t *const vs = reinterpret_cast<const uint16_t *>(svr);
     const int body = n & ~31;
-    float acc = 0.0f;
+    for (;;) {
+        float acc = 0.0f;
 #pragma unroll 8
-    for (int i = a; i < body; i += 32) acc = __builtin_fmaf(f16_bits_to_f32(vs[i]), f16_bits_to_f32(sp[i]), acc);
-    const float res = row_tree1(acc);
-    if (a == 0 && c < hd) A.out[(int64_t)W.h * hd + c] = add_tail<true>(res, vs + body, sp + body, n - body);
+        for (int i = a; i < body; i += 32)
+            acc = __builtin_fmaf(f16_bits_to_f32(vs[i]), f16_bits_to_f32(sp[i]), acc);
+        const float res = row_tree1(acc);
+        const int c = b * kAttnPvRows + r;
+        // (opaque, or the tail's 31 conditions are kept across the blocks in
+        // scalar registers that spill)
+        int cnt = n - body;
+        asm volatile("" : "+s"(cnt));
+        if (a == 0 && c < hd) A.out[(int64_t)W.h * hd + c] = add_tail<true>(res, vs + body, sp + body, cnt);
+        if (++b >= b1) break;
+        put_v(b);
+        if (b + 1 < b1) load_v(b + 1);
+    }
 }
 
 }  // namespace sihip

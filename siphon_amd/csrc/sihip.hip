@@ -57,7 +57,7 @@ struct Options {
     int64_t gemmq_xmode = -1;  // Q8_0-pair GEMM record mode 0 or 1 (gemmq_kernel XM; rule: 1 where it fits)
     int64_t gemmq_fuse = -1;   // Q8_0-pair GEMM quantizing X itself (XM 2) at 16-row m blocks, 0: off (rule: on)
     int64_t gemmh_fuse = -1;   // F16 GEMM converting X itself (XF) at 16-row m blocks, 0: off (rule: on)
-    int64_t attn_fuse = -1;    // decode attention in one launch up to 512 k positions, 0: three (rule: kAttnFuseMax)
+    int64_t attn_fuse = -1;    // decode attention in one launch up to 512 k positions, at most kAttnFuseCap, 0: three (rule: attn_fuse_max)
     int64_t gemm2s_max_m = -1; // largest M on the small-M Q4_K GEMM, 0: none (rule: 16)
     int64_t gemmks_max_m = -1; // largest M on the small-M K-quant GEMM, 0: none (rule: 16)
     int64_t gemmks_q4k = -1;   // Q4_K small M on gemmks.h (1) or gemm2s.h (0) (rule: 0)
@@ -3046,6 +3046,26 @@ extern "C" int sihip_gemm_dev_noalloc(sihip_ctx *ctx, const sihip_weight *w, con
     return launch_gemm_mfma(ctx, w, p, B, X, w->L.n_in, M, Y, w->L.n_out, st);
 }
 
+// Positions up to which the decode attention is one launch (the ATTN_FUSE
+// option k: 512 k, 0: never). us per layer, one against three launches:
+//   head_dim < 160: 32 heads of 128 at 600 8.5 / 12.8, 1025 10.8 / 13.1, 1500
+//     12.7 / 13.3; 128 heads 1025 16.0 / 18.9; 24 of 80 1200 13.1 / 13.1
+//   160 to 223: 16 of 192 at 1000 11.7 / 12.1, 1200 13.1 / 12.7
+//   wider: 16 of 256 at 700 11.4 / 11.6, 900 13.1 / 11.8; 8 of 256 900 12.3 /
+//     12.5; 8 of 512 800 14.3 / 14.9, 900 17.5 / 17.1
+//   pv_twice, the value launch needs a second round of the CUs: 32 of 288 at
+//     1025 17.8 / 19.7
+//   keys by single elements: 32 of 66 at 1024 11.0 / 11.3, 1300 15.4 / 14.1; 16
+//     of 330 at 600 21.0 / 19.0
+//   value rows by single elements, copied once per block: 32 of 128 at 1000
+//     11.4 / 12.8, 64 (two blocks) 600 11.2 / 12.8 and 1000 14.6 / 13.4
+static int64_t attn_fuse_max(int64_t head_dim, int kw, bool vvec, int rb, bool pv_twice) {
+    int64_t m = head_dim < 160 || pv_twice ? 1200 : head_dim < 224 ? 1024 : 800;
+    if (kw == 1) m = std::min<int64_t>(m, head_dim < 160 ? 1024 : head_dim < 288 ? 600 : 400);
+    if (!vvec) m = std::min<int64_t>(m, rb == 1 ? 1000 : 600);
+    return m;
+}
+
 extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint16_t *k_cache,
                                      const uint16_t *v_cache, int64_t n_head, int64_t n_head_kv,
                                      int64_t head_dim, int64_t n_ctx, int64_t pos, float kq_scale,
@@ -3109,27 +3129,27 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
                    : head_dim % 4 == 0 && (uintptr_t)k_cache % 8 == 0 ? 4 : 1;
     const bool vvec = n_ctx % 8 == 0 && (uintptr_t)v_cache % 16 == 0 &&
                       n_ctx * 2 * kAttnPvRows <= (int64_t)UINT32_MAX;
-    const bool narrow = head_dim < 160;  // key rows of at most 4 whole 32-steps
-    // one launch up to kAttnFuseMax positions (the ATTN_FUSE option k: 512 k,
-    // 0: never). One against three launches, us per layer: 32 heads of 128
-    // over 8 KV heads, n = 600 8.6 against 13.0, 1000 11.1 against 13.8, 1300
-    // 13.3 against 14.5, 1536 12.4 against 12.3; 40 heads 1000 14.1 against
-    // 15.1, 1300 17.1 against 16.4; 16 heads of 80 1000 11.7 against 11.9,
-    // 1300 13.8 against 12.7
+    // 16-row blocks of values per workgroup of the single launch: as few as
+    // leave one workgroup per CU, since each repeats its head's scores (32
+    // heads of 128 one, 64 two, 128 four: n = 600 10.5 against 11.8 us for 64
+    // heads, 13.2 against 20.0 for 128; 32 heads of 256 two, 12.3 against 21.2)
+    A.rb = 1;
+    while (A.rb < row_blocks && (row_blocks + A.rb - 1) / A.rb * n_head > ctx->n_cu) A.rb++;
     const int64_t fmax = ctx->opt.attn_fuse >= 0
                              ? std::min<int64_t>(ctx->opt.attn_fuse * 512, kAttnFuseCap)
-                             : kAttnFuseMax;
-#define SIHIP_BY_KEYS(LAUNCH)               \
-    switch (narrow ? kw : -kw) {            \
-        case 8: { LAUNCH(4, 8) } break;     \
-        case 4: { LAUNCH(4, 4) } break;     \
-        case 1: { LAUNCH(4, 1) } break;     \
-        case -8: { LAUNCH(16, 8) } break;   \
-        case -4: { LAUNCH(16, 4) } break;   \
-        default: { LAUNCH(16, 1) } break;   \
+                             : attn_fuse_max(head_dim, kw, vvec, A.rb, gv > 2 * ctx->n_cu);
+#define SIHIP_BY_WIDTH(T, LAUNCH)           \
+    switch (kw) {                           \
+        case 8: { LAUNCH(T, 8) } break;     \
+        case 4: { LAUNCH(T, 4) } break;     \
+        default: { LAUNCH(T, 1) } break;    \
     }
+#define SIHIP_BY_KEYS(LAUNCH)                                    \
+    if (head_dim < 160) { SIHIP_BY_WIDTH(4, LAUNCH) }            \
+    else if (head_dim < 288) { SIHIP_BY_WIDTH(8, LAUNCH) }       \
+    else { SIHIP_BY_WIDTH(16, LAUNCH) }
     if (A.n <= fmax) {
-        const dim3 g((unsigned)gv), t(kAttnFusedThreads);
+        const dim3 g((unsigned)((row_blocks + A.rb - 1) / A.rb * n_head)), t(kAttnFusedThreads);
         const size_t lds = (size_t)attn_fused_lds(A.n);
 #define SIHIP_AF(T, W)                                                                               \
     if (vvec) hipLaunchKernelGGL((attn_fused_kernel<T, W, true>), g, t, lds, st, A);                 \
@@ -3154,6 +3174,7 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
             hipLaunchKernelGGL(attn_pv_kernel<false>, dim3((unsigned)gv), t, 0, st, A);
     }
 #undef SIHIP_BY_KEYS
+#undef SIHIP_BY_WIDTH
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_err(ctx, SIHIP_EDEVICE, "attention launch: %s", hipGetErrorString(e));
     return order_after(ctx, ctx->order, st);

@@ -43,6 +43,7 @@ def test_refuses_more_positions_than_it_indexes():
     (128, 512, 2, "4,1,true"),
     (100, 512, 0, "4,4,true"),
     (66, 515, 0, "4,1,false"),
+    (256, 515, 0, "8,8,false"),
     (300, 512, 0, "16,4,true"),
 ])
 def test_keys_and_values_load_by_their_own_alignment(hd, n_ctx, k_offset, want):
@@ -51,3 +52,29 @@ def test_keys_and_values_load_by_their_own_alignment(hd, n_ctx, k_offset, want):
     got = launches(8, 8, hd, 1300, n_ctx + 1024, k_offset)
     keys, values = want.rsplit(",", 1)
     assert [k for k, *_ in got] == [f"attn_scores_kernel<{keys}>", "attn_exp_kernel", f"attn_pv_kernel<{values}>"]
+
+
+@pytest.mark.parametrize("n_head,hd,workgroups", [
+    (32, 128, 256), (33, 128, 132), (64, 128, 256), (128, 128, 256), (96, 96, 192), (32, 256, 256),
+    (40, 200, 200),   # 13 blocks in fives
+    (300, 64, 300),   # never less than one a head
+    (1, 1, 1),
+])
+def test_the_single_launch_fits_the_cus(n_head, hd, workgroups):
+    """A workgroup takes as many 16-row blocks of values as leave one per CU."""
+    got = launches(n_head, n_head, hd, 100)
+    assert len(got) == 1 and got[0][1] == workgroups
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,n_ctx,one,three", [
+    (32, 8, 128, 2048, 1200, 1201),
+    (16, 8, 192, 2048, 1024, 1025),
+    (16, 16, 256, 2048, 800, 801),
+    (32, 8, 288, 2048, 1200, 1201),  # 576 value workgroups: two rounds of the CUs
+    (32, 8, 66, 2048, 1024, 1025),
+    (32, 8, 128, 2047, 1000, 1001),
+    (64, 8, 128, 2047, 600, 601),
+])
+def test_one_launch_or_three(n_head, n_kv, hd, n_ctx, one, three):
+    assert len(launches(n_head, n_kv, hd, one, n_ctx)) == 1
+    assert len(launches(n_head, n_kv, hd, three, n_ctx)) == 3

@@ -78,6 +78,21 @@ def test_any_alignment(dev, oracle, option, hd, n_ctx, n, k_shift, v_shift, fuse
             b.free()
 
 
+@pytest.mark.parametrize("n_head,n_kv,hd,n_ctx,n", [
+    (64, 8, 128, 264, 257),    # two blocks of value rows per workgroup
+    (96, 4, 96, 200, 190),     # three of six
+    (128, 128, 128, 64, 40),   # four
+    (40, 8, 200, 72, 70),      # five of thirteen: the last workgroup has three
+    (300, 100, 24, 48, 47),    # all of a head; half a block of rows
+    (64, 8, 128, 131, 131),    # value rows by elements
+    (20, 4, 512, 100, 99),     # sixteen 32-steps, three of 32 blocks
+])
+def test_row_blocks_of_the_single_launch(dev, oracle, n_head, n_kv, hd, n_ctx, n):
+    q, k, v, kq = _case(np.random.default_rng(n_head + hd), n_head, n_kv, hd, n_ctx)
+    want = oracle.attn_decode(q, k, v, n_head, n_kv, hd, n_ctx, n - 1, kq)
+    check(run_attn(dev, q, k, v, n_head, n_kv, hd, n_ctx, n - 1, kq), want, n, f"{n_head} heads hd={hd}")
+
+
 def test_more_blocks_than_one_grid_row(dev):
     """1025 heads of 2^18 positions: 4 198 400 score blocks, past the 2^22 of
     a grid row. Equal scores give probabilities of 2^-18 exactly, so each
