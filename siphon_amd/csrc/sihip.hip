@@ -2133,12 +2133,13 @@ static int launch_gemmsk_group(sihip_ctx *ctx, int count, const sihip_weight *co
         for (int i = 0; i < count; i++)
             if (w[i]->L.type == t0 || w[i]->L.type == t1) blocks += (w[i]->L.n_out + 31) / 32 * p.MB;
         // few 32-row blocks: half a block per workgroup and eight waves
-        // instead of four (M = 37: ffn_down 4096 x 14336, 128 blocks, 27.8 ->
-        // 24.5 us, 2048 x 5632, 64 blocks, 15.4 -> 12.4, 4096 x 4096 11.4 ->
-        // 10.9; q/k/v, 192 blocks, 13.4 against 16.6); the GEMMS_WAVES option
-        // 4 or 8 sets it
+        // instead of four, while these workgroups, one per CU, fit one round
+        // (five formats, rows of 2048 to 14336: 112 to 128 blocks 0.8 to 1.0
+        // of the time, 140 to 256 blocks 1.1 to 1.5 times it; M = 37: 4096 x
+        // 14336, 128 blocks, 27.8 -> 24.5 us, 2048 x 5632 15.4 -> 12.4); the
+        // GEMMS_WAVES option 4 or 8 sets it
         const int64_t ow = ctx->opt.gemms_waves;
-        const bool narrow = ow == 4 || ow == 8 ? ow == 8 : 8 * blocks <= 5 * (int64_t)ctx->n_cu;
+        const bool narrow = ow == 4 || ow == 8 ? ow == 8 : 2 * blocks <= (int64_t)ctx->n_cu;
         const int rows = narrow ? 16 : 32;
         int64_t wg = 0;
         for (int i = 0; i < count; i++) {

@@ -61,3 +61,19 @@ def test_noalloc_after_a_short_prompt(wt, n_out, n_in, M, launches):
         result = [k[0] for k in launched() if "quantize" not in k[0]]
     """)
     assert len(got) == launches and all(k.startswith(("gemmsk", "gemmx", "gemm6", "gemm_kq")) for k in got), got
+
+
+@pytest.mark.parametrize("n_out,M,waves,grid", [
+    (4096, 48, 8, 256), (4128, 48, 4, 136), (5120, 9, 4, 160), (2048, 96, 8, 256), (2080, 96, 4, 144),
+])
+def test_short_prompts_fit_one_round(n_out, M, waves, grid):
+    """Workgroups of eight waves only where each has a CU of its own."""
+    got = fake_hip.run(f"""
+        w = upload(sa.Q4_K, {n_out}, 1024)
+        w.prepare_gemm()
+        fake.fake_reset(0)
+        dev.set_option("GEMMSK_MAX_M", 1000)
+        dev.gemm_dev(w, X, {M}, X)
+        result = launched()[-1]
+    """)
+    assert got[0].startswith("gemmsk_kernel") and got[0].endswith(f",{waves}>") and got[1] == grid, got
