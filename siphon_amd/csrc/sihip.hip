@@ -1193,6 +1193,7 @@ struct GemmPlan {
     int64_t steps;     // K steps of a tile: super-blocks, or 128-element
                        // steps for the F16 and Q8_0-pair kernels
     int64_t part_bytes;
+    double cost = 0.0;   // plan_tiles: its estimate, in the units of its TileCost
     bool fuseq = false;  // a GEMM that quantizes or converts X itself (gemmq_kernel XM 2,
                          // gemmh_f16_kernel XF)
 };
@@ -2057,6 +2058,10 @@ static SKPlan plan_gemmsk(int64_t M, int64_t nb) {
     return p;
 }
 
+// The GEMM that a single matrix takes by the built-in rule.
+enum class OnGemm { kShort, kRing, kOlder };  // gemmsk.h, gemmx.h / gemmd.h, the plan of plan_gemm
+static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M);
+
 // Whether an option puts M rows of a K-quant on one of the other GEMMs
 // (GEMMKS_MAX_M, GEMM2S_MAX_M, GEMM2_MIN_M, GEMM6_MIN_M): what it names keeps
 // its range, and gemmsk.h and gemmx.h, by their built-in rules, the rest.
@@ -2088,6 +2093,7 @@ static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight 
     }
     if (here != other && (noalloc || capturing(st))) return here;
     if (ctx->opt.gemmsk_max_m >= 0) return M <= ctx->opt.gemmsk_max_m;
+    if (count == 1) return single_kquant(ctx, w[0]->L, M) == OnGemm::kShort;
     int64_t blocks = 0;
     for (int i = 0; i < count; i++) blocks += (w[i]->L.n_out + 31) / 32;
     return M <= kGemmSKMaxM || (M < kGemm2MinM && blocks * ((M + 15) / 16) <= kGemmSKTiles &&
@@ -2239,7 +2245,7 @@ static GemmPlan plan_tiles(const sihip_ctx *ctx, int64_t M, int64_t steps, int64
             const double cost = C.share((wgs + ctx->n_cu - 1) / ctx->n_cu) * sbk * (C.fixed + C.per_tile * mt) +
                                 (S > 1 ? C.slice : 0.0) + C.byte * part;
             if (best >= 0.0 && cost >= best) continue;
-            best = cost;
+            best = p.cost = cost;
             p.mt = mt;
             p.S = (int)((steps + sbk - 1) / sbk);
             p.SBK = (int)sbk;
@@ -2276,23 +2282,90 @@ static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *
     }
     if (here != other && (noalloc || capturing(st))) return here;
     if (ctx->opt.gemmx_min_m > 0) return M >= ctx->opt.gemmx_min_m;
+    if (count == 1) return single_kquant(ctx, w[0]->L, M) == OnGemm::kRing;
     // Q4_K from M = kGemm2MinM runs on gemm2.h, whose copy holds the scales
     // and mins split beforehand (8B gate + up at M = 2048 502 us against 520
-    // here, wo at M = 512 33.5 against 38.1); other types' single matrices of
-    // few rows on the kernels whose m tiles need fewer K slices and, for
-    // Q6_K, no decode (M = 512, wo: Q6_K 33.3 against 50.8, Q3_K 32.4 against
-    // 41.7, Q2_K 30.1 against 32.9; M = 2048: 90.6 / 81.0 / 72.3 against 93.4
-    // / 71.7 / 68.9). Everything else is faster here (M = 512, 8B gate + up:
-    // Q5_K 264 -> 162 us, Q3_K 142 -> 116, Q6_K 179 -> 159).
+    // here). Everything else is faster here (M = 512, 8B gate + up: Q5_K 264 ->
+    // 162 us, Q3_K 142 -> 116, Q6_K 179 -> 159).
     // (A Q6_K matrix beside Q4_K ones there keeps the launch, and the bits, of
     // a call of its own.)
-    const uint32_t t = w[0]->L.type;
     for (int i = 0; i < count; i++)
         if (w[i]->L.type == T_Q4_K && M >= gemm2_min_m(ctx->opt)) return false;
-    if (count == 1 && w[0]->L.n_out <= 8192 && M >= 128 &&
-        (t == T_Q6_K || ((t == T_Q2_K || t == T_Q3_K) && M < 1024)))
-        return false;
     return true;
+}
+
+// ---- single matrices -----------------------------------------------------------
+//
+// A group shares its launches and one record, so it is faster on the kernels of
+// this section at nearly every size. A single matrix (the engine's prompt is one
+// call per matrix) gains less, and where its workgroups on one kernel fill their
+// last round of the CUs and on the other do not, that decides. So the kernels'
+// times are estimated, in us: a launch's start, and steps times rounds times what
+// a step takes by format, from timings of 20 shapes (256 to 128256 rows of 896 to
+// 28672 elements) at 9 to 700 activation rows: within 5% at the median, 10 to 15
+// at nine tenths. The older kernel is taken unless it is estimated slower by the
+// margins below: of 2500 K-quant timings 254 were slower than on the kernels
+// before, by up to 1.5 times, under a rule by M and n_out, 8 with this.
+
+// Rounds of w workgroups of which a CU runs two at a time, one alone taking `one`
+// of the time of two.
+static double rounds2(int64_t w, int64_t n_cu, double one) {
+    const int64_t k = (w + n_cu - 1) / n_cu;
+    return (double)(k / 2) + (k % 2 ? one : 0.0);
+}
+
+// us per super-block: gemmsk.h (of one of four waves; its decode, and each of mt
+// tiles), gemmx.h per unit of its plan's cost, and the older kernel with 16-,
+// 32- and 64-row m blocks.
+struct KQuantStep {
+    double decode, tile, ring, older[3];
+};
+static KQuantStep kquant_step(uint32_t type) {
+    switch (type) {
+        case T_Q2_K: return {0.39, 0.51, 0.151, {1.00, 1.00, 1.36}};
+        case T_Q3_K: return {1.07, 0.34, 0.176, {1.25, 1.25, 1.56}};
+        case T_Q4_K: return {0.72, 0.49, 0.194, {1.39, 1.39, 1.93}};
+        case T_Q5_K: return {1.17, 0.48, 0.222, {1.77, 1.77, 1.77}};
+        default: return {1.84, 0.30, 0.234, {1.27, 2.05, 2.17}};
+    }
+}
+
+static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M) {
+    const int64_t nb = L.n_in / 256;
+    // Q4_K from kGemm2MinM rows on gemm2.h (4096 x 4096 at M = 512 33.5 us
+    // against 38.1 here), and up to 16 with long rows on gemm2s.h (4096 x 14336
+    // 13.7 against 15.0, 4096 x 11008 1.12 times)
+    if (L.type == T_Q4_K && (M >= gemm2_min_m(ctx->opt) || (M <= 16 && L.n_in > kGemmSKMaxK)))
+        return OnGemm::kOlder;
+    // few rows of output, from kGemm2MinM: kernels whose m tiles need fewer K
+    // slices and, for Q6_K, no decode (4096 x 4096 at M = 512: Q6_K 33.3 against
+    // 50.8, Q3_K 32.4 against 41.7; at M = 2048 90.6 / 81.0 against 93.4 / 71.7)
+    if (M >= kGemm2MinM && L.n_out <= 8192 &&
+        (L.type == T_Q6_K || ((L.type == T_Q2_K || L.type == T_Q3_K) && M < 1024)))
+        return OnGemm::kOlder;
+    const KQuantStep c = kquant_step(L.type);
+    double sk = 1e30;
+    if (M < kGemm2MinM) {
+        const SKPlan q = plan_gemmsk(M, nb);
+        const int64_t blocks = (L.n_out + 31) / 32 * q.MB;
+        if (2 * blocks <= ctx->n_cu)  // eight waves: the same work in half as long a chain
+            sk = 6.3 + (double)((nb + 7) / 8) * (0.4 * c.decode + 0.9 * c.tile * q.mt);
+        else
+            sk = 6.3 + (double)((nb + 3) / 4) * (c.decode + c.tile * q.mt) * rounds2(blocks, ctx->n_cu, 0.55);
+    }
+    const GemmPlan x = plan_gemmx(ctx, M, nb, (L.n_out + kG2BN - 1) / kG2BN);
+    const double ring = 8.8 + c.ring * x.cost;
+    const OnGemm newer = sk <= ring ? OnGemm::kShort : OnGemm::kRing;
+    if (M < 17) return newer;
+    const GemmPlan p = plan_gemm(ctx, L, M);
+    const int64_t bm = p.v2 ? 16 * p.mt : 32 * p.mt;
+    const double start = L.type == T_Q6_K ? 5.8 : bm == 32 ? 8.7 : 11.6;
+    const double older = start + c.older[bm == 16 ? 0 : bm == 32 ? 1 : 2] * p.SBK *
+                                     rounds2(p.Mp / bm * ((L.n_out + kG2BN - 1) / kG2BN) * p.S, ctx->n_cu, 0.8) +
+                         0.5e-6 * (double)p.part_bytes;
+    // (Q6_K up to 96 rows: the estimate of the older kernel's K slices is low)
+    const double margin = L.type != T_Q6_K ? 1.08 : M <= 96 ? 0.80 : 1.12;
+    return older < margin * std::min(sk, ring) ? OnGemm::kOlder : newer;
 }
 
 template <int MT>

@@ -77,3 +77,24 @@ def test_short_prompts_fit_one_round(n_out, M, waves, grid):
         result = launched()[-1]
     """)
     assert got[0].startswith("gemmsk_kernel") and got[0].endswith(f",{waves}>") and got[1] == grid, got
+
+
+@pytest.mark.parametrize("wt,n_out,n_in,want", [
+    # timed faster there by 5% and more
+    ("Q6_K", 14336, 4096, {64: "gemmsk", 112: "gemm6_q6k", 256: "gemm6_q6k", 512: "gemm6_q6k"}),
+    ("Q6_K", 4096, 4096, {96: "gemmsk", 300: "gemm6_q6k"}),
+    ("Q4_K", 14336, 4096, {64: "gemmsk", 112: "gemm_kq", 224: "gemm_kq", 300: "gemmx"}),
+    ("Q4_K", 4096, 14336, {16: "gemm2s_q4k", 32: "gemmsk", 340: "gemmx"}),
+    ("Q5_K", 14336, 4096, {112: "gemm_kq", 144: "gemmsk", 300: "gemmx"}),
+    ("Q2_K", 32000, 2048, {48: "gemmsk", 64: "gemm_kq"}),
+    ("Q2_K", 1024, 4096, {9: "gemmsk", 300: "gemmsk"}),
+])
+def test_single_matrices(wt, n_out, n_in, want):
+    """A call of one matrix takes the kernel that is the faster for it."""
+    got = gemms({}, [wt], n_out, n_in, list(want))
+    assert {M: v[0].split("_kernel")[0] for M, v in got.items()} == want
+
+
+def test_a_group_keeps_the_newer_kernels():
+    got = gemms({}, ["Q6_K", "Q6_K"], 14336, 4096, [112, 256])
+    assert {M: v[0].split("_kernel")[0] for M, v in got.items()} == {112: "gemmsk", 256: "gemmx"}
