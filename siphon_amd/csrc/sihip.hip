@@ -2549,6 +2549,38 @@ static GemmPlan plan_gemmd(const sihip_ctx *ctx, int count, const sihip_weight *
     return p;
 }
 
+// A single matrix of these formats, as single_kquant: by the kernels' estimated
+// times (2072 timings at 17 to 700 rows; of those from 100 rows 305 were slower
+// than on the kernels before under a rule by M and n_out, by up to 1.5 times, 21
+// with this). us per step of 128 elements; plan_tiles' costs in their units.
+static OnGemm single_dense(const sihip_ctx *ctx, const sihip_weight *w, int64_t M) {
+    const Layout &L = w->L;
+    const bool f16 = L.type == T_F16, q8 = L.type == T_Q8_0;
+    const GemmPlan d = plan_gemmd(ctx, 1, &w, M);
+    double newer;
+    if (d.small) {
+        const double steps = (double)((d.steps + kGDSWaves - 1) / kGDSWaves);
+        newer = (f16 ? 6.1 : 7.8) + steps * (f16 ? 0.10 + 0.29 * d.mt : q8 ? 0.20 + 0.59 * d.mt : 0.14 + 0.40 * d.mt);
+    } else {
+        newer = f16 ? 7.9 + 0.063 * d.cost : q8 ? 10.4 + 0.164 * d.cost : 9.6 + 0.187 * d.cost;
+    }
+    // the older kernel by its 16-, 32-, 64- or 128-row m blocks: start, step, and
+    // a megabyte of partial sums
+    struct Older { double start, step, part; };
+    static const Older of16[4] = {{3.5, 0.46, 3.1}, {4.9, 0.59, 0.87}, {5.9, 0.71, 0.62}, {4.9, 2.01, 0.55}};
+    static const Older oq8[3] = {{6.9, 1.36, 0.68}, {7.6, 1.41, 0.74}, {10.2, 2.36, 0.34}};
+    static const Older oq[3] = {{7.2, 1.10, 0.65}, {9.5, 1.04, 0.65}, {10.8, 2.60, 0.26}};
+    const GemmPlan p = plan_gemm(ctx, L, M);
+    const int i = p.mt >= 8 ? 3 : p.mt >= 4 ? 2 : p.mt - 1;
+    const Older &o = f16 ? of16[i] : q8 ? oq8[i] : oq[i];
+    const int64_t wgs = p.Mp / (16 * p.mt) * ((L.n_out + kG2BN - 1) / kG2BN) * p.S;
+    const int64_t k = (wgs + ctx->n_cu - 1) / ctx->n_cu;
+    const double rounds = f16 ? (i == 3 ? rounds2(wgs, ctx->n_cu, 0.8) : (double)k)
+                              : k == 1 ? 0.6 : k == 2 ? 0.8 : (double)k / 3.0;
+    const double older = o.start + o.step * p.SBK * rounds + o.part * 1e-6 * (double)p.part_bytes;
+    return newer < 0.94 * older ? OnGemm::kRing : OnGemm::kOlder;
+}
+
 // Whether weights over one X take this launch: one format of these, unless an
 // option sets the tiling of the other kernels.
 static bool gemmd_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M) {
@@ -2570,11 +2602,10 @@ static bool gemmd_eligible(const sihip_ctx *ctx, int count, const sihip_weight *
     // 522 us there against 554, ffn_down 269 against 307; 1.1B gate + up at
     // M = 1500, 8448 each: 119 against 94 here, 8B at M = 300, 10752: 143
     // against 110)
-    if (L.type == T_F16)
-        return gemm_blocks(count, w) * ((M + 127) / 128) * (L.n_in / 128) < (int64_t)32768 * count;
-    // a single Q8_0-pair matrix of few rows from 512: no faster here (2048 x
-    // 2048 at M = 600: Q4_0 29.4 us there, 33.0 here; M = 500: 27.9 and 21.1)
-    return count > 1 || M <= 512 || L.n_out >= 4096;
+    if (L.type == T_F16 &&
+        gemm_blocks(count, w) * ((M + 127) / 128) * (L.n_in / 128) >= (int64_t)32768 * count)
+        return false;
+    return count > 1 || single_dense(ctx, w[0], M) == OnGemm::kRing;
 }
 
 template <uint32_t FMT, int BM>

@@ -88,6 +88,13 @@ def test_short_prompts_fit_one_round(n_out, M, waves, grid):
     ("Q5_K", 14336, 4096, {112: "gemm_kq", 144: "gemmsk", 300: "gemmx"}),
     ("Q2_K", 32000, 2048, {48: "gemmsk", 64: "gemm_kq"}),
     ("Q2_K", 1024, 4096, {9: "gemmsk", 300: "gemmsk"}),
+    ("Q8_0", 256, 2048, {128: "gemmq", 200: "gemmq"}),
+    ("Q8_0", 4096, 4096, {128: "gemmq", 144: "gemmd", 600: "gemmq"}),
+    ("Q4_0", 1024, 4096, {129: "gemmq", 383: "gemmq"}),
+    ("Q5_0", 4096, 4096, {160: "gemmd", 512: "gemmq"}),
+    ("F16", 896, 896, {200: "gemmh_f16"}),
+    ("F16", 5632, 2048, {144: "gemmd", 300: "gemmd"}),
+    ("F16", 27648, 5120, {256: "gemmh_f16"}),
 ])
 def test_single_matrices(wt, n_out, n_in, want):
     """A call of one matrix takes the kernel that is the faster for it."""
@@ -98,3 +105,5 @@ def test_single_matrices(wt, n_out, n_in, want):
 def test_a_group_keeps_the_newer_kernels():
     got = gemms({}, ["Q6_K", "Q6_K"], 14336, 4096, [112, 256])
     assert {M: v[0].split("_kernel")[0] for M, v in got.items()} == {112: "gemmsk", 256: "gemmx"}
+    got = gemms({}, ["Q8_0"] * 3, 256, 2048, [17, 200])
+    assert all(v[0].startswith("gemmd") and len(v) == 1 for v in got.values())
