@@ -67,6 +67,8 @@ struct Options {
     int64_t gemmsk_max_m = -1; // largest M on the short-prompt K-quant GEMM, 0: none (rule: kGemmSKMaxM)
     int64_t gemmd_min_m = -1;  // smallest M on the F16 and Q8_0-pair GEMM of prompts, 0: never (rule: kGemmDMinM)
     int64_t gemmx_min_m = -1;  // smallest M on the K-quant GEMM of longer prompts, 0: never (rule: past GEMMSK_MAX_M)
+    int64_t ring_mt = -1;      // m tiles of the ring-buffered GEMMs (gemmx.h, gemmd.h), where they have that instance (rule: plan_tiles)
+    int64_t ring_sbk = -1;     // their K-slice length in steps, 0: none (rule: plan_tiles)
     int64_t gemm_group = -1;   // Q4_K matrices over one X in one 16x16 GEMM launch, 0: off (rule: on)
     int64_t q80_scalar = -1;   // Q8_0 activations by the scalar quantizer (reference
                                // kernels.c:542-558, its SI_SCALAR mode), 1: on (rule: off)
@@ -93,6 +95,7 @@ static const OptionName kOptionNames[] = {
     {"GEMMKF_MAX_M", &Options::gemmkf_max_m}, {"GEMMKF_SBK", &Options::gemmkf_sbk},
     {"GEMM_GROUP", &Options::gemm_group}, {"GEMMSK_MAX_M", &Options::gemmsk_max_m},
     {"GEMMX_MIN_M", &Options::gemmx_min_m}, {"GEMMD_MIN_M", &Options::gemmd_min_m},
+    {"RING_MT", &Options::ring_mt},       {"RING_SBK", &Options::ring_sbk},
 };
 
 // Order of launches that share mutable device state across streams: a
@@ -2233,14 +2236,26 @@ static GemmPlan plan_tiles(const sihip_ctx *ctx, int64_t M, int64_t steps, int64
     p.v2 = true;
     p.steps = steps;
     double best = -1.0;
+    // the options RING_MT, where there is that instance, and RING_SBK, where the
+    // partial sums keep 32-bit offsets
+    const int64_t omt = ctx->opt.ring_mt, osbk = ctx->opt.ring_sbk;
+    const bool one_mt = omt >= 2 && omt <= C.max_mt && omt != 7;
     for (int mt : {2, 3, 4, 5, 6, 8}) {
         if (mt > C.max_mt) break;
+        if (one_mt && mt != omt) continue;
         const int64_t MB = (tiles + mt - 1) / mt;
-        for (int64_t S = 1; S <= std::max<int64_t>(steps / 2, 1); S++) {
+        const bool counted = MB * NB <= kGemmCounters;
+        int64_t s0 = 1, s1 = counted ? std::max<int64_t>(steps / 2, 1) : 1;
+        if (osbk >= 0) {
+            s0 = osbk > 0 ? (steps + osbk - 1) / osbk : 1;
+            if (!counted || 4 * s0 * MB * 16 * mt * NB * kG2BN > INT32_MAX) s0 = 1;
+            s1 = s0;
+        }
+        for (int64_t S = s0; S <= s1; S++) {
             const int64_t wgs = MB * ((NB + 7) / 8 * 8) * S;
-            if (S > 1 && (wgs > slots || MB * NB > kGemmCounters)) break;
-            const int64_t sbk = (steps + S - 1) / S;
-            if (S > 1 && sbk == (steps + S - 2) / (S - 1)) continue;  // the same slices as S - 1
+            if (S > s0 && wgs > slots) break;
+            const int64_t sbk = S == 1 ? steps : osbk > 0 ? osbk : (steps + S - 1) / S;
+            if (S > s0 && sbk == (steps + S - 2) / (S - 1)) continue;  // the same slices as S - 1
             const double part = S > 1 ? 4.0 * S * MB * 16 * mt * NB * kG2BN : 0.0;
             const double cost = C.share((wgs + ctx->n_cu - 1) / ctx->n_cu) * sbk * (C.fixed + C.per_tile * mt) +
                                 (S > 1 ? C.slice : 0.0) + C.byte * part;
@@ -2532,7 +2547,7 @@ static GemmPlan plan_gemmd(const sihip_ctx *ctx, int count, const sihip_weight *
     int64_t wgs = 0;
     for (int i = 0; i < count; i++) wgs += (w[i]->L.n_out + 255) / 256 * 8 * q.MB;
     GemmPlan p;
-    if (wgs <= ctx->n_cu && (f16 || nk * q.mt <= 64)) {
+    if (ctx->opt.ring_mt < 0 && wgs <= ctx->n_cu && (f16 || nk * q.mt <= 64)) {
         p.v2 = p.small = true;
         p.mt = q.mt;
         p.Mp = q.Mp;

@@ -107,3 +107,38 @@ def test_a_group_keeps_the_newer_kernels():
     assert {M: v[0].split("_kernel")[0] for M, v in got.items()} == {112: "gemmsk", 256: "gemmx"}
     got = gemms({}, ["Q8_0"] * 3, 256, 2048, [17, 200])
     assert all(v[0].startswith("gemmd") and len(v) == 1 for v in got.values())
+
+
+def _ring_runs():
+    """What test_ring of test_gpu_gemm_short.py and test_gpu_gemm_dense.py run:
+    [type, m tiles, steps, slice length, options, elements per step]."""
+    import siphon_amd as sa
+
+    from . import test_gpu_gemm_dense as dense
+    from . import test_gpu_gemm_short as short
+    kq = {"GEMMSK_MAX_M": 0, "GEMMX_MIN_M": 9}
+    for t in short.KQ:
+        for mt, u in short.ROUND.items():
+            yield from ((sa.NAMES[t], mt, *c, kq, 256) for c in short.ring_cases(u))
+    for t, mt in dense.RING:
+        yield from ((sa.NAMES[t], mt, *c, {"GEMMD_MIN_M": 9}, 128) for c in short.ring_cases(dense.ROUND[t][mt]))
+
+
+def test_ring_cases_run_what_they_name():
+    runs = list(_ring_runs())
+    got = fake_hip.run(f"""
+        result = []
+        for t, mt, steps, sbk, options, size in {runs!r}:
+            for name, value in [*options.items(), ("RING_MT", mt), ("RING_SBK", sbk)]:
+                dev.set_option(name, value)
+            w = upload(getattr(sa, t), 140, size * steps)
+            w.prepare_gemm()
+            fake.fake_reset(0)
+            dev.gemm_dev(w, X, 16 * mt + 5, X)
+            result.append([sa.TYPES[t], *launched()[-1]])
+            w.free()
+    """)
+    for (t, mt, steps, sbk, _, size), (number, kernel, grid, _) in zip(runs, got):
+        name = f"gemmx_kernel<{number},{number},{mt}>" if size == 256 else f"gemmd_kernel<{number},{mt}>"
+        slices = -(-steps // sbk) if sbk else 1
+        assert (kernel, grid) == (name, 8 * 2 * slices), (t, mt, steps, sbk)

@@ -10,12 +10,18 @@ from siphon_amd import synth
 
 from .test_gpu_gemm import _rows
 from .test_gpu_gemm_multi import _run
+from .test_gpu_gemm_short import ring_cases
 from .test_gpu_parity import assert_close
 from .test_gpu_slices import _HipGraph, bits
 
 pytestmark = pytest.mark.gpu
 
 TYPES = [sa.F16, sa.Q4_0, sa.Q5_0, sa.Q8_0]
+
+# gemmd.h: m tiles -> steps of a round
+ROUND = {sa.F16: {2: 12, 3: 12, 4: 12, 5: 6, 6: 6}}
+ROUND.update({t: {2: 12, 3: 12, 4: 12, 5: 4} for t in TYPES[1:]})
+RING = [(t, mt) for t in TYPES for mt in ROUND[t]]
 
 
 def _check(dev, oracle, mats, n_in, M, what):
@@ -35,14 +41,27 @@ def _check(dev, oracle, mats, n_in, M, what):
 
 @pytest.mark.parametrize("wt", TYPES, ids=[sa.NAMES[t] for t in TYPES])
 def test_single(dev, oracle, option, wt):
-    """Small workgroups of one, two and three m tiles with fewer, as many and
-    more steps than waves; tiles (many rows or a large M) with fewer steps than
-    the ring, K slices, and rows past n_out and M."""
+    """Small workgroups (gemmds_kernel) of one, two and three m tiles with fewer,
+    as many and more steps than waves, rows past n_out and M; the longest rows of
+    the Q8_0 pairs in tiles."""
     option("GEMMD_MIN_M", 9)
     for n_out, n_in, M in ((33, 128, 9), (200, 512, 17), (96, 2304, 33), (70, 1152, 49),
                            (300, 256, 600), (2080, 640, 129), (260, 4096, 400), (130, 1280, 700)):
         print(f"single {sa.NAMES[wt]} {n_out}x{n_in} M={M}", flush=True)
         _check(dev, oracle, [(wt, n_out)], n_in, M, "single")
+
+
+@pytest.mark.parametrize("wt,mt", RING, ids=[f"{sa.NAMES[t]}-{mt}" for t, mt in RING])
+def test_ring(dev, oracle, option, wt, mt):
+    """Tiles of every m tile count at the edges of their rounds; two m blocks, the
+    second of five rows, two n blocks, the second of 12. test_gemm_dispatch.py
+    checks that these cases run the instance and the slices they name."""
+    option("GEMMD_MIN_M", 9)
+    option("RING_MT", mt)
+    for steps, sbk in ring_cases(ROUND[wt][mt]):
+        option("RING_SBK", sbk)
+        print(f"ring {sa.NAMES[wt]} mt={mt} steps={steps} sbk={sbk}", flush=True)
+        _check(dev, oracle, [(wt, 140)], 128 * steps, 16 * mt + 5, f"mt={mt} sbk={sbk}")
 
 
 @pytest.mark.parametrize("wt", TYPES, ids=[sa.NAMES[t] for t in TYPES])
@@ -53,9 +72,14 @@ def test_groups(dev, oracle, wt):
 
 
 @pytest.mark.parametrize("wt", [sa.F16, sa.Q8_0], ids=["F16", "Q8_0"])
-def test_capture(dev, oracle, wt):
+@pytest.mark.parametrize("tiles", [False, True], ids=["rule", "tiles"])
+def test_capture(dev, oracle, option, wt, tiles):
     """After an eager call of more rows, captured calls of fewer find their
-    workspaces; each replay gives the bits of the first."""
+    workspaces, by the rule (small workgroups and the older kernels) and in tiles;
+    each replay gives the bits of the first."""
+    if tiles:
+        option("GEMMD_MIN_M", 9)
+        option("RING_MT", 3)
     rng = np.random.default_rng(9)
     n_out, n_in, M = 520, 2048, 300
     W = synth.make_weights(wt, n_out, n_in, rng)

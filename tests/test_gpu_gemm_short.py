@@ -17,6 +17,18 @@ pytestmark = pytest.mark.gpu
 
 KQ = [sa.Q2_K, sa.Q3_K, sa.Q4_K, sa.Q5_K, sa.Q6_K]
 
+# gemmx.h: m tiles -> steps of a round (ring slots times super-blocks of weights
+# in registers)
+ROUND = {2: 6, 3: 6, 4: 3, 5: 3, 6: 2, 8: 2}
+
+
+def ring_cases(u):
+    """(steps, K-slice length or 0) at the edges of a round of u steps: fewer
+    steps than the ring holds, one short of a round (the longest partial one), a
+    round, one and u + 1 more; slices of a round and one with a ragged last one,
+    and of two."""
+    return [(1, 0), (2, 0), (u - 1, 0), (u, 0), (u + 1, 0), (2 * u + 1, 0), (2 * u + 1, u + 1), (5, 2)]
+
 
 def _check(dev, oracle, mats, n_in, M, what, seed=0):
     rng = np.random.default_rng(M * 131 + n_in + seed)
@@ -48,15 +60,30 @@ def test_short_prompts(dev, oracle, option, wt, waves):
 
 @pytest.mark.parametrize("wt", KQ, ids=[sa.NAMES[t] for t in KQ])
 def test_longer_prompts(dev, oracle, option, wt):
-    """Rings of one and two super-blocks ahead at fewer, as many and more
-    super-blocks than slots, K slices (few rows, long rows), every m tile
-    count of the plan, and a row block past n_out in the last n block."""
+    """The plans of small products (32-row m blocks) with fewer, as many and more
+    super-blocks than slots, K slices (few rows, long rows), and a row block past
+    n_out in the last n block."""
     option("GEMMSK_MAX_M", 0)
     option("GEMMX_MIN_M", 9)
     for n_out, n_in, M in ((33, 256, 17), (200, 512, 40), (130, 768, 64), (128, 8192, 33),
                            (96, 1792, 80), (160, 2304, 96), (300, 1280, 129)):
         print(f"longer {sa.NAMES[wt]} {n_out}x{n_in} M={M}", flush=True)
         _check(dev, oracle, [(wt, n_out)], n_in, M, "ring")
+
+
+@pytest.mark.parametrize("wt", KQ, ids=[sa.NAMES[t] for t in KQ])
+@pytest.mark.parametrize("mt", list(ROUND))
+def test_ring(dev, oracle, option, wt, mt):
+    """Every m tile count at the edges of its rounds; two m blocks, the second of
+    five rows, two n blocks, the second of 12. test_gemm_dispatch.py checks that
+    these cases run the instance and the slices they name."""
+    option("GEMMSK_MAX_M", 0)
+    option("GEMMX_MIN_M", 9)
+    option("RING_MT", mt)
+    for steps, sbk in ring_cases(ROUND[mt]):
+        option("RING_SBK", sbk)
+        print(f"ring {sa.NAMES[wt]} mt={mt} steps={steps} sbk={sbk}", flush=True)
+        _check(dev, oracle, [(wt, 140)], 256 * steps, 16 * mt + 5, f"mt={mt} sbk={sbk}", steps)
 
 
 @pytest.mark.parametrize("short", [1000, 0], ids=["short", "longer"])
@@ -111,3 +138,38 @@ def test_capture_takes_the_copy_that_exists(dev, oracle, option):
             yd.free()
             w.free()
             other.free()
+
+
+@pytest.mark.parametrize("wt,n_in", [(sa.Q5_K, 2048), (sa.F16, 1024)], ids=["Q5_K", "F16"])
+def test_capture_without_room_for_slices(wt, n_in):
+    """A captured call whose partial sums were never allocated runs without K
+    slices: the bits of the eager unsliced call."""
+    rng = np.random.default_rng(7)
+    n_out, M = 140, 40
+    dev = sa.Device(0)  # its workspaces hold what the calls below ask for
+    hg = _HipGraph()
+    bufs, w = [], None
+    try:
+        for name, v in (("GEMMSK_MAX_M", 0), ("GEMMX_MIN_M", 9), ("GEMMD_MIN_M", 9), ("RING_MT", 2), ("RING_SBK", 0)):
+            dev.set_option(name, v)
+        w = dev.upload(wt, n_out, n_in, synth.make_weights(wt, n_out, n_in, rng))
+        bufs = [dev.to_device(_rows(rng, M, n_in)), *(dev.to_device(np.full(M * n_out, np.nan, np.float32)) for _ in range(2))]
+        x, eager, got = (b.ptr for b in bufs)
+        dev.gemm_dev(w, x, M, eager, hg.stream.value)
+        dev.synchronize()
+        dev.set_option("RING_SBK", 2)
+        hg.begin()
+        dev.gemm_dev(w, x, M, got, hg.stream.value)
+        hg.end()
+        want = bits(bufs[1].to_host(np.float32, M * n_out))
+        for _ in range(3):
+            bufs[2].fill(np.full(M * n_out, np.nan, np.float32))
+            hg.replay()
+            assert np.array_equal(bits(bufs[2].to_host(np.float32, M * n_out)), want)
+    finally:
+        hg.close()
+        for b in bufs:
+            b.free()
+        if w:
+            w.free()
+        dev.close()

@@ -4,7 +4,8 @@ turned off (GEMMKF_MAX_M = 0) gemm2s_q4k_kernel (Q4_K, 3 <= M <= 16) and
 gemmks_kernel (Q2_K, Q5_K up to M = 8, Q3_K, Q6_K up to M = 12, by option
 every K-quant up to 16) against the oracle, every output, |gpu - ref| <=
 1e-5 * sum|terms| + 1e-6; the M values past a format's rule run its larger
-GEMM. Shapes cover a single super-block per row (fewer super-blocks than
+GEMM (the prompt GEMMs, which the built-in rule takes from M = 9, are off in
+those cases and have tests of their own). Shapes cover a single super-block per row (fewer super-blocks than
 waves per workgroup), super-block counts that the waves do not divide,
 row counts that leave a 32-row block part empty, every 4-row activation
 group count (M = 3 to 16), each waves-per-workgroup choice, and rows at
@@ -59,6 +60,9 @@ M_CASES = [(m, True) for m in (3, 4, 5, 8)] + [(m, False) for m in (3, 4, 5, 8, 
 @pytest.mark.parametrize("n_out,n_in", [(33, 256), (200, 1024), (96, 2304)])
 def test_small_m_vs_oracle(dev, oracle, option, wt, M, n_out, n_in, fused):
     option("GEMMKF_MAX_M", 8 if fused else 0)
+    if not fused:
+        option("GEMMSK_MAX_M", 0)
+        option("GEMMX_MIN_M", 0)
     _check(dev, oracle, wt, n_out, n_in, M, 7000 + 97 * wt + 13 * M + n_in,
            f"{sa.NAMES[wt]} {n_out}x{n_in} M={M} {'fused' if fused else 'separate'}")
 
