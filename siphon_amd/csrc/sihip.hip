@@ -2063,7 +2063,9 @@ static SKPlan plan_gemmsk(int64_t M, int64_t nb) {
 
 // The GEMM that a single matrix takes by the built-in rule.
 enum class OnGemm { kShort, kRing, kOlder };  // gemmsk.h, gemmx.h / gemmd.h, the plan of plan_gemm
-static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M);
+static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M, bool newer_only = false);
+static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M,
+                           hipStream_t st, bool noalloc = false);
 
 // Whether an option puts M rows of a K-quant on one of the other GEMMs
 // (GEMMKS_MAX_M, GEMM2S_MAX_M, GEMM2_MIN_M, GEMM6_MIN_M): what it names keeps
@@ -2079,7 +2081,9 @@ static bool placed_by_option(const Options &o, uint32_t type, int64_t M) {
 // and M in its range, unless an option sets the tiling of the other GEMMs or
 // puts M on one of them.
 // Where a missing weight copy cannot be built (under graph capture, and with
-// noalloc), the kernel whose copies exist is taken.
+// noalloc), a kernel whose copies exist is taken: with gemmks.h's alone this
+// one or gemmx.h, which share it, by the rule for the size (Q5_K 4096 x 14336
+// at M = 350 77.5 us here, 65.6 there, at M = 2048 619 and 280).
 static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w,
                             int64_t M, hipStream_t st, bool noalloc = false) {
     if (count < 1 || count > kSKMaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
@@ -2094,9 +2098,10 @@ static bool gemmsk_eligible(const sihip_ctx *ctx, int count, const sihip_weight 
         here = here && w[i]->gsmall;
         other = other && plan_copy(w[i], plan_gemm(ctx, L, M));
     }
-    if (here != other && (noalloc || capturing(st))) return here;
+    const bool one_copy = here != other && (noalloc || capturing(st));
+    if (one_copy && (!here || !gemmx_eligible(ctx, count, w, M, st, noalloc))) return here;
     if (ctx->opt.gemmsk_max_m >= 0) return M <= ctx->opt.gemmsk_max_m;
-    if (count == 1) return single_kquant(ctx, w[0]->L, M) == OnGemm::kShort;
+    if (count == 1) return single_kquant(ctx, w[0]->L, M, one_copy) == OnGemm::kShort;
     int64_t blocks = 0;
     for (int i = 0; i < count; i++) blocks += (w[i]->L.n_out + 31) / 32;
     return M <= kGemmSKMaxM || (M < kGemm2MinM && blocks * ((M + 15) / 16) <= kGemmSKTiles &&
@@ -2282,7 +2287,7 @@ static GemmPlan plan_gemmx(const sihip_ctx *ctx, int64_t M, int64_t nb, int64_t 
 }
 
 static bool gemmx_eligible(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M,
-                           hipStream_t st, bool noalloc = false) {
+                           hipStream_t st, bool noalloc) {
     if (count < 1 || count > kG2MaxSegs || ctx->opt.gemm_mt >= 0 || ctx->opt.gemm_sbk >= 0) return false;
     if (ctx->opt.gemmx_min_m == 0 || M < 9 || M < gemm_min_m(ctx->opt)) return false;
     bool here = true, other = true;
@@ -2345,17 +2350,19 @@ static KQuantStep kquant_step(uint32_t type) {
     }
 }
 
-static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M) {
+// newer_only: the older kernels' copy does not exist.
+static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M, bool newer_only) {
     const int64_t nb = L.n_in / 256;
     // Q4_K from kGemm2MinM rows on gemm2.h (4096 x 4096 at M = 512 33.5 us
     // against 38.1 here), and up to 16 with long rows on gemm2s.h (4096 x 14336
     // 13.7 against 15.0, 4096 x 11008 1.12 times)
-    if (L.type == T_Q4_K && (M >= gemm2_min_m(ctx->opt) || (M <= 16 && L.n_in > kGemmSKMaxK)))
+    if (!newer_only && L.type == T_Q4_K &&
+        (M >= gemm2_min_m(ctx->opt) || (M <= 16 && L.n_in > kGemmSKMaxK)))
         return OnGemm::kOlder;
     // few rows of output, from kGemm2MinM: kernels whose m tiles need fewer K
     // slices and, for Q6_K, no decode (4096 x 4096 at M = 512: Q6_K 33.3 against
     // 50.8, Q3_K 32.4 against 41.7; at M = 2048 90.6 / 81.0 against 93.4 / 71.7)
-    if (M >= kGemm2MinM && L.n_out <= 8192 &&
+    if (!newer_only && M >= kGemm2MinM && L.n_out <= 8192 &&
         (L.type == T_Q6_K || ((L.type == T_Q2_K || L.type == T_Q3_K) && M < 1024)))
         return OnGemm::kOlder;
     const KQuantStep c = kquant_step(L.type);
@@ -2371,7 +2378,7 @@ static OnGemm single_kquant(const sihip_ctx *ctx, const Layout &L, int64_t M) {
     const GemmPlan x = plan_gemmx(ctx, M, nb, (L.n_out + kG2BN - 1) / kG2BN);
     const double ring = 8.8 + c.ring * x.cost;
     const OnGemm newer = sk <= ring ? OnGemm::kShort : OnGemm::kRing;
-    if (M < 17) return newer;
+    if (newer_only || M < 17) return newer;
     const GemmPlan p = plan_gemm(ctx, L, M);
     const int64_t bm = p.v2 ? 16 * p.mt : 32 * p.mt;
     const double start = L.type == T_Q6_K ? 5.8 : bm == 32 ? 8.7 : 11.6;
@@ -3103,34 +3110,37 @@ extern "C" int sihip_gemm_dev_noalloc(sihip_ctx *ctx, const sihip_weight *w, con
     }
     GemmPlan p = plan_gemm(ctx, w->L, M);
     const bool planned = plan_copy(w, p) != nullptr;
-    if (w->gsmall && gemmsk_eligible(ctx, 1, &w, M, st, true)) {
-        const int64_t nb = w->L.n_in / 256;
-        float *Yp = Y;
-        SKPlan sp = plan_gemmsk(M, nb);
-        if ((size_t)sp.ws_bytes <= room)  // else the kernels below
-            return launch_gemmsk_group(ctx, 1, &w, sp, X, M, &Yp, ctx->scratch, st);
-        // planes that only the plan's kernel fits into the scratch, whose copy
-        // is missing: pieces of whole m blocks of three 16-row tiles
-        const int64_t piece = (int64_t)(room / (size_t)(nb * g2_rec_bytes(16))) / 3 * 48;
-        if (!planned && (size_t)p.ws_bytes <= room && piece > 0) {
-            for (int64_t m = 0; m < M; m += piece) {
-                const int64_t n = std::min(piece, M - m);
-                Yp = Y + m * w->L.n_out;
-                sp = plan_gemmsk(n, nb);
-                const int rc = launch_gemmsk_group(ctx, 1, &w, sp, X + m * w->L.n_in, n, &Yp, ctx->scratch, st);
-                if (rc) return rc;
-            }
-            return SIHIP_OK;
-        }
-    }
-    if (w->gsmall && gemmx_eligible(ctx, 1, &w, M, st, true)) {
-        const GemmPlan gp = plan_gemmx(ctx, M, w->L.n_in / 256, gemm_blocks(1, &w));
-        const size_t off = ((size_t)gp.ws_bytes + 255) & ~(size_t)255;
-        float *Yp = Y;
-        if ((size_t)gp.ws_bytes <= room) {
+    const bool on_sk = w->gsmall && gemmsk_eligible(ctx, 1, &w, M, st, true);
+    const bool on_gx = w->gsmall && gemmx_eligible(ctx, 1, &w, M, st, true);
+    if (on_sk || on_gx) {
+        const int64_t n_in = w->L.n_in, nb = n_in / 256;
+        // rows m .. m + n - 1, where the planes fit
+        auto part_on = [&](bool sk, int64_t m, int64_t n, bool &fits) -> int {
+            float *Yp = Y + m * w->L.n_out;
+            const SKPlan sp = plan_gemmsk(n, nb);
+            const GemmPlan gp = plan_gemmx(ctx, n, nb, gemm_blocks(1, &w));
+            fits = (size_t)(sk ? sp.ws_bytes : gp.ws_bytes) <= room;
+            if (!fits) return SIHIP_OK;
+            if (sk) return launch_gemmsk_group(ctx, 1, &w, sp, X + m * n_in, n, &Yp, ctx->scratch, st);
+            const size_t off = ((size_t)gp.ws_bytes + 255) & ~(size_t)255;
             const bool slices = gp.S > 1 && off + (size_t)gp.part_bytes <= room;
             const GemmBufs GB{ctx->scratch, (float *)(ctx->scratch + off), (uint32_t *)(ctx->scratch + room)};
-            return launch_gemmx_group(ctx, 1, &w, X, M, &Yp, GB, slices, st);
+            return launch_gemmx_group(ctx, 1, &w, X + m * n_in, n, &Yp, GB, slices, st);
+        };
+        bool fits = false;
+        int rc = SIHIP_OK;
+        if (on_sk) rc = part_on(true, 0, M, fits);
+        if (!fits && on_gx) rc = part_on(false, 0, M, fits);
+        if (fits) return rc;
+        // planes that only the plan's kernel fits into the scratch, whose copy
+        // is missing: pieces of eight 16-row tiles (gemmsk.h: three) and multiples
+        const int64_t tiles = (int64_t)(room / (size_t)(nb * g2_rec_bytes(16)));
+        const bool sk = on_sk || tiles < 15;
+        const int64_t piece = sk ? tiles / 3 * 48 : (tiles - 7) / 8 * 128;  // (a piece's planes: at most 7 tiles more)
+        if (!planned && (size_t)p.ws_bytes <= room && piece > 0) {
+            fits = true;
+            for (int64_t m = 0; m < M && !rc && fits; m += piece) rc = part_on(sk, m, std::min(piece, M - m), fits);
+            if (rc || fits) return rc;
         }
     }
     if (w->gemm2 && gemmd_eligible(ctx, 1, &w, M)) {

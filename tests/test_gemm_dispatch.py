@@ -63,6 +63,34 @@ def test_noalloc_after_a_short_prompt(wt, n_out, n_in, M, launches):
     assert len(got) == launches and all(k.startswith(("gemmsk", "gemmx", "gemm6", "gemm_kq")) for k in got), got
 
 
+@pytest.mark.parametrize("types,n_out,n_in,M", [
+    (["Q5_K"], 4096, 14336, 2048), (["Q5_K"], 14336, 4096, 200), (["Q2_K"], 4096, 14336, 350),
+    (["Q4_K"], 14336, 4096, 350), (["Q3_K"] * 2, 27648, 512, 1568), (["Q5_K"] * 2, 4096, 5120, 187),
+    (["Q4_K"], 4096, 4096, 37), (["Q6_K"], 4096, 4096, 300),
+])
+def test_a_capture_takes_the_kernel_of_the_call_before(types, n_out, n_in, M):
+    """The first call builds the copy of its own kernel alone, which two GEMMs
+    share: a captured repetition launches what the call did."""
+    eager, captured, noalloc = fake_hip.run(f"""
+        ws = [upload(getattr(sa, t), {n_out}, {n_in}) for t in {types!r}]
+        call = lambda: dev.gemm_multi_dev(ws, X, {M}, [X] * len(ws), 1)
+        call()
+        result = []
+        for capture in (0, 1):
+            fake.fake_reset(0)
+            fake.fake_capture(capture)
+            call()
+            result.append(launched())
+        fake.fake_reset(0)
+        if {n_in * M} < 1 << 24:  # (the planes fit the scratch)
+            dev.gemm_dev_noalloc(ws[0], X, {M}, X, 1)
+        result.append(launched())
+    """)
+    assert eager == captured
+    if len(types) == 1 and noalloc:
+        assert noalloc[-1][0].split("<")[0] == eager[-1][0].split("<")[0]
+
+
 @pytest.mark.parametrize("n_out,M,waves,grid", [
     (4096, 48, 8, 256), (4128, 48, 4, 136), (5120, 9, 4, 160), (2048, 96, 8, 256), (2080, 96, 4, 144),
 ])
