@@ -2803,6 +2803,25 @@ static XKey xkey(const Layout &L, const GemmPlan &p) {
     return XKey{1, 16 * p.mt, 0};
 }
 
+// Under capture: some of the matrices hold only the copy of gemmsk.h and
+// gemmx.h and others only their plan's, as calls of one matrix each leave
+// them. A launch for all would need a copy that cannot be built; a call for each
+// takes what it has.
+static bool copies_differ(const sihip_ctx *ctx, int count, const sihip_weight *const *w, int64_t M,
+                          hipStream_t st) {
+    if (!capturing(st)) return false;
+    bool here = true, other = true;
+    for (int i = 0; i < count; i++) {
+        const bool planned = plan_copy(w[i], plan_gemm(ctx, w[i]->L, M)) != nullptr;
+        const bool newer = is_kquant(w[i]->L.type) && w[i]->gsmall &&
+                           (gemmsk_eligible(ctx, 1, &w[i], M, st) || gemmx_eligible(ctx, 1, &w[i], M, st));
+        if (!planned && !newer) return false;
+        here = here && w[i]->gsmall;
+        other = other && planned;
+    }
+    return !here && !other;
+}
+
 // The MFMA GEMMs of several weights over one X: the weights of one record
 // family get one m-tile count (the largest of their own plans that each
 // kernel has), so X is quantized once per distinct record layout and the
@@ -2811,6 +2830,13 @@ static int run_gemm_multi(sihip_ctx *ctx, int count, const sihip_weight *const *
                           const float *X, int64_t M, float *const *Y, hipStream_t st) {
     if (count <= kKFMaxSegs && gemmkf_eligible(ctx, count, wc, M))
         return run_gemmkf(ctx, count, wc, X, M, Y, st);
+    if (count > 1 && copies_differ(ctx, count, wc, M, st)) {
+        for (int i = 0; i < count; i++) {
+            const int rc = run_gemm_mfma(ctx, wc[i], X, wc[i]->L.n_in, M, Y[i], wc[i]->L.n_out, st);
+            if (rc) return rc;
+        }
+        return SIHIP_OK;
+    }
     if (gemmsk_eligible(ctx, count, wc, M, st)) return run_gemmsk(ctx, count, wc, X, M, Y, st);
     if (gemmx_eligible(ctx, count, wc, M, st)) return run_gemmx(ctx, count, wc, X, M, Y, st);
     if (gemmd_eligible(ctx, count, wc, M)) return run_gemmd(ctx, count, wc, X, M, Y, st);

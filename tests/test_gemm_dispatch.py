@@ -91,6 +91,27 @@ def test_a_capture_takes_the_kernel_of_the_call_before(types, n_out, n_in, M):
         assert noalloc[-1][0].split("<")[0] == eager[-1][0].split("<")[0]
 
 
+@pytest.mark.parametrize("types,M", [(["Q4_K", "Q6_K"], 200), (["Q6_K", "Q6_K", "Q6_K"], 130), (["Q4_K", "Q4_K"], 200)])
+def test_a_captured_group_after_calls_of_its_matrices(types, M):
+    """Calls of one matrix each leave some with the newer kernels' copy alone and
+    some with their plan's: a captured call of the group, whose launch would
+    need one copy of all, runs each matrix on the copy it has."""
+    calls, group = fake_hip.run(f"""
+        ws = [upload(getattr(sa, t), 14336 if i else 1024, 4096) for i, t in enumerate({types!r})]
+        result = [[]]
+        for w in ws:
+            dev.gemm_dev(w, X, {M}, X, 1)
+            fake.fake_reset(0)
+            dev.gemm_dev(w, X, {M}, X, 1)
+            result[0] += launched()
+        fake.fake_reset(0)
+        fake.fake_capture(1)
+        dev.gemm_multi_dev(ws, X, {M}, [X] * len(ws), 1)
+        result.append(launched())
+    """)
+    assert group == calls and len({k.split("_kernel")[0] for k, *_ in calls if "_kernel" in k}) > 1
+
+
 @pytest.mark.parametrize("n_out,M,waves,grid", [
     (4096, 48, 8, 256), (4128, 48, 4, 136), (5120, 9, 4, 160), (2048, 96, 8, 256), (2080, 96, 4, 144),
 ])
