@@ -19,6 +19,7 @@ INSTANCES = [
     ("gemmd_kernel<1, 5>(GDArgs)", 3),
     ("gemmd_kernel<6, 5>(GDArgs)", 4),
     ("gemmd_kernel<8, 3>(GDArgs)", 4),
+    ("gemmd_kernel<8, 4>(GDArgs)", 4),
 ]
 # the build's flags, and two other schedules that the compiler might choose: the
 # order must not rest on one

@@ -20,7 +20,7 @@ TYPES = [sa.F16, sa.Q4_0, sa.Q5_0, sa.Q8_0]
 
 # gemmd.h: m tiles -> steps of a round
 ROUND = {sa.F16: {2: 12, 3: 12, 4: 12, 5: 6, 6: 6}}
-ROUND.update({t: {2: 12, 3: 12, 4: 12, 5: 4} for t in TYPES[1:]})
+ROUND.update({t: {2: 12, 3: 12, 4: 4, 5: 4} for t in TYPES[1:]})
 RING = [(t, mt) for t in TYPES for mt in ROUND[t]]
 
 
