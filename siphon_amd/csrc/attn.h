@@ -55,8 +55,10 @@ struct AttnArgs {
     int64_t n_ctx, ld, lw;
     int n, hd, gqa, n_kv;
     int nbs, nbe;
-    int gx;                // blocks per row of the grid (attn_block)
-    int rb;                // 16-row blocks of values per workgroup of the single launch
+    union {
+        int gx;            // blocks per row of the grid (attn_block)
+        int rb;            // 16-row blocks of values per workgroup of the single launch
+    };
     float kq_scale;
 };
 
@@ -169,10 +171,10 @@ __device__ inline float tail_exp(float x) { return (float)exp((double)x); }
 struct AttnWg {
     int hk, h, blk;
 };
-__device__ inline AttnWg attn_wg(const AttnArgs &A, int id) {
-    const int rest = id / A.n_kv;
+__device__ inline AttnWg attn_wg(const AttnArgs &A, int n_kv, int id) {
+    const int rest = id / n_kv;
     AttnWg w;
-    w.hk = id % A.n_kv;
+    w.hk = id % n_kv;
     w.h = w.hk * A.gqa + rest % A.gqa;
     w.blk = rest / A.gqa;
     return w;
@@ -287,8 +289,9 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
     __shared__ float red[kAttnHeads][4];
     const int chunks = (A.gqa + kAttnHeads - 1) / kAttnHeads;
     const int id = attn_block(A), hk = id % A.n_kv, rest = id / A.n_kv;
+    // (a spare block scores row n - 1 and stores nothing: to return here would
+    // put a second round trip for arguments before the key loads, 0.2 us)
     const int hc = rest % chunks * kAttnHeads, blk = rest / chunks;
-    if (blk >= A.nbs) return;
     const int h0 = hk * A.gqa + hc, nh = min(kAttnHeads, A.gqa - hc);
     const int hd = A.hd;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, L = lane & 3;
@@ -315,7 +318,7 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs A) {
         if (lane == 0) red[hh][wave] = mx;
     }
     __syncthreads();
-    if ((int)threadIdx.x < nh) {
+    if ((int)threadIdx.x < nh && blk < A.nbs) {
         const float *r = red[threadIdx.x];
         A.pm[(int64_t)(h0 + threadIdx.x) * A.nbs + blk] =
             max_sel(max_sel(r[0], r[1]), max_sel(r[2], r[3]));
@@ -355,7 +358,10 @@ constexpr int kAttnExpBlock = 1024;
 __global__ __launch_bounds__(256) void attn_exp_kernel(AttnArgs A) {
     __shared__ float redf[4];
     __shared__ double redd[4];
-    const AttnWg W = attn_wg(A, attn_block(A));
+    // one round trip for the arguments, not another behind the branch
+    int n_kv = A.n_kv;
+    asm volatile("" : "+s"(n_kv) : "s"(A.gx), "s"(A.n), "s"(A.sw), "s"(A.lw), "s"(A.pm));
+    const AttnWg W = attn_wg(A, n_kv, attn_block(A));
     if (W.blk >= A.nbe) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int j = W.blk * kAttnExpBlock + 4 * (int)threadIdx.x;
@@ -514,7 +520,7 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs A) {
     __shared__ __attribute__((aligned(16))) uint8_t ring[kR * kAttnSlot];
     __shared__ __attribute__((aligned(16))) float se[kR][kAttnChunk];
     __shared__ __attribute__((aligned(16))) uint16_t sp[2][kAttnChunk];
-    const AttnWg W = attn_wg(A, (int)blockIdx.x);
+    const AttnWg W = attn_wg(A, A.n_kv, (int)blockIdx.x);
     const int tid = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r = tid >> 4, L = tid & 15;
     const int rows = min(kAttnPvRows, A.hd - W.blk * kAttnPvRows);
@@ -684,7 +690,11 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ float redf[8];
     __shared__ double redd[8];
-    const AttnWg W = attn_wg(A, (int)blockIdx.x);
+    // one round trip for the arguments, not another for rb before the value loads
+    // (0.25 us of a launch)
+    int n_kv = A.n_kv;
+    asm volatile("" : "+s"(n_kv) : "s"(A.n_ctx), "s"(A.k), "s"(A.rb));
+    const AttnWg W = attn_wg(A, n_kv, (int)blockIdx.x);
     const int n = A.n, np = attn_fused_np(n), hd = A.hd;
     uint16_t *const sq = reinterpret_cast<uint16_t *>(smem);
     float *const ss = reinterpret_cast<float *>(smem + kAttnMaxHd * 2);

@@ -14,10 +14,12 @@
 // MFMAs per wave, a fraction of a microsecond, and one step of loads ahead does
 // not cover one; at more rows the LDS reads of the activations (F16, 0.12 us
 // per m tile and step) or the epilogue's 12 VALU instructions per MFMA (Q8_0
-// pairs, 0.26 us). Layer of 7 matrices, us before -> now: 1.1B F16 M = 40 68 ->
-// 47, M = 200 124 -> 75, M = 500 200 -> 107; Q8_0 M = 200 156 -> 96, 0.5B M =
-// 300 104 -> 75; Q5_0 M = 64 88 -> 62. The records of the next gd_ring(MT) - 1 steps are copied to LDS by DMA
-// and the weights of the next gd_wdepth(MT) are loaded into registers; each
+// pairs, 0.26 us). Layer of 7 matrices, four groups called one after another, us on
+// the kernels of gemmh.h and gemmq.h -> here: 1.1B F16 M = 40 61 -> 42, M = 200
+// 120 -> 68, M = 500 202 -> 98; Q8_0 M = 200 148 -> 91, 0.5B M = 300 98 -> 72;
+// Q5_0 M = 64 82 -> 61. The records of the next gd_ring(MT) - 1 steps are copied
+// to LDS by DMA and the weights of the next gd_wdepth(MT) are loaded into
+// registers; each
 // step waits for its own record by count and meets the other waves at a bare
 // s_barrier. The ring is at least as deep as the weights run ahead: loads
 // retire in order, and a record must not wait for weights of later steps.

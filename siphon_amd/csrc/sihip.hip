@@ -1067,12 +1067,13 @@ static int64_t gemmkf_max_m(const Options &o) {
 constexpr int64_t kGemm2MinM = 384;
 static int64_t gemm2_min_m(const Options &o) { return o.gemm2_min_m > 0 ? o.gemm2_min_m : kGemm2MinM; }
 
-// The short-prompt K-quant GEMM (gemmsk.h) takes M from 9 to kGemmSKMaxM, and
-// longer ones, short of kGemm2MinM, of small products: up to kGemmSKTiles
-// 32 x 16 output tiles with rows of at most kGemmSKMaxK (option GEMMSK_MAX_M: up to that M instead,
-// 0: never). 8B Q4_K_M layer, us per layer on the kernels before / gemmsk.h /
-// gemmx.h: M = 16 79 / 60 / 78, 37 123 / 79 / 94, 64 127 / 87 / 104, 96 155 /
-// 104 / 133, 130 197 / 140 / 144, 300 282 / 267 / 224; its q/k/v (192 blocks
+// The short-prompt K-quant GEMM (gemmsk.h) takes groups of M from 9 to
+// kGemmSKMaxM, and longer ones, short of kGemm2MinM, of small products: up to
+// kGemmSKTiles 32 x 16 output tiles with rows of at most kGemmSKMaxK (option
+// GEMMSK_MAX_M: up to that M instead, 0: never). 8B Q4_K_M layer, four groups
+// called one after another, us on the kernels before / gemmsk.h / gemmx.h: M = 16
+// 87 / 58 / 75, 37 133 / 75 / 89, 64 137 / 84 / 95, 96 165 / 100 / 111, 130 200 /
+// 141 / 139, 200 212 / 198 / 178, 300 282 / 263 / 217; its q/k/v (192 blocks
 // of 32 rows) at M = 200 56 / 29 / 33 and 300 60 / 38 / 37, gate + up (896) at
 // M = 130 78 / 57 / 54, ffn_down (14336 long) at M = 130 43 / 44 / 41.
 constexpr int64_t kGemmSKMaxM = 112;
