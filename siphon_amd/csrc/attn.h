@@ -683,10 +683,11 @@ __host__ __device__ inline int attn_fused_lds(int n) {
     return np * 4 + np * 2 + kAttnPvRows * (np * 2 + 64) + kAttnMaxHd * 2;
 }
 
-// VEC: value rows by 16-byte loads (n_ctx % 8 == 0, v 16-byte aligned).
-template <int T, int KW, bool VEC>
-__global__ __launch_bounds__(kAttnFusedThreads)
-__attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(AttnArgs A) {
+// VEC: value rows by 16-byte loads (n_ctx % 8 == 0, v 16-byte aligned). ONE: rb is
+// 1, a kernel of its own (32 heads of 128 at n = 600 9.0 us per layer against 9.2
+// with the loop over blocks).
+template <int T, int KW, bool VEC, bool ONE>
+__device__ inline void attn_fused_body(const AttnArgs &A) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ float redf[8];
     __shared__ double redd[8];
@@ -694,6 +695,7 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
     // (0.25 us of a launch)
     int n_kv = A.n_kv;
     asm volatile("" : "+s"(n_kv) : "s"(A.n_ctx), "s"(A.k), "s"(A.rb));
+    const int rb = ONE ? 1 : A.rb;
     const AttnWg W = attn_wg(A, n_kv, (int)blockIdx.x);
     const int n = A.n, np = attn_fused_np(n), hd = A.hd;
     uint16_t *const sq = reinterpret_cast<uint16_t *>(smem);
@@ -723,7 +725,7 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
     // value rows, a block of 16 after another: 32 lanes per row; rows past hd
     // repeat the last, positions past n are not used
     const int r = tid >> 5, a = tid & 31;
-    const int b1 = min((W.blk + 1) * A.rb, (hd + kAttnPvRows - 1) / kAttnPvRows);
+    const int b1 = min((W.blk + 1) * rb, (hd + kAttnPvRows - 1) / kAttnPvRows);
     constexpr int kVP = kAttnFuseCap / 256;
     const int per8 = (n + 7) / 8;
     uint4 vq[kVP];
@@ -749,7 +751,7 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
             for (int i = a; i < n; i += 32) reinterpret_cast<uint16_t *>(svr)[i] = p[i];
         }
     };
-    int b = W.blk * A.rb;
+    int b = W.blk * rb;
     load_v(b);
     if (tid < hd) sq[tid] = (uint16_t)f32_to_f16_hw(qv);
     __syncthreads();
@@ -761,9 +763,13 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
         for (int u = 0; u < kD; u++) {
             const int pass = p0 + u;
             if (pass < passes) {
-                const uint16_t *const next = key_row(min(pass + kD, passes - 1));
-                const float v = key_score<T, KW, kD == 1>(kr[u], qr, hd, A.kq_scale, next, L4);
-                if (kD > 1 && pass + kD < passes) load_key<T, KW>(next, hd, L4, kr[u]);
+                float v;
+                if constexpr (kD == 1) {
+                    v = key_score<T, KW, true>(kr[u], qr, hd, A.kq_scale, key_row(min(pass + 1, passes - 1)), L4);
+                } else {
+                    v = key_score<T, KW>(kr[u], qr, hd, A.kq_scale);
+                    if (pass + kD < passes) load_key<T, KW>(key_row(pass + kD), hd, L4, kr[u]);
+                }
                 const int j = 128 * pass + jr;
                 if (L4 == 0 && j < n) {
                     ss[j] = v;
@@ -774,7 +780,7 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
         }
     }
     put_v(b);
-    if (b + 1 < b1) load_v(b + 1);
+    if (!ONE && b + 1 < b1) load_v(b + 1);
     mx = wave_max(mx);
     if (lane == 0) redf[wave] = mx;
     __syncthreads();
@@ -829,12 +835,23 @@ __attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(Attn
         // (opaque, or the tail's 31 conditions are kept across the blocks in
         // scalar registers that spill)
         int cnt = n - body;
-        asm volatile("" : "+s"(cnt));
+        if constexpr (!ONE) asm volatile("" : "+s"(cnt));
         if (a == 0 && c < hd) A.out[(int64_t)W.h * hd + c] = add_tail<true>(res, vs + body, sp + body, cnt);
-        if (++b >= b1) break;
+        if (ONE || ++b >= b1) break;
         put_v(b);
         if (b + 1 < b1) load_v(b + 1);
     }
+}
+
+template <int T, int KW, bool VEC>
+__global__ __launch_bounds__(kAttnFusedThreads)
+__attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_kernel(AttnArgs A) {
+    attn_fused_body<T, KW, VEC, true>(A);
+}
+template <int T, int KW, bool VEC>
+__global__ __launch_bounds__(kAttnFusedThreads)
+__attribute__((amdgpu_waves_per_eu(T <= 4 ? 4 : 2))) void attn_fused_blocks_kernel(AttnArgs A) {
+    attn_fused_body<T, KW, VEC, false>(A);
 }
 
 }  // namespace sihip

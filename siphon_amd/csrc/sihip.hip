@@ -3308,9 +3308,11 @@ extern "C" int sihip_attn_decode_dev(sihip_ctx *ctx, const float *q, const uint1
     if (A.n <= fmax) {
         const dim3 g((unsigned)((row_blocks + A.rb - 1) / A.rb * n_head)), t(kAttnFusedThreads);
         const size_t lds = (size_t)attn_fused_lds(A.n);
-#define SIHIP_AF(T, W)                                                                               \
-    if (vvec) hipLaunchKernelGGL((attn_fused_kernel<T, W, true>), g, t, lds, st, A);                 \
-    else hipLaunchKernelGGL((attn_fused_kernel<T, W, false>), g, t, lds, st, A);
+#define SIHIP_AF(T, W)                                                                                  \
+    if (A.rb == 1 && vvec) hipLaunchKernelGGL((attn_fused_kernel<T, W, true>), g, t, lds, st, A);       \
+    else if (A.rb == 1) hipLaunchKernelGGL((attn_fused_kernel<T, W, false>), g, t, lds, st, A);         \
+    else if (vvec) hipLaunchKernelGGL((attn_fused_blocks_kernel<T, W, true>), g, t, lds, st, A);        \
+    else hipLaunchKernelGGL((attn_fused_blocks_kernel<T, W, false>), g, t, lds, st, A);
         SIHIP_BY_KEYS(SIHIP_AF)
 #undef SIHIP_AF
     } else {
