@@ -74,10 +74,13 @@ const char *sihip_last_error(const sihip_ctx *ctx);
  * TILE_COLS (these four apply to later uploads and launches), GEMM_MIN_M,
  * GEMM_MT, GEMM_SBK, GEMM2_MIN_M, GEMM2_WAVES, GEMM6_MIN_M, GEMMH_MIN_M,
  * GEMMQ_MIN_M, GEMMQ_XMODE, GEMM2S_MAX_M, GEMMKS_MAX_M (the largest M on
- * the small-M K-quant GEMMs, 0: none), GEMMKS_Q4K, GEMMS_WAVES, GEMMSK_MAX_M
+ * the small-M K-quant GEMMs, 0: none), GEMMKS_Q4K, GEMMS_WAVES, GEMMKF_MAX_M,
+ * GEMMKF_SBK, GEMMQ_FUSE, GEMMH_FUSE, GEMM_GROUP, GEMMSK_MAX_M
  * (the largest M on the short-prompt K-quant GEMM, 0: none), GEMMX_MIN_M and
  * GEMMD_MIN_M (the smallest M on the prompt GEMMs of the K-quants and of the
- * other formats, 0: never), and
+ * other formats, 0: never), RING_MT and RING_SBK (m tiles and K-slice length of
+ * these two), ATTN_FUSE (k: decode attention in one launch up to 512 k
+ * positions, at most 1536, 0: never), and
  * Q80_SCALAR: 1 quantizes Q8_0-pair
  * activations with the reference's portable scalar routine (reference
  * kernels.c:542-558), as the reference does when SI_SCALAR is set or the
