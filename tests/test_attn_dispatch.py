@@ -66,6 +66,16 @@ def test_the_single_launch_fits_the_cus(n_head, hd, workgroups):
     assert len(got) == 1 and got[0][1] == workgroups
 
 
+@pytest.mark.parametrize("n_head,hd,kernel", [
+    (32, 128, "attn_fused_kernel<4,8,true>"), (33, 128, "attn_fused_blocks_kernel<4,8,true>"),
+    (16, 256, "attn_fused_kernel<8,8,true>"), (16, 512, "attn_fused_blocks_kernel<16,8,true>"),
+    (300, 16, "attn_fused_kernel<4,8,true>"),  # one block of value rows a head
+])
+def test_one_block_of_values_has_a_kernel_of_its_own(n_head, hd, kernel):
+    got = launches(n_head, n_head, hd, 100, 512)
+    assert [k for k, *_ in got] == [kernel]
+
+
 @pytest.mark.parametrize("n_head,n_kv,hd,n_ctx,one,three", [
     (32, 8, 128, 2048, 1200, 1201),
     (16, 8, 192, 2048, 1024, 1025),
